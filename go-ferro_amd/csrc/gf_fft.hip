@@ -18,6 +18,7 @@
 // Transforms are radix-2: forward decimation in time (bit-reversed load,
 // natural result), inverse decimation in frequency (natural load,
 // bit-reversed result read back at the store), twiddles staged in LDS.
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -455,32 +456,54 @@ static gf_status make_table(gf_ctx* c, Twiddles& t, int64_t n) {
     return hip_check(c, hipMemcpy(t.dev, h.data(), sizeof(double2) * n, hipMemcpyHostToDevice), "copy twiddles");
 }
 
-// Radices of n from {4, 2, 3, 5, 7}, or false when n has another prime
-// factor.
-static bool factor(int64_t n, FftFactors& f) {
-    f = FftFactors{};
+// The passes of a line of length n: radices from {1..10, 12, 14, 15, 16}
+// whose product is n in rising order, as few as possible but at least two (a
+// line of up to 16 elements takes a 1 and its length), and among those with
+// the largest smallest one (the fewest butterflies per line); the first is at
+// most first_max.  False when n has a prime factor above 7.
+static bool factor(int64_t n, LinePlan& f, int first_max = 16) {
+    static const int kRadices[] = {16, 15, 14, 12, 10, 9, 8, 7, 6, 5, 4, 3, 2};
+    f = LinePlan{};
     f.n = static_cast<int>(n);
-    int64_t m = n;
-    auto push = [&](int r) {
-        if (f.count >= kMaxRadices) return false;
-        f.r[f.count++] = r;
-        m /= r;
-        return true;
+    int best[kMaxPasses], cur[kMaxPasses], nbest = kMaxPasses + 1, rbest = 0;
+    auto search = [&](auto&& self, int64_t m, int depth, int from) -> void {
+        if (m == 1) {
+            // a line of one radix takes a 1 before it
+            const int low = depth < 2 ? 1 : cur[depth - 1];
+            if (low <= first_max && (depth < nbest || (depth == nbest && low > rbest))) {
+                nbest = depth;
+                rbest = low;
+                std::copy(cur, cur + depth, best);
+            }
+            return;
+        }
+        if (depth >= kMaxPasses || depth >= nbest) return;
+        for (int i = from; i < 13; i++)
+            if (m % kRadices[i] == 0) {
+                cur[depth] = kRadices[i];
+                self(self, m / kRadices[i], depth + 1, i);
+            }
     };
-    while (m % 4 == 0) if (!push(4)) return false;
-    while (m % 2 == 0) if (!push(2)) return false;
-    for (int r : {3, 5, 7})
-        while (m % r == 0) if (!push(r)) return false;
-    return m == 1;
-}
-
-// Pencils per workgroup of the mixed-radix passes: as many lines as keep
-// the two LDS buffers within 2048 elements (z and y) or 1024 (x, three
-// components), a power of two, at most 16.
-static int any_pencils(int64_t len, int64_t budget, int64_t other) {
-    int64_t p = 1;
-    while (p * 2 <= 16 && p * 2 * len <= budget && p * 2 <= other) p *= 2;
-    return static_cast<int>(p);
+    search(search, n, 0, 0);
+    if (nbest > kMaxPasses) return false;
+    while (nbest < 2) best[nbest++] = 1;
+    std::reverse(best, best + nbest);
+    f.count = nbest;
+    auto fast = [](int64_t d) {
+        return FastDiv{static_cast<uint32_t>(d), static_cast<uint32_t>(((uint64_t{1} << 32) + d - 1) / d)};
+    };
+    int64_t L = 1;
+    for (int i = 0; i < f.count; i++) {
+        f.r[i] = best[i];
+        f.per[i] = fast(n / best[i]);
+        f.L[i] = fast(L);
+        f.unit[i] = static_cast<int>(n / (L * best[i]));
+        f.maxr = std::max(f.maxr, best[i]);
+        // a radix of 1 only hands its elements on; it counts like the others
+        f.width = std::max(f.width, static_cast<int>(n / best[i]));
+        L *= best[i];
+    }
+    return true;
 }
 
 static AnyPassArgs any_args(const gf_ctx* c, const DemagPlan& d) {
@@ -490,7 +513,8 @@ static AnyPassArgs any_args(const gf_ctx* c, const DemagPlan& d) {
     a.kre = d.kre; a.kim = d.kim;
     a.nh = c->nx * c->ny * d.nzh;
     a.nhb = a.nh;
-    a.den = -c->dx * c->dy * c->dz;
+    a.rden = 1. / (-c->dx * c->dy * c->dz);
+    a.nmat = static_cast<int>(c->host_mats.size());
     a.nx = static_cast<int>(c->nx); a.ny = static_cast<int>(c->ny); a.nzh = static_cast<int>(d.nzh);
     return a;
 }
@@ -510,9 +534,7 @@ static hipError_t run_zfwd(gf_ctx* c, DemagPlan& d, bool raw, const double* cons
         }
         a.raw_in = raw ? 1 : 0;
         a.f = d.fz; a.tw = d.gtz.dev;
-        a.pencils = any_pencils(c->nz, 2048, c->ny);
-        dim3 grid(blocks_for(c->ny, a.pencils), static_cast<unsigned>(c->nx), static_cast<unsigned>(comps));
-        const hipError_t e = launch_any_pass(AnyPass::kZFwd, a, grid, c->stream);
+        const hipError_t e = launch_any_pass(AnyPass::kZFwd, a, comps, 0, c->stream);
         timer_end(c, GF_K_FFT_Z_FWD, ev);
         return e;
     }
@@ -558,9 +580,7 @@ static hipError_t run_y(gf_ctx* c, DemagPlan& d, bool inverse, int comps, KzRang
         a.spec = inverse ? d.spec_a : d.spec_m;
         a.nhb = kr.nhb; a.kz0 = kr.k0; a.kzb0 = kr.kb0;
         a.f = d.fy; a.tw = d.gty.dev;
-        a.pencils = any_pencils(c->ny, 2048, c->nx);
-        dim3 grid(blocks_for(c->nx, a.pencils), static_cast<unsigned>(kr.cnt), static_cast<unsigned>(comps));
-        const hipError_t e = launch_any_pass(inverse ? AnyPass::kYInv : AnyPass::kYFwd, a, grid, c->stream);
+        const hipError_t e = launch_any_pass(inverse ? AnyPass::kYInv : AnyPass::kYFwd, a, comps, kr.cnt, c->stream);
         timer_end(c, cls, ev);
         return e;
     }
@@ -589,9 +609,7 @@ static hipError_t run_x(gf_ctx* c, DemagPlan& d, bool conv, KzRange kr, bool adj
         a.conv = conv ? 1 : 0;
         a.adjoint = adjoint ? 1 : 0;
         a.f = d.fx; a.tw = d.gtx.dev;
-        a.pencils = any_pencils(c->nx, conv ? 1024 / 3 : 1024, c->ny);
-        dim3 grid(blocks_for(c->ny, a.pencils), static_cast<unsigned>(kr.cnt));
-        const hipError_t e = launch_any_pass(AnyPass::kXConv, a, grid, c->stream);
+        const hipError_t e = launch_any_pass(AnyPass::kXConv, a, 1, kr.cnt, c->stream);
         timer_end(c, GF_K_FFT_X_CONV, ev);
         return e;
     }
@@ -619,9 +637,7 @@ static hipError_t run_zinv(gf_ctx* c, DemagPlan& d, double* const* out = nullptr
         a.spec = d.spec_a;
         for (int i = 0; i < 3; i++) a.out[i] = out ? out[i] : c->hstat[i];
         a.f = d.fz; a.tw = d.gtz.dev;
-        a.pencils = any_pencils(c->nz, 2048, c->ny);
-        dim3 grid(blocks_for(c->ny, a.pencils), static_cast<unsigned>(c->nx), 3);
-        const hipError_t e = launch_any_pass(AnyPass::kZInv, a, grid, c->stream);
+        const hipError_t e = launch_any_pass(AnyPass::kZInv, a, 3, 0, c->stream);
         timer_end(c, GF_K_FFT_Z_INV, ev);
         return e;
     }
@@ -651,7 +667,7 @@ static gf_status plan_alloc(gf_ctx* c, DemagPlan& d, const char* what) {
     const std::string name(what);
     d.general = !pow2(c->nx) || !pow2(c->ny) || !pow2(c->nz);
     if (d.general) {
-        if (!factor(c->nx, d.fx) || !factor(c->ny, d.fy) || !factor(c->nz, d.fz))
+        if (!factor(c->nx, d.fx) || !factor(c->ny, d.fy) || !factor(c->nz, d.fz, 8))
             return set_error(c, GF_ERR_UNSUPPORTED,
                              name + " needs nx, ny, nz whose prime factors are 2, 3, 5 and 7");
         if (c->nx > 1024 || c->ny > 2048 || c->nz > 2048)

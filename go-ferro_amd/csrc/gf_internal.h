@@ -485,13 +485,26 @@ struct Twiddles {
     double2* dev = nullptr;
 };
 
-// Radices of a mixed-radix line transform of length n (their product), for
-// the passes of grids that are not powers of two.
-constexpr int kMaxRadices = 16;
-struct FftFactors {
+// Division by a launch constant d of values x with x d < 2^32:
+// x / d = (x m) >> 32 with m = ceil(2^32 / d), and x itself for d = 1.
+struct FastDiv {
+    uint32_t d = 1;
+    uint32_t m = 0;
+};
+
+// A mixed-radix line transform of length n (gf_fft_line.h): its passes'
+// radices, the butterflies per line (n / R), the product of the radices
+// before a pass, and the twiddle step n / (L R).
+constexpr int kMaxPasses = 8;
+struct LinePlan {
     int n = 0;
     int count = 0;
-    int r[kMaxRadices] = {};
+    int maxr = 0;                    // largest radix
+    int width = 0;                   // most butterflies per line of a pass
+    int r[kMaxPasses] = {};
+    int unit[kMaxPasses] = {};
+    FastDiv per[kMaxPasses];
+    FastDiv L[kMaxPasses];
 };
 
 struct DemagPlan {
@@ -500,7 +513,7 @@ struct DemagPlan {
     // kernels (gf_fft_any.hip) with natural-order twiddle tables of n
     // entries, w[t] = exp(-2 pi i t / n).
     bool general = false;
-    FftFactors fx, fy, fz;
+    LinePlan fx, fy, fz;
     Twiddles gtx, gty, gtz;
     int64_t nzh = 0;                 // nz/2 + 1
     double2* spec_m = nullptr;       // M z-spectrum, 3 components, layout [x][kz][y]
@@ -542,16 +555,19 @@ struct AnyPassArgs {
     const double* kre;          // tensor spectra (real, FP32 imaginary), [kz][y][x]
     const float* kim;
     const double2* tw;          // twiddle table of the pass's length
-    FftFactors f;               // the pass's transform length and radices
+    LinePlan f;                 // the pass's transform
+    FastDiv nn;                 // by the length
     int64_t nh, nhb;
-    double den;                 // -dx dy dz
-    int nx, ny, nzh;
-    int pencils;
+    double rden;                // 1 / (-dx dy dz)
+    int nx, ny, nzh, nmat;
+    int pencils, logp;          // lines a workgroup takes per component (z: columns), a power of two
+    int stride;                 // LDS slots of a line
     int kz0, kzb0;
     int raw_in, conv, adjoint;
 };
-size_t any_pass_lds(int lines, int n);
-hipError_t launch_any_pass(AnyPass kind, const AnyPassArgs& a, dim3 grid, hipStream_t s);
+// planes: the kz planes (y and x passes) or components (z passes) the
+// launch covers in its other grid dimensions
+hipError_t launch_any_pass(AnyPass kind, AnyPassArgs a, int comps, int planes, hipStream_t s);
 
 struct TimerSlot {
     hipEvent_t start, stop;

@@ -66,6 +66,27 @@ def test_static_field_matches_oracle(shape, scale):
     o.close()
 
 
+# every radix of the mixed-radix line transforms (1..10, 12, 14, 15, 16), two,
+# three and four passes a line, odd counts of z columns (a pair without its
+# second), lines fewer than a workgroup's, and the longest lines
+@pytest.mark.parametrize("shape", [(9, 10, 12), (14, 15, 16), (3, 5, 7), (2, 1, 9), (81, 6, 49), (105, 2, 90),
+                                   (35, 15, 256), (1, 112, 6), (6, 2, 1701), (7, 2000, 2), (1000, 3, 2),
+                                   (12, 28, 30)])
+def test_line_transforms_of_every_radix(shape):
+    """Static field within 1e-12 of its peak: the rounding of two transforms of
+    n points is a few eps log2(n), about 5e-15."""
+    say("case line transforms", shape)
+    prob, p, q = block(shape)
+    g, o = pair(prob, p, q)
+    g.demag()
+    o.demag()
+    d = rel(g.download(FIELD_ESTAT), o.get(FIELD_ESTAT))
+    say("  rel", d)
+    assert d <= 1e-12
+    g.close()
+    o.close()
+
+
 def test_ferroelectric_steps_with_electrostatics():
     say("case FE steps with electrostatics")
     prob, p, q = block()
