@@ -1621,7 +1621,9 @@ FeStageArgs fe_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
         a.estat[i] = c->estat[i];
         a.flexo[i] = c->d_flexo ? c->flexo_force[i] : nullptr;
     }
-    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz; a.dt = c->dt;
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dt = c->dt;
+    const double h[3] = {c->dx, c->dy, c->dz};
+    for (int i = 0; i < 3; i++) a.rh2[i] = (1. / h[i]) * (1. / h[i]);
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
     std::memcpy(a.Tc2g, c->Tc2g, sizeof(a.Tc2g));
     a.rotate = (c->flags & GF_FLAG_ORIENT_ROTATE) ? 1 : 0;
@@ -2005,9 +2007,12 @@ gf_status gf_em_stage(gf_ctx* c, int stage) {
     for (int q = 0; q < 9; q++) a.jps[q] = c->jp_on ? c->Jps[q] : nullptr;
     a.jf_comp = jf_comp; a.jf_value = jf_value; a.jf_spatial = jf_spatial;
     for (int i = 0; i < 3; i++) { a.jf_lo[i] = c->jf_lo[i]; a.jf_hi[i] = c->jf_hi[i]; }
-    a.nx = nx; a.ny = ny; a.nz = nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz; a.dt = c->dt;
+    a.nx = nx; a.ny = ny; a.nz = nz;
+    a.dt = c->dt; a.ce = c->dt / kEps0; a.rdt = 1. / c->dt;
+    a.rdx = 1. / c->dx; a.rdy = 1. / c->dy; a.rdz = 1. / c->dz;
     for (int i = 0; i < 3; i++) a.per[i] = c->per[i];
     a.stage = stage;
+    a.nmat = static_cast<int32_t>(c->host_mats.size());
     // Ampere and Faraday with the RK updates (both read the stage-s stores),
     // with a deferred ferroelectric stage in the same launch
     if (!st) {

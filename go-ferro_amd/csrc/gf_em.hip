@@ -32,18 +32,16 @@ namespace {
 
 using em_dev::em_edge;
 using em_dev::em_face;
-using em_dev::rk_state;
 
 // Ampere and Faraday of a stage in one launch: both read only the stage
-// stores and write other arrays, so the edges (first nE threads) and the
-// faces (the rest) are independent.
-__global__ void __launch_bounds__(256) em_eh_kernel(EmArgs a) {
-    const int64_t nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t nE = nx * (ny + 1) * (nz + 1) + (nx + 1) * ny * (nz + 1) + (nx + 1) * (ny + 1) * nz;
-    const int64_t nH = (nx + 1) * ny * nz + nx * (ny + 1) * nz + nx * ny * (nz + 1);
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t < nE) em_edge(a, t);
-    else if (t < nE + nH) em_face(a, t - nE);
+// stores and write other arrays, so the edges and the faces are independent.
+template <class I>
+__global__ void __launch_bounds__(em_dev::kEmGroup) em_eh_kernel(EmArgs a) {
+    extern __shared__ double emtab[];
+    const unsigned gE = em_dev::em_groups(em_dev::em_edges(a)), b = blockIdx.x;
+    const I t = static_cast<I>(b < gE ? b : b - gE) * em_dev::kEmGroup + static_cast<I>(threadIdx.x);
+    if (b < gE) em_edge<I>(a, emtab, t);
+    else if (t < static_cast<I>(em_dev::em_faces(a))) em_face<I>(a, t);
 }
 
 __global__ void __launch_bounds__(256) em_jp_kernel(EmJpArgs a) {
@@ -58,7 +56,9 @@ __global__ void __launch_bounds__(256) em_jp_kernel(EmJpArgs a) {
                 k_ = (kEps0 * M.wp[p] * M.wp[p] * a.ecell[c][id] * M.cn[p] - M.re[p] * a.jps[3 * p + c][id]) * a.dt;
             }
             // the store is updated in place: only this thread reads it now
-            rk_state(a.stage, id, k_, a.jp[3 * p + c], a.jacc[3 * p + c], a.jps[3 * p + c]);
+            const int v = 3 * p + c;
+            em_dev::rk_state(a.stage, id, k_, a.jp[v][id], a.stage > 1 ? a.jacc[v][id] : 0., a.jp[v], a.jacc[v],
+                             a.jps[v]);
             if (a.stage == 4) a.jps[3 * p + c][id] = a.jp[3 * p + c][id];
         }
 }
@@ -75,19 +75,20 @@ __device__ __forceinline__ double z_wall_value(const EmWallArgs& w, int comp, in
     return w.t1[comp][inner] + cf * (w.t1[comp][wall] - w.b[comp][inner]);
 }
 
+template <class I>
 __global__ void __launch_bounds__(256) em_cells_kernel(EmCellArgs a) {
-    const int64_t nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t id = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
+    const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= nx * ny * nz) return;
-    const int64_t i = id / (ny * nz), j = (id / nz) % ny, k = id % nz;
+    const I l = id / nz, k = id - l * nz, i = l / ny, j = l - i * ny;
     if (a.do_e) {
         const double* ex = a.es[0];
         const double* ey = a.es[1];
         const double* ez = a.es[2];
-        const int64_t x00 = (i * (ny + 1) + j) * (nz + 1) + k, x10 = (i * (ny + 1) + j + 1) * (nz + 1) + k;
-        const int64_t y00 = (i * ny + j) * (nz + 1) + k, y10 = ((i + 1) * ny + j) * (nz + 1) + k;
-        double vx[4] = {ex[x00], ex[x10], ex[x00 + 1], ex[x10 + 1]};
-        double vy[4] = {ey[y00], ey[y10], ey[y00 + 1], ey[y10 + 1]};
+        const I x00 = (i * (ny + 1) + j) * (nz + 1) + k, x10 = (i * (ny + 1) + j + 1) * (nz + 1) + k;
+        const I y00 = (i * ny + j) * (nz + 1) + k, y10 = ((i + 1) * ny + j) * (nz + 1) + k;
+        double vx[4] = {ldd(ex, x00), ldd(ex, x10), ldd(ex, x00 + 1), ldd(ex, x10 + 1)};
+        double vy[4] = {ldd(ey, y00), ldd(ey, y10), ldd(ey, y00 + 1), ldd(ey, y10 + 1)};
         if (a.zwall && (k == 0 || k == nz - 1)) {
             // the wall edges this cell reads, from the wall condition; the
             // cell of a line's own (i, j) writes it (and the last cell the
@@ -97,27 +98,27 @@ __global__ void __launch_bounds__(256) em_cells_kernel(EmCellArgs a) {
             for (int top = 0; top < 2; top++) {
                 if (top ? k != nz - 1 : k != 0) continue;
                 const int slot = top ? 2 : 0;
-                const int64_t cx0 = x00 - k, cx1 = x10 - k, cy0 = y00 - k, cy1 = y10 - k;   // line starts
+                const I cx0 = x00 - k, cx1 = x10 - k, cy0 = y00 - k, cy1 = y10 - k;   // line starts
                 vx[slot] = z_wall_value(a.w, 0, cx0, top);
                 vx[slot + 1] = z_wall_value(a.w, 0, cx1, top);
                 vy[slot] = z_wall_value(a.w, 1, cy0, top);
                 vy[slot + 1] = z_wall_value(a.w, 1, cy1, top);
-                const int64_t off = top ? nz : 0;
-                wx[cx0 + off] = vx[slot];
-                if (j == ny - 1) wx[cx1 + off] = vx[slot + 1];
-                wy[cy0 + off] = vy[slot];
-                if (i == nx - 1) wy[cy1 + off] = vy[slot + 1];
+                const I off = top ? nz : 0;
+                std_(wx, cx0 + off, vx[slot]);
+                if (j == ny - 1) std_(wx, cx1 + off, vx[slot + 1]);
+                std_(wy, cy0 + off, vy[slot]);
+                if (i == nx - 1) std_(wy, cy1 + off, vy[slot + 1]);
             }
         }
-        a.ecell[0][id] = (vx[0] + vx[1] + vx[2] + vx[3]) / 4.;
-        a.ecell[1][id] = (vy[0] + vy[1] + vy[2] + vy[3]) / 4.;
-        const int64_t z00 = (i * (ny + 1) + j) * nz + k, z10 = ((i + 1) * (ny + 1) + j) * nz + k;
-        const int64_t z01 = (i * (ny + 1) + j + 1) * nz + k, z11 = ((i + 1) * (ny + 1) + j + 1) * nz + k;
-        a.ecell[2][id] = (ez[z00] + ez[z10] + ez[z01] + ez[z11]) / 4.;
+        std_(a.ecell[0], id, (vx[0] + vx[1] + vx[2] + vx[3]) / 4.);
+        std_(a.ecell[1], id, (vy[0] + vy[1] + vy[2] + vy[3]) / 4.);
+        const I z00 = (i * (ny + 1) + j) * nz + k, z10 = ((i + 1) * (ny + 1) + j) * nz + k;
+        const I z01 = (i * (ny + 1) + j + 1) * nz + k, z11 = ((i + 1) * (ny + 1) + j + 1) * nz + k;
+        std_(a.ecell[2], id, (ldd(ez, z00) + ldd(ez, z10) + ldd(ez, z01) + ldd(ez, z11)) / 4.);
     }
     if (a.do_h) {
-        a.hcell[0][id] = (a.hs[0][(i * ny + j) * nz + k] + a.hs[0][((i + 1) * ny + j) * nz + k]) / 2.;
-        a.hcell[1][id] = (a.hs[1][(i * (ny + 1) + j) * nz + k] + a.hs[1][(i * (ny + 1) + j + 1) * nz + k]) / 2.;
+        std_(a.hcell[0], id, (ldd(a.hs[0], (i * ny + j) * nz + k) + ldd(a.hs[0], ((i + 1) * ny + j) * nz + k)) / 2.);
+        std_(a.hcell[1], id, (ldd(a.hs[1], (i * (ny + 1) + j) * nz + k) + ldd(a.hs[1], (i * (ny + 1) + j + 1) * nz + k)) / 2.);
         if (a.one_d) {
             // 1D magnetostatics through the cell field (EMdynamic_solver.cpp:3793-3804)
             const uint32_t t = a.code[id] & kMatMask;
@@ -127,9 +128,9 @@ __global__ void __launch_bounds__(256) em_cells_kernel(EmCellArgs a) {
                 const double mz = a.mz ? a.mz[id] : 0., mz1 = a.mz1 ? a.mz1[id] : 0., mz2 = a.mz2 ? a.mz2[id] : 0.;
                 h = -1. * M.Ms * mz - 1. * M.aMs[0] * mz1 - 1. * M.aMs[1] * mz2 - a.hzstat[id];
             }
-            a.hcell[2][id] = h;
+            std_(a.hcell[2], id, h);
         } else {
-            a.hcell[2][id] = (a.hs[2][(i * ny + j) * (nz + 1) + k] + a.hs[2][(i * ny + j) * (nz + 1) + k + 1]) / 2.;
+            std_(a.hcell[2], id, (ldd(a.hs[2], (i * ny + j) * (nz + 1) + k) + ldd(a.hs[2], (i * ny + j) * (nz + 1) + k + 1)) / 2.);
         }
     }
 }
@@ -226,9 +227,11 @@ unsigned blocks_for(int64_t n) { return static_cast<unsigned>((n + 255) / 256); 
 }  // namespace
 
 hipError_t launch_em_eh(const EmArgs& a, hipStream_t s) {
-    const int64_t nE = a.nx * (a.ny + 1) * (a.nz + 1) + (a.nx + 1) * a.ny * (a.nz + 1) + (a.nx + 1) * (a.ny + 1) * a.nz;
-    const int64_t nH = (a.nx + 1) * a.ny * a.nz + a.nx * (a.ny + 1) * a.nz + a.nx * a.ny * (a.nz + 1);
-    hipLaunchKernelGGL(em_eh_kernel, dim3(blocks_for(nE + nH)), dim3(256), 0, s, a);
+    const int64_t nE = em_dev::em_edges(a), nH = em_dev::em_faces(a);
+    const dim3 grid(em_dev::em_groups(nE) + em_dev::em_groups(nH)), block(em_dev::kEmGroup);
+    const size_t lds = sizeof(double) * em_dev::kEmC * static_cast<size_t>(a.nmat);
+    if (narrow(nE + nH)) hipLaunchKernelGGL(em_eh_kernel<uint32_t>, grid, block, lds, s, a);
+    else hipLaunchKernelGGL(em_eh_kernel<int64_t>, grid, block, lds, s, a);
     return hipGetLastError();
 }
 
@@ -286,7 +289,10 @@ hipError_t launch_spin_save(const SpinSaveArgs& a, hipStream_t s) {
 }
 
 hipError_t launch_em_cells(const EmCellArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(em_cells_kernel, dim3(blocks_for(a.nx * a.ny * a.nz)), dim3(256), 0, s, a);
+    const int64_t n = a.nx * a.ny * a.nz;
+    // the edge arrays hold at most four times the cells
+    if (narrow(4 * n)) hipLaunchKernelGGL(em_cells_kernel<uint32_t>, dim3(blocks_for(n)), dim3(256), 0, s, a);
+    else hipLaunchKernelGGL(em_cells_kernel<int64_t>, dim3(blocks_for(n)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 

@@ -6,27 +6,65 @@
 // cells (get_dH_RK*, :2239-3475) fused with update_DH_RK* (:3477-3586).
 // RK4 keeps a state accumulator, acc = y + k1/6, acc += k2/3, acc += k3/3,
 // y = acc + k4/6, the reference's left-to-right sum.
+// On a thin column (8x8x1024: 65k cells, 230k edges, 200k faces) a launch is
+// a few waves per SIMD, so the depth of the chain of loads and the index
+// arithmetic (64-bit divisions) set its time: all reads of an edge or face
+// go out together, offsets are 32-bit where they reach, and the launch with
+// the ferroelectric cells takes 12.8 us against 13.8.
 #pragma once
 
-#include "gf_internal.h"
+#include "gf_llg_dev.h"
 
 namespace gf {
 namespace em_dev {
 
-__device__ __forceinline__ void rk_state(int stage, int64_t i, double k, double* base, double* acc, double* out) {
-    const double y = base[i];
+// Edges and faces of an EM grid: the elements of the E and of the H arrays.
+__host__ __device__ __forceinline__ int64_t em_edges(const EmArgs& a) {
+    return a.nx * (a.ny + 1) * (a.nz + 1) + (a.nx + 1) * a.ny * (a.nz + 1) + (a.nx + 1) * (a.ny + 1) * a.nz;
+}
+__host__ __device__ __forceinline__ int64_t em_faces(const EmArgs& a) {
+    return (a.nx + 1) * a.ny * a.nz + a.nx * (a.ny + 1) * a.nz + a.nx * a.ny * (a.nz + 1);
+}
+
+// Workgroups of kEmGroup threads: those of the edges come first, then those
+// of the faces, each kind rounded up (a workgroup has one kind only).
+constexpr int kEmGroup = 256;
+__host__ __device__ __forceinline__ unsigned em_groups(int64_t n) {
+    return static_cast<unsigned>((n + kEmGroup - 1) / kEmGroup);
+}
+
+// RK update of element i from its preloaded base and (at stages 2-4)
+// accumulator.
+template <class I>
+__device__ __forceinline__ void rk_state(int stage, I i, double k, double y, double ac, double* base, double* acc,
+                                         double* out) {
     if (stage == 1) {
-        out[i] = y + k * 0.5;
-        acc[i] = y + k * kSixth;
+        std_(out, i, y + k * 0.5);
+        std_(acc, i, y + k * kSixth);
     } else if (stage == 2) {
-        out[i] = y + k * 0.5;
-        acc[i] = acc[i] + k * kThird;
+        std_(out, i, y + k * 0.5);
+        std_(acc, i, ac + k * kThird);
     } else if (stage == 3) {
-        out[i] = y + k;
-        acc[i] = acc[i] + k * kThird;
+        std_(out, i, y + k);
+        std_(acc, i, ac + k * kThird);
     } else {
-        base[i] = acc[i] + k * kSixth;
+        std_(base, i, ac + k * kSixth);
     }
+}
+
+// The workgroup's LDS copy of what an edge needs of every material: the
+// relative permittivity, the conductivity and whether it is ferroelectric.
+// An edge waits for its cells' codes and then for an LDS read, not for a
+// second trip to global memory.
+constexpr int kEmC = 3;
+
+__device__ __forceinline__ void load_emtab(double* tab, const DevMaterial* mats, int nmat) {
+    for (int t = threadIdx.x; t < kEmC * nmat; t += blockDim.x) {
+        const DevMaterial& M = mats[t / kEmC];
+        const int q = t % kEmC;
+        tab[t] = q == 0 ? M.em_er : q == 1 ? M.em_cond : (M.is_fe ? 1. : 0.);
+    }
+    __syncthreads();
 }
 
 // The free current of cell (i, j, k), component comp, at the stage time:
@@ -41,167 +79,182 @@ __device__ __forceinline__ double jf_at(const EmArgs& a, int comp, int64_t i, in
 
 // Four-cell means around an edge and the Ampere increment
 // (EMdynamic_solver.cpp:392-499), with the spin-pumping current on x and y.
-// The cells are (ci, cj, ck)[q], index cell[q].
-__device__ __forceinline__ double edge_increment(const EmArgs& a, int comp, const int64_t cell[4], const int64_t ci[4],
-                                                 const int64_t cj[4], const int64_t ck[4], double curl,
+// The cells are (ci, cj, ck)[q], index cell[q], codes tq[q], q store qv[q];
+// the quotients by four, the cell count and dt are products with their
+// reciprocals (within an ulp of the reference's).
+template <class I>
+__device__ __forceinline__ double edge_increment(const EmArgs& a, const double* tab, int comp, const I (&cell)[4],
+                                                 const I (&ci)[4], const I (&cj)[4], const I (&ck)[4],
+                                                 const uint32_t (&tq)[4], const double (&qv)[4], double curl,
                                                  double e_store) {
     double Jf = 0., Jp = 0., Ji = 0., dP = 0., er = 0., cond = 0., pc = 0.;
-    // the codes and the q store of the four cells are read together, before
-    // any code is known (every index is in bounds)
-    uint32_t tq[4];
-    double qv[4] = {0., 0., 0., 0.};
     for (int q = 0; q < 4; q++) {
-        tq[q] = a.code[cell[q]] & kMatMask;
-        if (a.q[0]) qv[q] = a.q[comp][cell[q]];
-    }
-    for (int q = 0; q < 4; q++) {
-        const int64_t id = cell[q];
-        const uint32_t t = tq[q];
+        const I id = cell[q];
+        const uint32_t t = tq[q] & kMatMask;
         if (!t) {
             er = er + 1.;
         } else {
-            const DevMaterial& M = a.mats[t - 1];
+            const double* M = tab + (t - 1u) * kEmC;
             if (a.q[0]) dP = dP + qv[q] * a.dt;
-            if (M.is_fe) pc = pc + 1.;
-            er = er + M.em_er;
-            cond = cond + M.em_cond;
+            er = er + M[0];
+            cond = cond + M[1];
+            pc = pc + M[2];
         }
         if (a.jf_comp >= 0) Jf = Jf + jf_at(a, comp, ci[q], cj[q], ck[q]);
-        if (a.jps[0]) Jp = Jp + a.jps[comp][id] + a.jps[3 + comp][id] + a.jps[6 + comp][id];
-        if (a.jishe[0] && comp < 2) Ji = Ji + a.jishe[comp][id];
+        if (a.jps[0]) Jp = Jp + ldd(a.jps[comp], id) + ldd(a.jps[3 + comp], id) + ldd(a.jps[6 + comp], id);
+        if (a.jishe[0] && comp < 2) Ji = Ji + ldd(a.jishe[comp], id);
     }
-    if (pc < 0.5) pc = 1.;
-    Jf = Jf / 4.;
-    Jp = Jp / 4.;
-    Ji = Ji / 4.;
-    dP = dP / pc;
-    er = er / 4.;
-    cond = cond / 4.;
-    return a.dt / kEps0 / er * (curl - Jf - Jp - Ji - cond * e_store - dP / a.dt);
+    const double rpc = pc < 1.5 ? 1. : (pc < 2.5 ? 0.5 : (pc < 3.5 ? kThird : 0.25));
+    Jf = Jf * 0.25;
+    Jp = Jp * 0.25;
+    Ji = Ji * 0.25;
+    dP = dP * rpc;
+    er = er * 0.25;
+    cond = cond * 0.25;
+    return a.ce / er * (curl - Jf - Jp - Ji - cond * e_store - dP * a.rdt);
 }
 
 // Ampere on edge e of the concatenated Ex|Ey|Ez grids, with its RK update.
-__device__ __forceinline__ void em_edge(const EmArgs& a, int64_t e) {
-    const int64_t nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t nEx = nx * (ny + 1) * (nz + 1), nEy = (nx + 1) * ny * (nz + 1);
-    auto C = [&](int64_t i, int64_t j, int64_t k) { return (i * ny + j) * nz + k; };
-    auto HX = [&](int64_t i, int64_t j, int64_t k) { return (i * ny + j) * nz + k; };
-    auto HY = [&](int64_t i, int64_t j, int64_t k) { return (i * (ny + 1) + j) * nz + k; };
-    auto HZ = [&](int64_t i, int64_t j, int64_t k) { return (i * ny + j) * (nz + 1) + k; };
+// Everything an edge reads (its base, accumulator and store, the H store
+// around it, its cells' codes and q store) is loaded before any of it is
+// used: every index is in bounds, on the wall edges too (they wrap).
+// A whole workgroup calls it, with e past the last edge in the last one's
+// spare threads: tab is the workgroup's material table, staged here after
+// the edge's own loads have been issued, so that both take one round trip.
+template <class I>
+__device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
+    const I nE = static_cast<I>(em_edges(a));
+    const bool live = e < nE;
+    if (!live) e = nE - 1;
+    const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
+    const I nEx = nx * (ny + 1) * (nz + 1), nEy = (nx + 1) * ny * (nz + 1);
+    auto C = [&](I i, I j, I k) { return (i * ny + j) * nz + k; };
+    auto HY = [&](I i, I j, I k) { return (i * (ny + 1) + j) * nz + k; };
+    auto HZ = [&](I i, I j, I k) { return (i * ny + j) * (nz + 1) + k; };
+    auto near = [](I v, I n) { return v <= 1 || v >= n - 1; };
     int comp;
-    double k_ = 0.;
-    bool hist = false;   // the edge lies on a plane a Mur wall reads (two next to each non-periodic wall)
-    auto near = [](int64_t v, int64_t n) { return v <= 1 || v >= n - 1; };
+    bool hist, dead;      // on a plane a Mur wall reads (two next to each non-periodic wall); a wall edge
+    I cell[4], ci[4], cj[4], ck[4], hp[4];
+    int hf[2];            // curl = (H_hf0[hp0] - H_hf0[hp1]) rh0 - (H_hf1[hp2] - H_hf1[hp3]) rh1
+    double rh[2];
     if (e < nEx) {
         comp = 0;
-        const int64_t i = e / ((ny + 1) * (nz + 1)), j = (e / (nz + 1)) % (ny + 1), k = e % (nz + 1);
+        const I l = e / (nz + 1), k = e - l * (nz + 1), i = l / (ny + 1), j = l - i * (ny + 1);
         hist = (!a.per[1] && near(j, ny)) || (!a.per[2] && near(k, nz));
         const bool wj = j == 0 || j == ny, wk = k == 0 || k == nz;
-        if (!(wj && !a.per[1]) && !(wk && !a.per[2])) {
-            const int64_t y1 = wj ? ny - 1 : j - 1, y3 = wj ? 0 : j, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
-            const double dHzdy = (a.hs[2][HZ(i, y3, z2)] - a.hs[2][HZ(i, y1, z2)]) / a.dy;
-            const double dHydz = (a.hs[1][HY(i, y3, z2)] - a.hs[1][HY(i, y3, z1)]) / a.dz;
-            const int64_t cell[4] = {C(i, y1, z1), C(i, y1, z2), C(i, y3, z1), C(i, y3, z2)};
-            const int64_t ci[4] = {i, i, i, i}, cj[4] = {y1, y1, y3, y3}, ck[4] = {z1, z2, z1, z2};
-            k_ = edge_increment(a, 0, cell, ci, cj, ck, dHzdy - dHydz, a.es[0][e]);
-        }
+        dead = (wj && !a.per[1]) || (wk && !a.per[2]);
+        const I y1 = wj ? ny - 1 : j - 1, y3 = wj ? 0 : j, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
+        for (int q = 0; q < 4; q++) { ci[q] = i; cj[q] = q < 2 ? y1 : y3; ck[q] = q & 1 ? z2 : z1; }
+        hf[0] = 2; hf[1] = 1; rh[0] = a.rdy; rh[1] = a.rdz;
+        hp[0] = HZ(i, y3, z2); hp[1] = HZ(i, y1, z2); hp[2] = HY(i, y3, z2); hp[3] = HY(i, y3, z1);
     } else if (e < nEx + nEy) {
         comp = 1;
         e -= nEx;
-        const int64_t i = e / (ny * (nz + 1)), j = (e / (nz + 1)) % ny, k = e % (nz + 1);
+        const I l = e / (nz + 1), k = e - l * (nz + 1), i = l / ny, j = l - i * ny;
         hist = (!a.per[0] && near(i, nx)) || (!a.per[2] && near(k, nz));
         const bool wi = i == 0 || i == nx, wk = k == 0 || k == nz;
-        if (!(wi && !a.per[0]) && !(wk && !a.per[2])) {
-            const int64_t x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
-            const double dHxdz = (a.hs[0][HX(x3, j, z2)] - a.hs[0][HX(x3, j, z1)]) / a.dz;
-            const double dHzdx = (a.hs[2][HZ(x3, j, z2)] - a.hs[2][HZ(x1, j, z2)]) / a.dx;
-            const int64_t cell[4] = {C(x1, j, z1), C(x1, j, z2), C(x3, j, z1), C(x3, j, z2)};
-            const int64_t ci[4] = {x1, x1, x3, x3}, cj[4] = {j, j, j, j}, ck[4] = {z1, z2, z1, z2};
-            k_ = edge_increment(a, 1, cell, ci, cj, ck, dHxdz - dHzdx, a.es[1][e]);
-        }
+        dead = (wi && !a.per[0]) || (wk && !a.per[2]);
+        const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
+        for (int q = 0; q < 4; q++) { ci[q] = q < 2 ? x1 : x3; cj[q] = j; ck[q] = q & 1 ? z2 : z1; }
+        hf[0] = 0; hf[1] = 2; rh[0] = a.rdz; rh[1] = a.rdx;
+        hp[0] = C(x3, j, z2); hp[1] = C(x3, j, z1); hp[2] = HZ(x3, j, z2); hp[3] = HZ(x1, j, z2);
     } else {
         comp = 2;
         e -= nEx + nEy;
-        const int64_t i = e / ((ny + 1) * nz), j = (e / nz) % (ny + 1), k = e % nz;
+        const I l = e / nz, k = e - l * nz, i = l / (ny + 1), j = l - i * (ny + 1);
         hist = (!a.per[0] && near(i, nx)) || (!a.per[1] && near(j, ny));
         const bool wi = i == 0 || i == nx, wj = j == 0 || j == ny;
-        if (!(wi && !a.per[0]) && !(wj && !a.per[1])) {
-            const int64_t x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, y1 = wj ? ny - 1 : j - 1, y2 = wj ? 0 : j;
-            const double dHydx = (a.hs[1][HY(x3, y2, k)] - a.hs[1][HY(x1, y2, k)]) / a.dx;
-            const double dHxdy = (a.hs[0][HX(x3, y2, k)] - a.hs[0][HX(x3, y1, k)]) / a.dy;
-            const int64_t cell[4] = {C(x1, y1, k), C(x1, y2, k), C(x3, y1, k), C(x3, y2, k)};
-            const int64_t ci[4] = {x1, x1, x3, x3}, cj[4] = {y1, y2, y1, y2}, ck[4] = {k, k, k, k};
-            k_ = edge_increment(a, 2, cell, ci, cj, ck, dHydx - dHxdy, a.es[2][e]);
-        }
+        dead = (wi && !a.per[0]) || (wj && !a.per[1]);
+        const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, y1 = wj ? ny - 1 : j - 1, y2 = wj ? 0 : j;
+        for (int q = 0; q < 4; q++) { ci[q] = q < 2 ? x1 : x3; cj[q] = q & 1 ? y2 : y1; ck[q] = k; }
+        hf[0] = 1; hf[1] = 0; rh[0] = a.rdx; rh[1] = a.rdy;
+        hp[0] = HY(x3, y2, k); hp[1] = HY(x1, y2, k); hp[2] = C(x3, y2, k); hp[3] = C(x3, y1, k);
     }
+    const double y = ldd(a.eb[comp], e), es = ldd(a.es[comp], e), ac = a.stage > 1 ? ldd(a.eacc[comp], e) : 0.;
+    uint32_t tq[4];
+    double qv[4] = {0., 0., 0., 0.}, hv[4];
+    for (int q = 0; q < 4; q++) {
+        cell[q] = C(ci[q], cj[q], ck[q]);
+        tq[q] = ldu(a.code, cell[q]);
+        hv[q] = ldd(a.hs[hf[q >> 1]], hp[q]);
+        if (a.q[0]) qv[q] = ldd(a.q[comp], cell[q]);
+    }
+    load_emtab(tab, a.mats, a.nmat);
+    if (!live) return;
+    double k_ = 0.;
+    if (!dead)
+        k_ = edge_increment<I>(a, tab, comp, cell, ci, cj, ck, tq, qv, (hv[0] - hv[1]) * rh[0] - (hv[2] - hv[3]) * rh[1],
+                               es);
     // stage 4: the base value before the combine overwrites it, for the
     // Mur walls (transfer_pointer, EMdynamic_AbsorbingBoundary.cpp:3-56);
     // each edge's own thread reads and then writes its base
-    if (a.t1[0] && hist) a.t1[comp][e] = a.eb[comp][e];
-    rk_state(a.stage, e, k_, a.eb[comp], a.eacc[comp], a.eo[comp]);
+    if (a.t1[0] && hist) std_(a.t1[comp], e, y);
+    rk_state<I>(a.stage, e, k_, y, ac, a.eb[comp], a.eacc[comp], a.eo[comp]);
 }
 
-// dM of one cell next to a face (EMdynamic_solver.cpp:2290-2340)
-__device__ __forceinline__ double cell_dm(const EmArgs& a, int comp, int64_t id, double& count) {
-    const uint32_t t = a.code[id] & kMatMask;
+// dM of one cell next to a face (EMdynamic_solver.cpp:2290-2340); called
+// only where a magnetic increment is given.
+template <class I>
+__device__ __forceinline__ double cell_dm(const EmArgs& a, int comp, I id, double& count) {
+    const uint32_t t = ldu(a.code, id) & kMatMask;
     if (!t) return 0.;
     const DevMaterial& M = a.mats[t - 1];
-    double d = 0.;
-    if (a.dm[0] || a.dma1[0]) {
-        const double f = a.dm[0] ? a.dm[comp][id] : 0.;
-        const double f1 = a.dma1[0] ? a.dma1[comp][id] : 0.;
-        const double f2 = a.dma2[0] ? a.dma2[comp][id] : 0.;
-        d = f * M.Ms + f1 * M.aMs[0] + f2 * M.aMs[1];
-    }
+    const double f = a.dm[0] ? ldd(a.dm[comp], id) : 0.;
+    const double f1 = a.dma1[0] ? ldd(a.dma1[comp], id) : 0.;
+    const double f2 = a.dma2[0] ? ldd(a.dma2[comp], id) : 0.;
     if (M.is_fm || M.is_afm) count = count + 1.;
-    return d;
+    return f * M.Ms + f1 * M.aMs[0] + f2 * M.aMs[1];
 }
 
-// Faraday on face f of the concatenated Hx|Hy|Hz grids, with its RK update.
-__device__ __forceinline__ void em_face(const EmArgs& a, int64_t f) {
-    const int64_t nx = a.nx, ny = a.ny, nz = a.nz;
-    const int64_t nHx = (nx + 1) * ny * nz, nHy = nx * (ny + 1) * nz;
-    auto C = [&](int64_t i, int64_t j, int64_t k) { return (i * ny + j) * nz + k; };
-    auto EX = [&](int64_t i, int64_t j, int64_t k) { return (i * (ny + 1) + j) * (nz + 1) + k; };
-    auto EY = [&](int64_t i, int64_t j, int64_t k) { return (i * ny + j) * (nz + 1) + k; };
-    auto EZ = [&](int64_t i, int64_t j, int64_t k) { return (i * (ny + 1) + j) * nz + k; };
-    const double pre = -a.dt / kMu0;
-    int comp;
-    double k_, cnt = 0., d1, d2;
+// Faraday on face f of the concatenated Hx|Hy|Hz grids, with its RK update;
+// loads first, as em_edge.  Without magnetic increments the cells' part of
+// the increment is zero and their codes are not read.
+template <class I>
+__device__ __forceinline__ void em_face(const EmArgs& a, I f) {
+    const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
+    const I nHx = (nx + 1) * ny * nz, nHy = nx * (ny + 1) * nz;
+    auto C = [&](I i, I j, I k) { return (i * ny + j) * nz + k; };
+    auto EX = [&](I i, I j, I k) { return (i * (ny + 1) + j) * (nz + 1) + k; };
+    auto EY = [&](I i, I j, I k) { return (i * ny + j) * (nz + 1) + k; };
+    auto EZ = [&](I i, I j, I k) { return (i * (ny + 1) + j) * nz + k; };
+    int comp, ef[2];      // curl = (E_ef0[ep0] - E_ef0[ep1]) re0 - (E_ef1[ep2] - E_ef1[ep3]) re1
+    I c1, c2, ep[4];      // the two cells beside the face
+    double re[2];
     if (f < nHx) {
         comp = 0;
-        const int64_t i = f / (ny * nz), j = (f / nz) % ny, k = f % nz;
-        const int64_t x1 = i == 0 ? (a.per[0] ? nx - 1 : 0) : i - 1, x2 = i == nx ? (a.per[0] ? 0 : nx - 1) : i;
-        const double dEzdy = (a.es[2][EZ(i, j + 1, k)] - a.es[2][EZ(i, j, k)]) / a.dy;
-        const double dEydz = (a.es[1][EY(i, j, k + 1)] - a.es[1][EY(i, j, k)]) / a.dz;
-        d1 = cell_dm(a, 0, C(x1, j, k), cnt);
-        d2 = cell_dm(a, 0, C(x2, j, k), cnt);
-        if (cnt < 0.5) cnt = 1.;
-        k_ = pre * (dEzdy - dEydz) - (d1 + d2) / cnt;
+        const I l = f / nz, k = f - l * nz, i = l / ny, j = l - i * ny;
+        const I x1 = i == 0 ? (a.per[0] ? nx - 1 : 0) : i - 1, x2 = i == nx ? (a.per[0] ? 0 : nx - 1) : i;
+        ef[0] = 2; ef[1] = 1; re[0] = a.rdy; re[1] = a.rdz;
+        ep[0] = EZ(i, j + 1, k); ep[1] = EZ(i, j, k); ep[2] = EY(i, j, k + 1); ep[3] = EY(i, j, k);
+        c1 = C(x1, j, k); c2 = C(x2, j, k);
     } else if (f < nHx + nHy) {
         comp = 1;
         f -= nHx;
-        const int64_t i = f / ((ny + 1) * nz), j = (f / nz) % (ny + 1), k = f % nz;
-        const int64_t y1 = j == 0 ? (a.per[1] ? ny - 1 : 0) : j - 1, y2 = j == ny ? (a.per[1] ? 0 : ny - 1) : j;
-        const double dExdz = (a.es[0][EX(i, j, k + 1)] - a.es[0][EX(i, j, k)]) / a.dz;
-        const double dEzdx = (a.es[2][EZ(i + 1, j, k)] - a.es[2][EZ(i, j, k)]) / a.dx;
-        d1 = cell_dm(a, 1, C(i, y1, k), cnt);
-        d2 = cell_dm(a, 1, C(i, y2, k), cnt);
-        if (cnt < 0.5) cnt = 1.;
-        k_ = pre * (dExdz - dEzdx) - (d1 + d2) / cnt;
+        const I l = f / nz, k = f - l * nz, i = l / (ny + 1), j = l - i * (ny + 1);
+        const I y1 = j == 0 ? (a.per[1] ? ny - 1 : 0) : j - 1, y2 = j == ny ? (a.per[1] ? 0 : ny - 1) : j;
+        ef[0] = 0; ef[1] = 2; re[0] = a.rdz; re[1] = a.rdx;
+        ep[0] = EX(i, j, k + 1); ep[1] = EX(i, j, k); ep[2] = EZ(i + 1, j, k); ep[3] = EZ(i, j, k);
+        c1 = C(i, y1, k); c2 = C(i, y2, k);
     } else {
         comp = 2;
         f -= nHx + nHy;
-        const int64_t i = f / (ny * (nz + 1)), j = (f / (nz + 1)) % ny, k = f % (nz + 1);
-        const int64_t z1 = k == 0 ? (a.per[2] ? nz - 1 : 0) : k - 1, z2 = k == nz ? (a.per[2] ? 0 : nz - 1) : k;
-        const double dEydx = (a.es[1][EY(i + 1, j, k)] - a.es[1][EY(i, j, k)]) / a.dx;
-        const double dExdy = (a.es[0][EX(i, j + 1, k)] - a.es[0][EX(i, j, k)]) / a.dy;
-        d1 = cell_dm(a, 2, C(i, j, z1), cnt);
-        d2 = cell_dm(a, 2, C(i, j, z2), cnt);
-        if (cnt < 0.5) cnt = 1.;
-        k_ = pre * (dEydx - dExdy) - (d1 + d2) / cnt;
+        const I l = f / (nz + 1), k = f - l * (nz + 1), i = l / ny, j = l - i * ny;
+        const I z1 = k == 0 ? (a.per[2] ? nz - 1 : 0) : k - 1, z2 = k == nz ? (a.per[2] ? 0 : nz - 1) : k;
+        ef[0] = 1; ef[1] = 0; re[0] = a.rdx; re[1] = a.rdy;
+        ep[0] = EY(i + 1, j, k); ep[1] = EY(i, j, k); ep[2] = EX(i, j + 1, k); ep[3] = EX(i, j, k);
+        c1 = C(i, j, z1); c2 = C(i, j, z2);
     }
-    rk_state(a.stage, f, k_, a.hb[comp], a.hacc[comp], a.ho[comp]);
+    const double y = ldd(a.hb[comp], f), ac = a.stage > 1 ? ldd(a.hacc[comp], f) : 0.;
+    double ev[4];
+    for (int q = 0; q < 4; q++) ev[q] = ldd(a.es[ef[q >> 1]], ep[q]);
+    double k_ = -a.dt / kMu0 * ((ev[0] - ev[1]) * re[0] - (ev[2] - ev[3]) * re[1]);
+    if (a.dm[0] || a.dma1[0]) {
+        double cnt = 0.;
+        const double d1 = cell_dm<I>(a, comp, c1, cnt), d2 = cell_dm<I>(a, comp, c2, cnt);
+        if (cnt < 0.5) cnt = 1.;
+        k_ = k_ - (d1 + d2) / cnt;
+    }
+    rk_state<I>(a.stage, f, k_, y, ac, a.hb[comp], a.hacc[comp], a.ho[comp]);
 }
 
 }  // namespace em_dev

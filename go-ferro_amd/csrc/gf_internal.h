@@ -141,9 +141,11 @@ struct EmArgs {
     const double* jishe[2];     // inverse spin Hall current Jx, Jy, null when off
     double* t1[3];              // stage 4 with Mur walls: E of the planes the walls read, kept before the combine
     int64_t nx, ny, nz;
-    double dx, dy, dz, dt;
+    double dt, ce, rdt;         // time step, dt / eps0, 1 / dt
+    double rdx, rdy, rdz;       // 1/dx, 1/dy, 1/dz
     int32_t per[3];
     int32_t stage;
+    int32_t nmat;               // material records
 };
 
 // get_J_ISHE_RK* (magnetic_solver.cpp:231-283): per pumping plane k, the
@@ -397,7 +399,8 @@ struct FeStageArgs {
     const double* ecell[3];     // electrodynamic E at the cells, null when uncoupled
     const double* flexo[3];     // flexoelectric force of the stage, null when off
     int64_t nx, ny, nz;
-    double dx, dy, dz, dt;
+    double dt;
+    double rh2[3];              // 1 / spacing^2
     double eext[3];
     double Tg2c[3][3];
     double Tc2g[3][3];

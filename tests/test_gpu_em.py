@@ -107,6 +107,29 @@ def test_fe_em_stages(flags):
     o.close()
 
 
+@pytest.mark.parametrize("shape", [(1, 1, 9), (1, 2, 255), (2, 9, 64), (3, 5, 17), (8, 8, 12)])
+def test_fe_em_steps_at_group_edges(shape):
+    """gf_step runs the ferroelectric cells, the edges and the faces as whole
+    workgroups of one launch: grids whose three counts leave each kind's last
+    workgroup nearly empty, nearly full or alone, against the oracle (the
+    per-stage bound)."""
+    from oracle.oracle import Oracle
+    prob, p, q = fe_film(shape=shape)
+    say("case fe + em steps", shape)
+    g, o = Context(prob), Oracle(prob)
+    E = random_yee(shape, FIELD_E_EM, 1e6, 4)
+    H = random_yee(shape, FIELD_H_EM, 3e3, 5)
+    for fid, val in ((FIELD_P, p), (FIELD_Q, q), (FIELD_E_EM, E), (FIELD_H_EM, H)):
+        g.upload(fid, val)
+        o.set(fid, val)
+    g.step(3)
+    o.step(3)
+    for fid in (FIELD_P, FIELD_Q, FIELD_E_EM, FIELD_H_EM, FIELD_E_CELL):
+        assert rel(g.download(fid), o.get(fid)) <= 1e-12, fid
+    g.close()
+    o.close()
+
+
 def boxed_media(shape=(8, 10, 12), flags=0, jf_type=1, plane=True):
     """Non-periodic in every direction: Mur (or PEC) walls on all six faces,
     a conductor, a Drude metal with two poles, a PEC inclusion, a plane
