@@ -1670,7 +1670,12 @@ gf_status gf_mag_stage(gf_ctx* c, int stage) {
         st = hip_check(c, launch_mag_stage_fused(a, f, c->demag.h_in_spec, c->stream), "mag stage");
         if (!st) c->demag.m_in_spec = true;
     } else {
-        st = hip_check(c, launch_mag_stage(a, c->n, c->stream, c->d_fm_ids, c->n_fm_ids), "mag stage");
+        if (c->el_pending)
+            st = hip_check(c, launch_el_force_mag(c->el_args, a, c->d_fm_ids, c->d_fm_ids ? c->n_fm_ids : c->n,
+                                                  c->stream), "elastic force and mag stage");
+        else
+            st = hip_check(c, launch_mag_stage(a, c->n, c->stream, c->d_fm_ids, c->n_fm_ids), "mag stage");
+        c->el_pending = false;
     }
     timer_end(c, GF_K_MAG_STAGE, ev);
     if (st) return st;
@@ -1795,29 +1800,43 @@ gf_status gf_elastic_stage(gf_ctx* c, int stage) {
     const int64_t slot_size = static_cast<int64_t>(kHistPlanes) * 3 * nxy;
 
     gf_status st = GF_OK;
+    ElStageArgs sa{};
     // stage 4: u enters the boundary history before the final combine
     // (transfer_pointer, elastodynamics_AbsorbingBoundary.cpp:3-89)
     if (stage == 4) {
         c->hist_head = (c->hist_head + 1) % c->hist_slots;
-        ElHistArgs h{};
-        for (int i = 0; i < 3; i++) h.u[i] = c->u[i];
-        h.slot = c->hist + c->hist_head * slot_size;
-        h.nx = c->nx; h.ny = c->ny; h.nz = c->nz;
+        for (int i = 0; i < 3; i++) sa.h.u[i] = c->u[i];
+        sa.h.slot = c->hist + c->hist_head * slot_size;
         const int32_t lp[kHistPlanes] = {1, 2, 3, 4};
         const int32_t mp[kHistPlanes] = {0, 1, static_cast<int32_t>(c->nz - 2), static_cast<int32_t>(c->nz - 1)};
-        for (int p = 0; p < kHistPlanes; p++) h.planes[p] = mur ? mp[p] : lp[p];
-        hipEvent_t ev = nullptr;
-        timer_begin(c, GF_K_OTHER, &ev);
-        st = hip_check(c, launch_el_history(h, c->stream), "boundary history");
-        timer_end(c, GF_K_OTHER, ev);
+        for (int p = 0; p < kHistPlanes; p++) sa.h.planes[p] = mur ? mp[p] : lp[p];
     }
+    const double* hist[4];
+    for (int j = 0; j < 4; j++)
+        hist[j] = c->hist + ((c->hist_head - j) % c->hist_slots + c->hist_slots) % c->hist_slots * slot_size;
     const double t_stage = stage == 1 ? c->time - c->dt : (stage == 4 ? c->time : c->time - 0.5 * c->dt);
+    // the displacement source (elastic_dynamic_solver.cpp:3060-3284)
+    const int kind = stage < 3 ? 0 : (stage == 3 ? 1 : 2);
+    int32_t src_k = -1;
+    double src_val = 0.;
+    if (gauss && c->src_comp >= 0 && c->src_k >= 0 && c->src_k < c->nz) {
+        const double tsrc = kind == 0 ? c->time - 0.5 * c->dt : c->time;
+        const double sg = c->src_sigma, A = c->src_amp;
+        const double vsp = c->src_comp == 2 ? c->vl_first : c->vt_first;
+        if (c->src_type == 1 && c->time < 12.5 * sg) {
+            src_k = c->src_k;
+            src_val = A * 1.6487210 * sg * vsp * std::exp(-1. * std::pow((tsrc - 5.0 * sg), 2.) / (2. * sg * sg));
+        } else if (c->src_type == 2) {
+            src_k = c->src_k;
+            if (c->src_cycles == 0 || tsrc <= static_cast<double>(c->src_cycles) / sg)
+                src_val = A * vsp / 2. / kPi / sg * (std::cos(2. * kPi * sg * tsrc) - 1);
+        }
+    }
     // strain of the stage store (elastic_dynamic_solver.cpp:107-227), the
     // eigenstrain from the stores of this stage (:4-104) and the cells'
-    // parts of their face stresses; then the stress divergence and the v, u
-    // updates (:841-3057)
-    if (!st) {
-        ElStageArgs sa{};
+    // parts of their face stresses; then the stress divergence, the v, u
+    // updates (:841-3057), the Liao plane and the source
+    {
         ElStrainArgs& a = sa.s;
         a.code = c->d_code;
         // the face gradients are kept only for the flexoelectric force
@@ -1881,52 +1900,40 @@ gf_status gf_elastic_stage(gf_ctx* c, int stage) {
             f.trac_row = c->src_comp;
             f.trac_amp = c->src_amp * std::exp(-1. * std::pow(tv, 2.) / (2. * std::pow(sg, 2.)));
         }
+        f.liao = mur ? 0 : 1;
+        f.w = c->w_liao;
+        for (int j = 0; j < 4; j++) f.hist[j] = hist[j];
+        f.src_k = mur ? -1 : src_k; f.src_comp = c->src_comp; f.src_val = src_val;
         hipEvent_t ev = nullptr;
         timer_begin(c, GF_K_ELASTIC_STAGE, &ev);
-        st = hip_check(c, launch_el_stage(sa, c->stream), "elastic stage");
+        st = hip_check(c, launch_el_prep(sa, c->stream), "elastic stage");
+        if (!st && c->el_defer) {
+            c->el_args = sa;
+            c->el_pending = true;
+        } else if (!st) {
+            st = hip_check(c, launch_el_force(sa, c->stream), "elastic force");
+        }
         timer_end(c, GF_K_ELASTIC_STAGE, ev);
         // the store just written is the stage's u store from here on
         if (!st) std::swap(c->us, c->us_alt);
     }
-    // absorbing boundary and displacement source
+    // Mur planes and the source after them
     // (elastodynamics_AbsorbingBoundary.cpp:92-230, elastic_dynamic_solver.cpp:3060-3284)
-    if (!st) {
-        const int kind = stage < 3 ? 0 : (stage == 3 ? 1 : 2);
+    if (!st && mur) {
         ElBoundaryArgs b{};
         b.code = c->d_code;
         for (int i = 0; i < 3; i++) { b.u[i] = c->u[i]; b.us[i] = c->us[i]; }
-        for (int j = 0; j < 4; j++) {
-            const int slot = ((c->hist_head - j) % c->hist_slots + c->hist_slots) % c->hist_slots;
-            b.t[j] = c->hist + slot * slot_size;
-        }
+        b.t1 = hist[0];
         b.nx = c->nx; b.ny = c->ny; b.nz = c->nz;
         b.kind = kind;
-        b.liao = mur ? 0 : 1;
         b.mur_bottom = (c->flags & GF_FLAG_1D_ABC_ELAST_ONLYTOP) ? 0 : 1;
-        b.w = c->w_liao;
         const double num = kind == 0 ? 2. * c->dz : c->dz;
         const double dt = c->dt;
         b.cb_l = (num - c->vl_first * dt) / (num + c->vl_first * dt);
         b.cb_t = (num - c->vt_first * dt) / (num + c->vt_first * dt);
         b.ct_l = (num - c->vl_last * dt) / (num + c->vl_last * dt);
         b.ct_t = (num - c->vt_last * dt) / (num + c->vt_last * dt);
-        b.src_k = -1;
-        if (gauss && c->src_comp >= 0 && c->src_k >= 0 && c->src_k < c->nz) {
-            const double tsrc = kind == 0 ? c->time - 0.5 * c->dt : c->time;
-            const double sg = c->src_sigma, A = c->src_amp;
-            const double vsp = c->src_comp == 2 ? c->vl_first : c->vt_first;
-            if (c->src_type == 1 && c->time < 12.5 * sg) {
-                b.src_k = c->src_k;
-                b.src_val = A * 1.6487210 * sg * vsp * std::exp(-1. * std::pow((tsrc - 5.0 * sg), 2.) / (2. * sg * sg));
-            } else if (c->src_type == 2) {
-                b.src_k = c->src_k;
-                if (c->src_cycles == 0 || tsrc <= static_cast<double>(c->src_cycles) / sg)
-                    b.src_val = A * vsp / 2. / kPi / sg * (std::cos(2. * kPi * sg * tsrc) - 1);
-                else
-                    b.src_val = 0.;
-            }
-            b.src_comp = c->src_comp;
-        }
+        b.src_k = src_k; b.src_comp = c->src_comp; b.src_val = src_val;
         hipEvent_t ev = nullptr;
         timer_begin(c, GF_K_OTHER, &ev);
         st = hip_check(c, launch_el_boundary(b, c->stream), "elastic boundary");
@@ -2137,6 +2144,9 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
         return set_error(c, GF_ERR_STATE, "gf_step called in the middle of a step");
     // the FE stage runs inside the EM stage's launch (they are independent)
     c->fe_defer = c->any_fe && c->em_on;
+    // and the elastic force inside the FM stage's (Mur planes follow the
+    // force at once, so it is not deferred with them)
+    c->el_defer = c->el_on && c->any_fm && !c->demag.fused && !(c->flags & GF_FLAG_1D_ABC) && narrow(c->n);
     for (int64_t s = 0; s < nsteps; s++) {
         gf_status st = gf_time_advance(c);
         for (int stage = 1; stage <= 4 && !st; stage++) {
@@ -2152,9 +2162,12 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
         if (st) {
             c->fe_defer = false;
             c->fe_pending = false;
+            c->el_defer = false;
+            c->el_pending = false;
             return st;
         }
     }
+    c->el_defer = false;
     c->fe_defer = false;
     return GF_OK;
 }

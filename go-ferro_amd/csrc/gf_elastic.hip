@@ -1,25 +1,31 @@
 // gf_elastic.hip — elastodynamics RK4 stage for gfx950 (FP64).
 //
 // One stage of the reference's elastic solver (elastic_dynamic_solver.cpp,
-// elastodynamics_AbsorbingBoundary.cpp) is up to four launches:
-//   history   stage 4 only: the boundary planes of u into the history ring
-//             (transfer_pointer, elastodynamics_AbsorbingBoundary.cpp:3-89)
+// elastodynamics_AbsorbingBoundary.cpp) is two launches, with Mur planes three:
 //   prep      face gradients of the u store and the cell strain (:107-227),
 //             the eigenstrain from the m, m_AFM and p stores (:4-104) with
-//             back-action, and each cell's part of its face stresses
+//             back-action, and each cell's part of its face stresses; at
+//             stage 4 the boundary planes of u into the history ring
+//             (transfer_pointer, elastodynamics_AbsorbingBoundary.cpp:3-89)
 //   force     stress divergence, dv and du = v_s dt, the v and u RK updates
-//             (get_dv_RKs / get_du_RKs / update_v_RKs / update_u_RKs, :841-3057)
-//   boundary  Liao or Mur planes and the displacement source
+//             (get_dv_RKs / get_du_RKs / update_v_RKs / update_u_RKs, :841-3057),
+//             the Liao plane and the displacement source
 //             (elastodynamics_AbsorbingBoundary.cpp:92-230, :3060-3284)
+//   boundary  Mur planes and the source: a Mur plane reads its neighbour's
+//             new u, so it follows the update in a launch of its own
 // The force launch reads the u store around each cell (its face gradients)
 // and writes the next store into a second array (the two are swapped after
 // it); v and its store are read and written by their own cell's thread only.
+// The Liao plane k = 0 reads only the history, so the cell's own thread
+// writes it, and the planes the history keeps are the prep's own cells: the
+// two launches that did this took 4.2 and 2.7 us (70k cells) or 6.2 and 4.8 us
+// (1M cells, of which the force gives 6 back).
 //
 // RK4 bookkeeping keeps a state accumulator per field, acc = y + k1/6,
 // acc = acc + k2/3, acc = acc + k3/3, y = acc + k4/6, which is the
 // reference's left-to-right y + k1/6 + k2/3 + k3/3 + k4/6 (the weights applied
 // as products with the rounded reciprocals, within about an ulp of the quotients).
-#include "gf_llg_dev.h"
+#include "gf_fm_dev.h"
 
 namespace gf {
 
@@ -300,6 +306,7 @@ __device__ __forceinline__ const double (*stiffness(const double* ctab, uint32_t
 // The workgroup's LDS copy of every material's constants: the stiffness
 // matrices (36 each), then the eigenstrain constants (kEigC each), then
 // el_rho, el_mass, el_stiff (kElC each).
+constexpr int kGroup = 256;   // threads of a prep or force workgroup
 constexpr int kElC = 3;
 constexpr int kLdsPerMat = 36 + kEigC + kElC;
 
@@ -323,8 +330,9 @@ __device__ __forceinline__ void load_ctab(double* ctab, const DevMaterial* mats,
 
 // ---------------------------------------------------------------- prep
 // The strain of the u store and the eigenstrain of the stage stores, both
-// written out, and the cell's P^x, P^y, P^z.  kGeneral: rotation and the
-// flexoelectric terms (the face gradients are written out for the latter).
+// written out, and the cell's P^x, P^y, P^z; at stage 4 the boundary planes
+// of u go to the history.  kGeneral: rotation and the flexoelectric terms
+// (the face gradients are written out for the latter).
 template <bool kGeneral>
 __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
@@ -349,6 +357,12 @@ __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
         for (int c = 0; c < 6; c++) a.e.e0g[c][id] = e0[c];
         if (a.e.e0c[0] != a.e.e0g[0])
             for (int c = 0; c < 6; c++) a.e.e0c[c][id] = sc[c];
+    }
+    if (a.h.slot) {
+        const int64_t nxy = a.s.nx * a.s.ny, ij = i * a.s.ny + j;
+        for (int p = 0; p < kHistPlanes; p++)
+            if (k == a.h.planes[p])
+                for (int c = 0; c < 3; c++) a.h.slot[(p * 3 + c) * nxy + ij] = a.h.u[c][id];
     }
     double P[3][3] = {{0., 0., 0.}, {0., 0., 0.}, {0., 0., 0.}};
     if (code & kMatMask) {
@@ -375,13 +389,13 @@ __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
 // other axes are done, so that the kernel stays at 124 VGPRs and 4 waves per
 // SIMD (with them first: 141 and 3 waves).  1M cells (128x128x64): 95.4 ->
 // 86.5 us; 70k cells (45x38x41): 13.9 -> 12.2 us.
+// group: the workgroup's index among those of the force.
 template <class I>
-__global__ void __launch_bounds__(256) el_force_kernel(ElStageArgs a) {
-    extern __shared__ double ctab[];   // the materials' constants (load_ctab)
+__device__ __forceinline__ void el_force_group(const ElStageArgs& a, double* ctab, unsigned group) {
     const ElForceArgs& f = a.f;
     load_ctab(ctab, f.mats, f.nmat);
     const I nx = static_cast<I>(f.nx), ny = static_cast<I>(f.ny), nz = static_cast<I>(f.nz);
-    const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
+    const I id = static_cast<I>(group) * kGroup + static_cast<I>(threadIdx.x);
     if (id >= nx * ny * nz) return;
     const I cl = id / nz, k = id - cl * nz, i = cl / ny, j = cl - i * ny;
     const int stage = f.stage;
@@ -496,44 +510,79 @@ __global__ void __launch_bounds__(256) el_force_kernel(ElStageArgs a) {
             if (stage == 1) std_(f.fstore[c], id, fo);
         }
     }
+    const bool plane = f.liao && k == 0;
+    // fourth-order Liao extrapolation of the plane from planes 1..4 of t1..t4
+    double bv[3] = {0., 0., 0.};
+    if (plane) {
+        const I nxy = nx * ny, ij = i * ny + j, pl = 3 * nxy;
+        const double w = f.w;
+        for (int c = 0; c < 3; c++) {
+            const I o = static_cast<I>(c) * nxy + ij;
+            bv[c] = (4. * w + 2. * (1. - w)) * ldd(f.hist[0], o) - (6. * w + (1. - w)) * ldd(f.hist[1], pl + o) +
+                    (4. * w) * ldd(f.hist[2], 2 * pl + o) - w * ldd(f.hist[3], 3 * pl + o);
+        }
+    }
+    const bool source = static_cast<int64_t>(k) == f.src_k && (code & kMatMask) != 0u;
     for (int c = 0; c < 3; c++) {
         const double du = ldd(f.vs[c], id) * f.dt;
         const double v = ldd(f.v[c], id), u = ldd(f.u[c], id);
-        if (stage == 1) {
-            std_(f.vs[c], id, v + dv[c] * 0.5);
-            std_(f.accv[c], id, v + dv[c] * kSixth);
-            std_(f.us[c], id, u + du * 0.5);
-            std_(f.accu[c], id, u + du * kSixth);
-        } else if (stage == 2) {
-            std_(f.vs[c], id, v + dv[c] * 0.5);
-            std_(f.accv[c], id, ldd(f.accv[c], id) + dv[c] * kThird);
-            std_(f.us[c], id, u + du * 0.5);
-            std_(f.accu[c], id, ldd(f.accu[c], id) + du * kThird);
-        } else if (stage == 3) {
-            std_(f.vs[c], id, v + dv[c]);
-            std_(f.accv[c], id, ldd(f.accv[c], id) + dv[c] * kThird);
-            std_(f.us[c], id, u + du);
-            std_(f.accu[c], id, ldd(f.accu[c], id) + du * kThird);
-        } else {
+        const bool src = source && c == f.src_comp;
+        if (stage == 4) {
             const double vn = ldd(f.accv[c], id) + dv[c] * kSixth;
-            const double un = ldd(f.accu[c], id) + du * kSixth;
+            double un = ldd(f.accu[c], id) + du * kSixth;
+            if (plane) un = bv[c];
+            if (src) un = f.src_val;
             std_(f.v[c], id, vn);
             std_(f.vs[c], id, vn);
             std_(f.u[c], id, un);
             std_(f.us[c], id, un);
+            continue;
+        }
+        // stages 1-3 set the Liao plane of u itself, the source in its store
+        if (plane) std_(f.u[c], id, bv[c]);
+        if (stage == 1) {
+            std_(f.vs[c], id, v + dv[c] * 0.5);
+            std_(f.accv[c], id, v + dv[c] * kSixth);
+            std_(f.us[c], id, src ? f.src_val : u + du * 0.5);
+            std_(f.accu[c], id, u + du * kSixth);
+        } else if (stage == 2) {
+            std_(f.vs[c], id, v + dv[c] * 0.5);
+            std_(f.accv[c], id, ldd(f.accv[c], id) + dv[c] * kThird);
+            std_(f.us[c], id, src ? f.src_val : u + du * 0.5);
+            std_(f.accu[c], id, ldd(f.accu[c], id) + du * kThird);
+        } else {
+            std_(f.vs[c], id, v + dv[c]);
+            std_(f.accv[c], id, ldd(f.accv[c], id) + dv[c] * kThird);
+            std_(f.us[c], id, src ? f.src_val : u + du);
+            std_(f.accu[c], id, ldd(f.accu[c], id) + du * kThird);
         }
     }
 }
 
-// --------------------------------------------------------------- history
-__global__ void __launch_bounds__(256) el_history_kernel(ElHistArgs a) {
-    const int64_t nxy = a.nx * a.ny;
-    const int64_t t = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (t >= kHistPlanes * 3 * nxy) return;
-    const int64_t ij = t % nxy;
-    const int pc = static_cast<int>(t / nxy);   // plane * 3 + comp
-    const int p = pc / 3, c = pc % 3;
-    a.slot[t] = a.u[c][ij * a.nz + a.planes[p]];
+template <class I>
+__global__ void __launch_bounds__(kGroup) el_force_kernel(ElStageArgs a) {
+    extern __shared__ double ctab[];   // the materials' constants (load_ctab)
+    el_force_group<I>(a, ctab, blockIdx.x);
+}
+
+// The ferromagnet's stage and the elastic force in one launch: the magnet
+// reads the strain the prep launch wrote and its own stores, the force reads
+// the stress parts of the same launch, and neither reads what the other
+// writes.  The magnet's workgroups (over the list of FM cells when some
+// cells are not FM) come first: their chain is the longer one.  On 70k cells
+// (45x38x41) each launch is mostly latency, and the magnet's 7.8 us hide in
+// the force's: 60 steps 7.66 -> 6.34 ms; 128x128x64: 45.5 -> 43.7 ms.
+__global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, StageArgs m, const uint32_t* ids,
+                                                              uint32_t count, unsigned mag_groups) {
+    extern __shared__ double ctab[];   // the materials' constants (load_ctab)
+    if (blockIdx.x >= mag_groups) {
+        el_force_group<uint32_t>(a, ctab, blockIdx.x - mag_groups);
+        return;
+    }
+    const uint32_t t = blockIdx.x * kGroup + threadIdx.x;
+    if (t >= count) return;
+    if (ids) fm_point<uint32_t>(m, ldu(ids, t));
+    else fm_point<uint32_t, true>(m, t);
 }
 
 // -------------------------------------------------------------- boundary
@@ -542,39 +591,28 @@ __global__ void __launch_bounds__(256) el_boundary_kernel(ElBoundaryArgs a) {
     const int64_t ij = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (ij >= nxy) return;
     const int64_t col = ij * nz;
-    auto hist = [&](int slot, int plane, int c) { return a.t[slot][(plane * 3 + c) * nxy + ij]; };
-    if (a.liao) {
-        // fourth-order Liao extrapolation from planes 1..4 of t1..t4
-        const double w = a.w;
+    auto hist = [&](int plane, int c) { return a.t1[(plane * 3 + c) * nxy + ij]; };
+    if (a.mur_bottom) {
         for (int c = 0; c < 3; c++) {
-            const double val = (4. * w + 2. * (1. - w)) * hist(0, 0, c) - (6. * w + (1. - w)) * hist(1, 1, c) +
-                               (4. * w) * hist(2, 2, c) - w * hist(3, 3, c);
-            a.u[c][col] = val;
-            if (a.kind == 2) a.us[c][col] = val;
-        }
-    } else {
-        if (a.mur_bottom) {
-            for (int c = 0; c < 3; c++) {
-                const double cc = c == 2 ? a.cb_l : a.cb_t;
-                if (a.kind < 2) {
-                    a.us[c][col] = a.u[c][col + 1] + cc * (a.u[c][col] - a.us[c][col + 1]);
-                } else {
-                    const double val = hist(0, 1, c) + cc * (hist(0, 0, c) - a.u[c][col + 1]);
-                    a.u[c][col] = val;
-                    a.us[c][col] = val;
-                }
-            }
-        }
-        for (int c = 0; c < 3; c++) {
-            const double cc = c == 2 ? a.ct_l : a.ct_t;
-            const int64_t top = col + nz - 1, below = col + nz - 2;
+            const double cc = c == 2 ? a.cb_l : a.cb_t;
             if (a.kind < 2) {
-                a.us[c][top] = a.u[c][below] + cc * (a.u[c][top] - a.us[c][below]);
+                a.us[c][col] = a.u[c][col + 1] + cc * (a.u[c][col] - a.us[c][col + 1]);
             } else {
-                const double val = hist(0, 2, c) + cc * (hist(0, 3, c) - a.u[c][below]);
-                a.u[c][top] = val;
-                a.us[c][top] = val;
+                const double val = hist(1, c) + cc * (hist(0, c) - a.u[c][col + 1]);
+                a.u[c][col] = val;
+                a.us[c][col] = val;
             }
+        }
+    }
+    for (int c = 0; c < 3; c++) {
+        const double cc = c == 2 ? a.ct_l : a.ct_t;
+        const int64_t top = col + nz - 1, below = col + nz - 2;
+        if (a.kind < 2) {
+            a.us[c][top] = a.u[c][below] + cc * (a.u[c][top] - a.us[c][below]);
+        } else {
+            const double val = hist(2, c) + cc * (hist(3, c) - a.u[c][below]);
+            a.u[c][top] = val;
+            a.us[c][top] = val;
         }
     }
     if (a.src_k >= 0 && solid(a.code, col + a.src_k)) {
@@ -597,34 +635,45 @@ hipError_t launch_el_strain(const ElStrainArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-hipError_t launch_el_stage(const ElStageArgs& a, hipStream_t s) {
+static size_t el_lds(const ElStageArgs& a) {
+    return sizeof(double) * kLdsPerMat * static_cast<size_t>(a.f.nmat > 0 ? a.f.nmat : 1);
+}
+
+// Up to 255 materials: 96 KiB of the CU's 160 KiB.
+static hipError_t allow_lds(const void* kernel, size_t lds) {
+    if (lds <= 65536) return hipSuccess;
+    return hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+}
+
+hipError_t launch_el_prep(const ElStageArgs& a, hipStream_t s) {
     const bool general = a.s.rotate || a.e.rotate || a.e.flexo;
-    const void* prep = general ? reinterpret_cast<const void*>(el_prep_kernel<true>)
-                               : reinterpret_cast<const void*>(el_prep_kernel<false>);
-    // 32-bit element offsets where they reach: 124 VGPRs and 4 waves per SIMD
-    // for the force launch against 129 and 3 with 64-bit ones
-    const bool n32 = narrow(a.f.nx * a.f.ny * a.f.nz);
-    const void* force = n32 ? reinterpret_cast<const void*>(el_force_kernel<uint32_t>)
-                            : reinterpret_cast<const void*>(el_force_kernel<int64_t>);
-    const size_t lds = sizeof(double) * kLdsPerMat * static_cast<size_t>(a.f.nmat > 0 ? a.f.nmat : 1);
-    if (lds > 65536) {   // up to 255 materials: 96 KiB of the CU's 160 KiB
-        hipError_t e = hipFuncSetAttribute(prep, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e == hipSuccess)
-            e = hipFuncSetAttribute(force, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) return e;
-    }
-    const dim3 grid(blocks_for(a.f.nx * a.f.ny * a.f.nz));
-    if (general) hipLaunchKernelGGL(el_prep_kernel<true>, grid, dim3(256), lds, s, a);
-    else hipLaunchKernelGGL(el_prep_kernel<false>, grid, dim3(256), lds, s, a);
-    hipError_t e = hipGetLastError();
+    const auto prep = general ? el_prep_kernel<true> : el_prep_kernel<false>;
+    const size_t lds = el_lds(a);
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(prep), lds);
     if (e != hipSuccess) return e;
-    if (n32) hipLaunchKernelGGL(el_force_kernel<uint32_t>, grid, dim3(256), lds, s, a);
-    else hipLaunchKernelGGL(el_force_kernel<int64_t>, grid, dim3(256), lds, s, a);
+    hipLaunchKernelGGL(prep, dim3(blocks_for(a.f.nx * a.f.ny * a.f.nz)), dim3(kGroup), lds, s, a);
     return hipGetLastError();
 }
 
-hipError_t launch_el_history(const ElHistArgs& a, hipStream_t s) {
-    hipLaunchKernelGGL(el_history_kernel, dim3(blocks_for(kHistPlanes * 3 * a.nx * a.ny)), dim3(256), 0, s, a);
+hipError_t launch_el_force(const ElStageArgs& a, hipStream_t s) {
+    // 32-bit element offsets where they reach
+    const auto force = narrow(a.f.nx * a.f.ny * a.f.nz) ? el_force_kernel<uint32_t> : el_force_kernel<int64_t>;
+    const size_t lds = el_lds(a);
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(force), lds);
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(force, dim3(blocks_for(a.f.nx * a.f.ny * a.f.nz)), dim3(kGroup), lds, s, a);
+    return hipGetLastError();
+}
+
+// Grids of fewer than 2^28 cells (narrow); ids and count as launch_mag_stage.
+hipError_t launch_el_force_mag(const ElStageArgs& a, const StageArgs& m, const uint32_t* ids, int64_t count,
+                               hipStream_t s) {
+    const size_t lds = el_lds(a);
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(el_force_mag_kernel), lds);
+    if (e != hipSuccess) return e;
+    const unsigned mg = blocks_for(count);
+    hipLaunchKernelGGL(el_force_mag_kernel, dim3(mg + blocks_for(a.f.nx * a.f.ny * a.f.nz)), dim3(kGroup), lds, s, a, m,
+                       ids, static_cast<uint32_t>(count), mg);
     return hipGetLastError();
 }
 

@@ -312,7 +312,26 @@ struct ElForceArgs {
     int32_t trac_k;         // plane of a traction pulse, -1 when off
     int32_t trac_row;       // 0, 1, 2 for a traction along x, y, z (stress xz, yz, zz)
     double trac_amp;
+    // the Liao plane k = 0 (liao set: not with Mur planes) from planes 1..4
+    // of the history slots t1..t4, and the displacement source (not with Mur
+    // planes either: src_k is -1 then)
+    const double* hist[4];
+    double w;               // Liao weight of the fourth-order term
+    int32_t liao;
+    int32_t src_comp;
+    int64_t src_k;          // source plane written this stage, -1 when none
+    double src_val;
     int32_t nmat;           // material records (their stiffness matrices are staged in LDS)
+};
+
+// Displacement history of the absorbing boundary: slot = [plane][comp][nx*ny]
+// with the four planes k = 1..4 (Liao) or k = 0, 1, nz-2, nz-1 (Mur).
+constexpr int kHistPlanes = 4;
+
+struct ElHistArgs {
+    const double* u[3];
+    double* slot;           // null when the planes are not kept this stage
+    int32_t planes[kHistPlanes];
 };
 
 // One elastic stage (two launches): the face gradients and strain of the
@@ -327,6 +346,7 @@ struct ElStageArgs {
     ElStrainArgs s;
     ElEigenArgs e;
     ElForceArgs f;
+    ElHistArgs h;
     double* px[3];
     double* py[3];
     double* pz[3];
@@ -334,27 +354,15 @@ struct ElStageArgs {
     int32_t e0_out;
 };
 
-// Displacement history of the absorbing boundary: slot = [plane][comp][nx*ny]
-// with the four planes k = 1..4 (Liao) or k = 0, 1, nz-2, nz-1 (Mur).
-constexpr int kHistPlanes = 4;
-
-struct ElHistArgs {
-    const double* u[3];
-    double* slot;
-    int64_t nx, ny, nz;
-    int32_t planes[kHistPlanes];
-};
-
+// Mur planes (and the displacement source) after an elastic update.
 struct ElBoundaryArgs {
     const uint32_t* code;
     double* u[3];
     double* us[3];
-    const double* t[4];     // slots of t1..t4 (Mur reads t1 only)
+    const double* t1;       // history slot of t1
     int64_t nx, ny, nz;
     int32_t kind;           // 0 = stages 1-2, 1 = stage 3, 2 = after the step
-    int32_t liao;           // 1 = Liao at k = 0, 0 = Mur
     int32_t mur_bottom;     // Mur also at k = 0
-    double w;               // Liao weight of the fourth-order term
     double cb_l, cb_t, ct_l, ct_t;   // Mur coefficients, bottom/top, long/trans
     int32_t src_k;          // source plane written this call, -1 when none
     int32_t src_comp;
@@ -691,6 +699,11 @@ struct gf_ctx {
     double* em_dm1[3] = {};
     double* em_dm2[3] = {};
     const double* fe_q_used[3] = {}; // q store read by the last ferroelectric stage
+    // gf_step with elastodynamics and a ferromagnet: the elastic force is
+    // deferred and runs in the magnet stage's launch, which comes next
+    bool el_defer = false;
+    bool el_pending = false;
+    gf::ElStageArgs el_args{};
     // gf_step with a ferroelectric and electrodynamics: the FE stage's
     // launch is deferred and runs in the EM stage's Ampere/Faraday launch
     bool fe_defer = false;
@@ -807,8 +820,11 @@ hipError_t launch_fe_stage(const FeStageArgs& a, int64_t n, hipStream_t s);
 
 // elastodynamics (gf_elastic.hip)
 hipError_t launch_el_strain(const ElStrainArgs& a, hipStream_t s);
-hipError_t launch_el_stage(const ElStageArgs& a, hipStream_t s);
-hipError_t launch_el_history(const ElHistArgs& a, hipStream_t s);
+// an elastic stage is prep, then force (alone, or with the ferromagnet's stage)
+hipError_t launch_el_prep(const ElStageArgs& a, hipStream_t s);
+hipError_t launch_el_force(const ElStageArgs& a, hipStream_t s);
+hipError_t launch_el_force_mag(const ElStageArgs& a, const StageArgs& m, const uint32_t* ids, int64_t count,
+                               hipStream_t s);
 hipError_t launch_el_boundary(const ElBoundaryArgs& a, hipStream_t s);
 
 // electrodynamics (gf_em.hip)

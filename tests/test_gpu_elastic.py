@@ -109,6 +109,19 @@ def test_elastic_stages_liao_with_source(rotate):
     o.close()
 
 
+@pytest.mark.parametrize("shape,source", [((1, 1, 5), None), ((5, 3, 9), (1, 0, "z")), ((3, 9, 5), (2, 4, "y")),
+                                          ((4, 3, 64), (3, 63, "x")), ((2, 5, 65), (1, 64, "z"))])
+def test_elastic_stages_column_edges(shape, source):
+    """Columns shorter than, equal to and just longer than a wave, ny below
+    nz (the stress wraps inside the column at k = ny-1) and above it, one cell
+    across; the source on the Liao plane and on the top plane."""
+    prob = elastic_block(shape=shape, source=source)
+    u, v = random_uv(prob.shape, 8)
+    g, o = run_stages(prob, {FIELD_U: u, FIELD_V: v}, nsteps=3)
+    g.close()
+    o.close()
+
+
 @pytest.mark.parametrize("flags,source", [(FLAG_1D_ABC, (2, 0, "z")),
                                           (FLAG_1D_ABC | FLAG_1D_ABC_ELAST_ONLYTOP, (3, 11, "y")),
                                           (FLAG_1D_ABC, (3, 11, "z"))])
@@ -150,6 +163,31 @@ def test_magnetoelastic_stages(rotate):
     g, o = run_stages(prob, {FIELD_M: m, FIELD_U: u, FIELD_V: v}, nsteps=2, phys=("el", "fm"),
                       check=(FIELD_M_STORE,))
     np.testing.assert_allclose(g.download(FIELD_M), o.get(FIELD_M), rtol=0, atol=1e-12)
+    g.close()
+    o.close()
+
+
+@pytest.mark.parametrize("shape,layers,flags", [((1, 1, 5), 2, 0), ((3, 5, 17), 17, 0), ((4, 16, 16), 4, 0),
+                                                ((5, 3, 33), 7, 0), ((2, 7, 9), 3, FLAG_1D_ABC)])
+def test_magnetoelastic_steps_at_group_edges(shape, layers, flags):
+    """gf_step runs the magnet's cells and the elastic force as workgroups of
+    one launch (with Mur planes as two launches): magnets of a few cells, of
+    exactly one workgroup and of every cell, against the oracle (the per-stage
+    bound)."""
+    from oracle.oracle import Oracle
+    prob, m = magnetoelastic(shape=shape, layers=layers)
+    prob.flags |= flags
+    u, v = random_uv(shape, 9)
+    say("case magnetoelastic steps", shape, layers, hex(prob.flags))
+    g, o = Context(prob), Oracle(prob)
+    for fid, val in ((FIELD_M, m), (FIELD_U, u), (FIELD_V, v)):
+        g.upload(fid, val)
+        o.set(fid, val)
+    g.step(3)
+    o.step(3)
+    assert np.abs(g.download(FIELD_M) - o.get(FIELD_M)).max() <= 1e-12
+    for fid in (FIELD_U, FIELD_V):
+        assert rel(g.download(fid), o.get(fid)) <= 1e-12, fid
     g.close()
     o.close()
 
