@@ -337,7 +337,7 @@ template <bool kGeneral>
 __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
     load_ctab(ctab, a.e.mats, a.f.nmat);
-    const int64_t id = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    const int64_t id = static_cast<int64_t>(xcd_group(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     if (id >= a.s.nx * a.s.ny * a.s.nz) return;
     int64_t i, j, k;
     cell_ijk(id, a.s.ny, a.s.nz, i, j, k);
@@ -562,7 +562,7 @@ __device__ __forceinline__ void el_force_group(const ElStageArgs& a, double* cta
 template <class I>
 __global__ void __launch_bounds__(kGroup) el_force_kernel(ElStageArgs a) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
-    el_force_group<I>(a, ctab, blockIdx.x);
+    el_force_group<I>(a, ctab, xcd_group(blockIdx.x, gridDim.x));
 }
 
 // The ferromagnet's stage and the elastic force in one launch: the magnet
@@ -576,7 +576,7 @@ __global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, Sta
                                                               uint32_t count, unsigned mag_groups) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
     if (blockIdx.x >= mag_groups) {
-        el_force_group<uint32_t>(a, ctab, blockIdx.x - mag_groups);
+        el_force_group<uint32_t>(a, ctab, xcd_group(blockIdx.x - mag_groups, gridDim.x - mag_groups));
         return;
     }
     const uint32_t t = blockIdx.x * kGroup + threadIdx.x;

@@ -72,9 +72,7 @@ __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, Fused
     double2* cbuf = tw + (nz >> 1);          // [3][pairs][nz], element i at slot fpad(i)
     DevMaterial* ltab = reinterpret_cast<DevMaterial*>(cbuf + fft_lds_elems(3 * pairs * nz));
     const int tid = threadIdx.x, bd = blockDim.x;
-    const unsigned b = blockIdx.x, G = gridDim.x;
-    const unsigned q = G / 8u, r = G % 8u, xcd = b % 8u, slot = b / 8u;
-    const unsigned L = xcd * q + (xcd < r ? xcd : r) + slot;
+    const unsigned L = xcd_group(blockIdx.x, gridDim.x);
     const int gpx = ny / P;
     const int x = static_cast<int>(L) / gpx, y0 = (static_cast<int>(L) % gpx) * P;
     const int cells = P * nz;
