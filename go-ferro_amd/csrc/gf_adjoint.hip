@@ -33,7 +33,7 @@
 // only the first N - M steps are checkpointed.  The trajectory and the
 // gradients are the same bit for bit.  Per-cell gradient accumulators are summed once
 // at the end in a fixed order, so the gradients are deterministic.
-#include "gf_llg_dev.h"
+#include "gf_fm_dev.h"
 
 #include <algorithm>
 #include <cmath>
@@ -121,28 +121,39 @@ __device__ __forceinline__ void rot_t(const double T[3][3], double ix, double iy
     oz = T[0][2] * ix + T[1][2] * iy + T[2][2] * iz;
 }
 
+// Bound by the latency of its loads (3 waves per SIMD): the inputs go out
+// before the cell's code is known, the z neighbours come from the adjacent
+// lanes, and the gradient accumulators are read together, not each after the
+// write of the one before.  128x128x32: 39.2 -> 34.9 us.
 template <class I>
 __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
+    const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
+    const I col = id / nz, z = id - col * nz;
+    const I x = col / ny, y = col - x * ny;
+
+    // read before the cell's code is known (every index is in bounds)
     const uint32_t own = ldu(a.code, id);
+    const double yc[3] = {ldd(a.y[0], id), ldd(a.y[1], id), ldd(a.y[2], id)};
+    const P3 sp = {{a.y[0], a.y[1], a.y[2]}};
+    double nv[6][3];
+    uint32_t ncd[6];
+    gather6_lanes_load<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
+    const double kb0 = ldd(a.kbar[0], id), kb1 = ldd(a.kbar[1], id), kb2 = ldd(a.kbar[2], id);
+    const bool dem = a.hd[0] != nullptr;
+    const double hd0 = dem ? ldd(a.hd[0], id) : 0., hd1 = dem ? ldd(a.hd[1], id) : 0.;
+    const double hd2 = dem ? ldd(a.hd[2], id) : 0.;
+    gather6_lanes_shift<I>(z, nz, yc, own, nv, ncd);
     if (!(own & kIsFM)) {
         for (int c = 0; c < 3; c++) { std_(a.mbar[c], id, 0.); std_(a.hbar[c], id, 0.); }
         return;
     }
     GMat& M = mat_of(a.mats, own);
-    const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
-
-    const double mgx = ldd(a.y[0], id), mgy = ldd(a.y[1], id), mgz = ldd(a.y[2], id);
+    const double mgx = yc[0], mgy = yc[1], mgz = yc[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const P3 sp = {{a.y[0], a.y[1], a.y[2]}};
-    double nv[6][3];
-    uint32_t ncd[6];
-    gather6<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
     const Stencil st = stencil_core<true>(mgx, mgy, mgz, nv, ncd, a.mats, own, kFmSurfShift, -1, a.dx, a.dy, a.dz,
                                           M.Aex, M.Aex_self, M.dmi_slope);
     // exchange and interfacial DMI (zero without it) of the forward stage
@@ -184,7 +195,7 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     double ha0 = hac0, ha1 = hac1, ha2 = hac2;
     if (a.rotate) rot(a.Tc2g, hac0, hac1, hac2, ha0, ha1, ha2);
     double H0 = ha0 + hex0 + a.hext[0], H1 = ha1 + hex1 + a.hext[1], H2 = ha2 + hex2 + a.hext[2];
-    if (a.hd[0]) { H0 += ldd(a.hd[0], id); H1 += ldd(a.hd[1], id); H2 += ldd(a.hd[2], id); }
+    if (dem) { H0 += hd0; H1 += hd1; H2 += hd2; }
     double exx = 0., eyy = 0., ezz = 0., eyz = 0., exz = 0., exy = 0.;
     if (a.strain[0]) {
         exx = ldd(a.strain[0], id); eyy = ldd(a.strain[1], id); ezz = ldd(a.strain[2], id);
@@ -204,7 +215,6 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     double px, py, pz, qx, qy, qz;
     cross(mgx, mgy, mgz, H0, H1, H2, px, py, pz);
     cross(mgx, mgy, mgz, px, py, pz, qx, qy, qz);
-    const double kb0 = ldd(a.kbar[0], id), kb1 = ldd(a.kbar[1], id), kb2 = ldd(a.kbar[2], id);
     const double P = M.precess, Q = M.alpha_precess;
     const double qb0 = Q * kb0, qb1 = Q * kb1, qb2 = Q * kb2;
     double t0, t1, t2;
@@ -275,11 +285,16 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     // B1 at its own cells; the exchange field through the face coefficients
     // (its own faces and its interfaces)
     const bool mine = (own & kMatMask) == static_cast<uint32_t>(a.mat);
+    const bool me = mine && a.strain[0], drv = a.ghdrive[0] != nullptr;
+    // the accumulators are read together, before the first write
+    const double ga = mine ? ldd(a.galpha, id) : 0., gx0 = ldd(a.gaex, id), gb = me ? ldd(a.gb1, id) : 0.;
+    double gd[3] = {0., 0., 0.};
+    if (drv)
+        for (int c = 0; c < 3; c++) gd[c] = ldd(a.ghdrive[c], id);
     if (mine) {
         const double dP = -2. * a.alpha * P / (1. + a.alpha * a.alpha);
         const double dQ = P + a.alpha * dP;
-        std_(a.galpha, id,
-             ldd(a.galpha, id) + dP * (px * kb0 + py * kb1 + pz * kb2) + dQ * (qx * kb0 + qy * kb1 + qz * kb2));
+        std_(a.galpha, id, ga + dP * (px * kb0 + py * kb1 + pz * kb2) + dQ * (qx * kb0 + qy * kb1 + qz * kb2));
     }
     double gx = M.exch * (hb0 * exd0 + hb1 * exd1 + hb2 * exd2);
     if (mine && nxs + nys > 0) {
@@ -288,13 +303,12 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
         const double r = -M.dmi_slope / M.Aex * 0.5;
         gx += r * (M.dmi_pos * (hb0 * nxs * mgx + hb1 * nys * mgy) - M.dmi_neg * hb2 * (nxs + nys) * mgz);
     }
-    std_(a.gaex, id, ldd(a.gaex, id) + gx);
-    if (mine && a.strain[0])
-        std_(a.gb1, id, ldd(a.gb1, id) + -2. / kMu0 / M.Ms * (hc0 * exx * mx + hc1 * eyy * my + hc2 * ezz * mz));
-    if (a.ghdrive[0]) {
-        std_(a.ghdrive[0], id, ldd(a.ghdrive[0], id) + a.drive_s * hb0);
-        std_(a.ghdrive[1], id, ldd(a.ghdrive[1], id) + a.drive_s * hb1);
-        std_(a.ghdrive[2], id, ldd(a.ghdrive[2], id) + a.drive_s * hb2);
+    std_(a.gaex, id, gx0 + gx);
+    if (me) std_(a.gb1, id, gb + -2. / kMu0 / M.Ms * (hc0 * exx * mx + hc1 * eyy * my + hc2 * ezz * mz));
+    if (drv) {
+        std_(a.ghdrive[0], id, gd[0] + a.drive_s * hb0);
+        std_(a.ghdrive[1], id, gd[1] + a.drive_s * hb1);
+        std_(a.ghdrive[2], id, gd[2] + a.drive_s * hb2);
     }
     std_(a.mbar[0], id, mb0); std_(a.mbar[1], id, mb1); std_(a.mbar[2], id, mb2);
     std_(a.hbar[0], id, hb0); std_(a.hbar[1], id, hb1); std_(a.hbar[2], id, hb2);
@@ -317,28 +331,42 @@ struct AdjCombineArgs {
     double g;                      // loss gradient per probe cell (mode 1)
 };
 
+// As adj_point_kernel; a neighbour's constants are read only when it is of
+// another material.  128x128x32: 24.4 -> 22.4 us.
 template <class I>
 __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
+    const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
+    const I col = id / nz, z = id - col * nz;
+    const I x = col / ny, y = col - x * ny;
+    // Everything the cell reads, before its code is known and before the
+    // first write (every index is in bounds).
+    // the exchange part of the transposed Jacobian: the field at cell i is
+    // exch_i sum_j A_ij (y_j - y_i)/h^2, so cell j receives
+    // sum_i A_ij (exch_i Hbar_i - exch_j Hbar_j)/h^2, the stencil of
+    // exch Hbar (A_ij symmetric; a surface face carries nothing)
     const uint32_t own = ldu(a.code, id);
+    const P3 sp = {{a.hbar[0], a.hbar[1], a.hbar[2]}};
+    const double hb[3] = {ldd(a.hbar[0], id), ldd(a.hbar[1], id), ldd(a.hbar[2], id)};
+    double nv[6][3];
+    uint32_t ncd[6];
+    gather6_lanes_load<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
+    double mb[3], da[3], lam[3], acc[3];
+    const bool dem = a.dadj[0] != nullptr, step = a.mode != 0, later = step && a.mode != 4;
+    for (int c = 0; c < 3; c++) {
+        mb[c] = ldd(a.mbar[c], id);
+        da[c] = dem ? ldd(a.dadj[c], id) : 0.;
+        lam[c] = step ? ldd(a.lam[c], id) : 0.;
+        acc[c] = later ? ldd(a.acc[c], id) : 0.;
+    }
+    gather6_lanes_shift<I>(z, nz, hb, own, nv, ncd);
     if (!(own & kIsFM)) {
         if (a.mode == 0) for (int c = 0; c < 3; c++) std_(a.ybar[c], id, 0.);
         return;
     }
     GMat& M = mat_of(a.mats, own);
-    const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
-    // the exchange part of the transposed Jacobian: the field at cell i is
-    // exch_i sum_j A_ij (y_j - y_i)/h^2, so cell j receives
-    // sum_i A_ij (exch_i Hbar_i - exch_j Hbar_j)/h^2, the stencil of
-    // exch Hbar (A_ij symmetric; a surface face carries nothing)
-    const P3 sp = {{a.hbar[0], a.hbar[1], a.hbar[2]}};
-    double nv[6][3];
-    uint32_t ncd[6];
-    gather6<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
     // the DMI differences of the x and y neighbours that read this cell (a
     // face that is not a surface): a neighbour below reads it in its forward
     // slope (+), one above in its backward slope (-)
@@ -347,41 +375,43 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
         const double ih[2] = {1. / a.dx, 1. / a.dy};
         for (int f = 0; f < 4; f++) {
             if (((own >> (kFmSurfShift + f)) & 1u) || !(ncd[f] & kIsFM)) continue;
-            const DevMaterial& Mn = a.mats[(ncd[f] & kMatMask) - 1];
+            // the neighbour's own constants; its record is read only when it is another
+            double dn = M.dmi_neg, dp = M.dmi_pos;
+            if ((ncd[f] ^ own) & kMatMask) {
+                GMat& Mn = mat_of(a.mats, ncd[f]);
+                dn = Mn.dmi_neg; dp = Mn.dmi_pos;
+            }
             const double w = ((f & 1) ? -1. : 1.) * ih[f >> 1];
-            const double ga = Mn.dmi_neg * nv[f][2] * 0.5, td = Mn.dmi_pos * nv[f][f >> 1] * 0.5;
+            const double ga = dn * nv[f][2] * 0.5, td = dp * nv[f][f >> 1] * 0.5;
             yd[f >> 1] += w * ga;   // d_xx (x faces) or d_yy (y faces)
             yd[2] += w * td;        // d_zx or d_zy
         }
     }
     for (int f = 0; f < 6; f++) {
-        const double e = (ncd[f] & kIsFM) ? a.mats[(ncd[f] & kMatMask) - 1].exch : 0.;
+        double e = M.exch;
+        if ((ncd[f] ^ own) & kMatMask) e = (ncd[f] & kIsFM) ? mat_of(a.mats, ncd[f]).exch : 0.;
         for (int c = 0; c < 3; c++) nv[f][c] = e * nv[f][c];
     }
-    const Stencil st = stencil_core<false>(M.exch * ldd(a.hbar[0], id), M.exch * ldd(a.hbar[1], id),
-                                           M.exch * ldd(a.hbar[2], id), nv, ncd, a.mats, own, kFmSurfShift, -1, a.dx,
-                                           a.dy, a.dz, M.Aex, M.Aex_self, 0.);
+    const Stencil st = stencil_core<false>(M.exch * hb[0], M.exch * hb[1], M.exch * hb[2], nv, ncd, a.mats, own,
+                                           kFmSurfShift, -1, a.dx, a.dy, a.dz, M.Aex, M.Aex_self, 0.);
     const bool probe = x >= static_cast<I>(a.lo[0]) && x <= static_cast<I>(a.hi[0]) && y >= static_cast<I>(a.lo[1]) &&
                        y <= static_cast<I>(a.hi[1]) && z >= static_cast<I>(a.lo[2]) && z <= static_cast<I>(a.hi[2]);
     for (int c = 0; c < 3; c++) {
-        double yb = ldd(a.mbar[c], id) + st.ex[c] + yd[c];
-        if (a.dadj[0]) yb += M.Ms * ldd(a.dadj[c], id);
+        double yb = mb[c] + st.ex[c] + yd[c];
+        if (dem) yb += M.Ms * da[c];
         if (a.mode == 0) {
             std_(a.ybar[c], id, yb);
-            continue;
-        }
-        const double lam = ldd(a.lam[c], id);
-        if (a.mode == 4) {
-            std_(a.acc[c], id, lam + yb);
-            std_(a.kbar[c], id, lam / 3. + yb);
+        } else if (a.mode == 4) {
+            std_(a.acc[c], id, lam[c] + yb);
+            std_(a.kbar[c], id, lam[c] / 3. + yb);
         } else if (a.mode == 3) {
-            std_(a.acc[c], id, ldd(a.acc[c], id) + yb);
-            std_(a.kbar[c], id, lam / 3. + 0.5 * yb);
+            std_(a.acc[c], id, acc[c] + yb);
+            std_(a.kbar[c], id, lam[c] / 3. + 0.5 * yb);
         } else if (a.mode == 2) {
-            std_(a.acc[c], id, ldd(a.acc[c], id) + yb);
-            std_(a.kbar[c], id, lam / 6. + 0.5 * yb);
+            std_(a.acc[c], id, acc[c] + yb);
+            std_(a.kbar[c], id, lam[c] / 6. + 0.5 * yb);
         } else {
-            double l = ldd(a.acc[c], id) + yb;
+            double l = acc[c] + yb;
             if (c == 0 && probe) l += a.g;
             std_(a.lam[c], id, l);
             std_(a.kbar[c], id, l / 6.);
