@@ -706,6 +706,11 @@ gf_status em_setup(gf_ctx* c, const gf_desc* d) {
 double** e_store(gf_ctx* c, int sel) { return sel == 0 ? c->Eb : (sel == 1 ? c->Ea : c->Ebb); }
 double** h_store(gf_ctx* c, int sel) { return sel == 0 ? c->Hb : (sel == 1 ? c->Ha : c->Hbb); }
 
+// Walls normal to z only, and no PEC edges after them.
+bool em_only_z_walls(const gf_ctx* c) {
+    return !c->em_periodic_all && c->per[0] && c->per[1] && !c->per[2] && !c->em_pec_all && c->nz >= 2;
+}
+
 // Cell-centred E and/or H of the current stores (update_DE_cell /
 // update_DH_cell, EMdynamic_solver.cpp:3780-3826).
 gf_status em_cells(gf_ctx* c, bool do_e, bool do_h, const EmWallArgs* zwall = nullptr) {
@@ -1577,6 +1582,7 @@ std::string stage_io_conflict(const FeStageArgs& a) {
         }
         rd.add(a.estat[c], "Estat", c);
         rd.add(a.ecell[c], "E cell", c);
+        rd.add(a.es[c], "E store", c);
         rd.add(a.flexo[c], "flexo force", c);
         wr.add(a.pout[c], a.stage == 4 ? "p" : "next p store", c);
         wr.add(a.qout[c], a.stage == 4 ? "q" : "next q store", c);
@@ -1609,7 +1615,10 @@ FeStageArgs fe_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
         a.eigen0[i] = both ? c->e0t0[i] : nullptr;
     }
     const bool em_p = c->em_on && (c->flags & GF_FLAG_EM_BACKACTION_P);
-    for (int i = 0; i < 3; i++) a.ecell[i] = em_p ? c->Ecell[i] : nullptr;
+    for (int i = 0; i < 3; i++) {
+        a.ecell[i] = em_p && !c->cells_stale ? c->Ecell[i] : nullptr;
+        a.es[i] = em_p && c->cells_stale ? e_store(c, c->e_sel)[i] : nullptr;
+    }
     a.code = c->d_code; a.mats = c->d_mats;
     double** ps = fe_pstore(c, in_sel);
     double** qs = fe_qstore(c, in_sel);
@@ -1994,10 +2003,20 @@ gf_status gf_em_stage(gf_ctx* c, int stage) {
         if (write) jf_comp = c->jf_comp;
     }
     EmArgs a{};
-    // stage 4: the E update keeps the planes the Mur walls read before the
-    // combine (transfer_pointer, EMdynamic_AbsorbingBoundary.cpp:3-56)
-    const bool hist = stage == 4 && !c->em_periodic_all;
-    for (int i = 0; i < 3; i++) a.t1[i] = hist ? c->Et1[i] : nullptr;
+    const int kind = stage < 3 ? 0 : (stage == 3 ? 1 : 2);
+    // the E update keeps the planes the Mur walls read before the combine
+    // (transfer_pointer, EMdynamic_AbsorbingBoundary.cpp:3-56): at stage 4,
+    // or at stage 3 when the walls' own edges apply them
+    a.keep = !c->em_periodic_all && stage == (c->em_lean ? 3 : 4);
+    for (int i = 0; i < 3; i++) a.t1[i] = c->Et1[i];
+    if (c->em_lean && !c->em_periodic_all) {
+        a.zwall = 1;
+        const bool pec = c->flags & GF_FLAG_PEC_Z;
+        a.wall_zero[0] = pec || ((c->flags & GF_FLAG_1D_ABC) && (c->flags & GF_FLAG_1D_ABC_EM_ONLYTOP));
+        a.wall_zero[1] = pec;
+        a.wall_cf[0] = kind == 0 ? c->cf_bot_half : c->cf_bot;
+        a.wall_cf[1] = kind == 0 ? c->cf_top_half : c->cf_top;
+    }
     a.code = c->d_code; a.mats = c->d_mats;
     for (int i = 0; i < 3; i++) {
         a.es[i] = es[i]; a.hs[i] = hs[i];
@@ -2040,7 +2059,6 @@ gf_status gf_em_stage(gf_ctx* c, int stage) {
         st = hip_check(c, launch_em_jp(j, c->stream), "EM Jp");
         timer_end(c, GF_K_OTHER, ev);
     }
-    const int kind = stage < 3 ? 0 : (stage == 3 ? 1 : 2);
     // hard plane source (update_planeEM*, :3829-3883)
     if (!st && (c->flags & GF_FLAG_PLANE_EM)) {
         EmMiscArgs p{};
@@ -2057,10 +2075,9 @@ gf_status gf_em_stage(gf_ctx* c, int stage) {
     // Mur or PEC walls, x then y then z (EMdynamic_AbsorbingBoundary.cpp:58-874);
     // with only z walls (and no PEC edges after them) the cells launch
     // applies them to the edges it reads
-    const bool zwall_in_cells = !c->em_periodic_all && c->per[0] && c->per[1] && !c->per[2] && !c->em_pec_all &&
-                                c->nz >= 2;
+    const bool zwall_in_cells = em_only_z_walls(c);
     EmWallArgs zw{};
-    if (!c->em_periodic_all) {
+    if (!c->em_periodic_all && !c->em_lean) {
         for (int axis = 0; axis < 3 && !st; axis++) {
             if (c->per[axis]) continue;
             EmWallArgs w{};
@@ -2092,7 +2109,8 @@ gf_status gf_em_stage(gf_ctx* c, int stage) {
     if (st) return st;
     c->e_sel = out_e;
     c->h_sel = out_h;
-    st = em_cells(c, true, true, zwall_in_cells ? &zw : nullptr);
+    if (c->em_lean) c->cells_stale = true;
+    else st = em_cells(c, true, true, zwall_in_cells ? &zw : nullptr);
     // Ampere's law of stage 4 has read the stage current: now the step one
     if (!st && stage == 4 && c->spin_on) st = spin_pump_step(c);
     if (st) return st;
@@ -2144,6 +2162,10 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
         return set_error(c, GF_ERR_STATE, "gf_step called in the middle of a step");
     // the FE stage runs inside the EM stage's launch (they are independent)
     c->fe_defer = c->any_fe && c->em_on;
+    // and applies the z walls and forms the cells' E there, where nothing
+    // else reads the cell fields or writes E between two launches
+    c->em_lean = c->fe_defer && !c->any_fm && !c->any_afm && !c->jp_on && !c->spin_on && !c->em_pec_all &&
+                 !(c->flags & GF_FLAG_PLANE_EM) && (c->em_periodic_all || em_only_z_walls(c));
     // and the elastic force inside the FM stage's (Mur planes follow the
     // force at once, so it is not deferred with them)
     c->el_defer = c->el_on && c->any_fm && !c->demag.fused && !(c->flags & GF_FLAG_1D_ABC) && narrow(c->n);
@@ -2164,11 +2186,18 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
             c->fe_pending = false;
             c->el_defer = false;
             c->el_pending = false;
+            c->em_lean = false;
+            c->cells_stale = false;
             return st;
         }
     }
     c->el_defer = false;
     c->fe_defer = false;
+    c->em_lean = false;
+    if (c->cells_stale) {
+        c->cells_stale = false;
+        return em_cells(c, true, true);
+    }
     return GF_OK;
 }
 

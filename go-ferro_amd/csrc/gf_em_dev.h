@@ -114,6 +114,18 @@ __device__ __forceinline__ double edge_increment(const EmArgs& a, const double* 
     return a.ce / er * (curl - Jf - Jp - Ji - cond * e_store - dP * a.rdt);
 }
 
+// The new value of the wall edge e of a z wall (top: k = nz) from its base yw,
+// the base y and the new value yn of the edge next to it, in: the first-order
+// Mur condition, or zero (EMdynamic_AbsorbingBoundary.cpp:58-874).  At stage 4
+// the bases are those kept at stage 3, since the edges overwrite theirs.
+template <class I>
+__device__ __forceinline__ double z_wall_edge(const EmArgs& a, int comp, bool top, I e, I in, double yw, double y,
+                                              double yn) {
+    if (a.wall_zero[top]) return 0.;
+    if (a.stage < 4) return y + a.wall_cf[top] * (yw - yn);
+    return ldd(a.t1[comp], in) + a.wall_cf[top] * (ldd(a.t1[comp], e) - yn);
+}
+
 // Ampere on edge e of the concatenated Ex|Ey|Ez grids, with its RK update.
 // Everything an edge reads (its base, accumulator and store, the H store
 // around it, its cells' codes and q store) is loaded before any of it is
@@ -132,15 +144,17 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     auto HY = [&](I i, I j, I k) { return (i * (ny + 1) + j) * nz + k; };
     auto HZ = [&](I i, I j, I k) { return (i * ny + j) * (nz + 1) + k; };
     auto near = [](I v, I n) { return v <= 1 || v >= n - 1; };
-    int comp;
+    int comp, wall = 0;   // -1, 1: an edge of the bottom, top z wall whose thread takes the one next to it first
     bool hist, dead;      // on a plane a Mur wall reads (two next to each non-periodic wall); a wall edge
     I cell[4], ci[4], cj[4], ck[4], hp[4];
     int hf[2];            // curl = (H_hf0[hp0] - H_hf0[hp1]) rh0 - (H_hf1[hp2] - H_hf1[hp3]) rh1
     double rh[2];
     if (e < nEx) {
         comp = 0;
-        const I l = e / (nz + 1), k = e - l * (nz + 1), i = l / (ny + 1), j = l - i * (ny + 1);
+        const I l = e / (nz + 1), i = l / (ny + 1), j = l - i * (ny + 1);
+        I k = e - l * (nz + 1);
         hist = (!a.per[1] && near(j, ny)) || (!a.per[2] && near(k, nz));
+        if (a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
         const bool wj = j == 0 || j == ny, wk = k == 0 || k == nz;
         dead = (wj && !a.per[1]) || (wk && !a.per[2]);
         const I y1 = wj ? ny - 1 : j - 1, y3 = wj ? 0 : j, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
@@ -150,8 +164,10 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     } else if (e < nEx + nEy) {
         comp = 1;
         e -= nEx;
-        const I l = e / (nz + 1), k = e - l * (nz + 1), i = l / ny, j = l - i * ny;
+        const I l = e / (nz + 1), i = l / ny, j = l - i * ny;
+        I k = e - l * (nz + 1);
         hist = (!a.per[0] && near(i, nx)) || (!a.per[2] && near(k, nz));
+        if (a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
         const bool wi = i == 0 || i == nx, wk = k == 0 || k == nz;
         dead = (wi && !a.per[0]) || (wk && !a.per[2]);
         const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
@@ -170,7 +186,15 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         hf[0] = 1; hf[1] = 0; rh[0] = a.rdx; rh[1] = a.rdy;
         hp[0] = HY(x3, y2, k); hp[1] = HY(x1, y2, k); hp[2] = C(x3, y2, k); hp[3] = C(x3, y1, k);
     }
-    const double y = ldd(a.eb[comp], e), es = ldd(a.es[comp], e), ac = a.stage > 1 ? ldd(a.eacc[comp], e) : 0.;
+    // in: the edge whose increment this thread evaluates.  A wall's thread
+    // reads what its neighbour's own thread may write in this launch only at
+    // the stages where it does not (the base before stage 4, the accumulator
+    // at stage 4).
+    const I in = wall == 0 ? e : (wall < 0 ? e + 1 : e - 1);
+    const bool last = a.stage == 4;
+    const double y = wall && last ? 0. : ldd(a.eb[comp], in), es = ldd(a.es[comp], in);
+    const double yw = wall && !last ? ldd(a.eb[comp], e) : 0.;
+    const double ac = (wall ? last : a.stage > 1) ? ldd(a.eacc[comp], in) : 0.;
     uint32_t tq[4];
     double qv[4] = {0., 0., 0., 0.}, hv[4];
     for (int q = 0; q < 4; q++) {
@@ -185,10 +209,17 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     if (!dead)
         k_ = edge_increment<I>(a, tab, comp, cell, ci, cj, ck, tq, qv, (hv[0] - hv[1]) * rh[0] - (hv[2] - hv[3]) * rh[1],
                                es);
-    // stage 4: the base value before the combine overwrites it, for the
-    // Mur walls (transfer_pointer, EMdynamic_AbsorbingBoundary.cpp:3-56);
-    // each edge's own thread reads and then writes its base
-    if (a.t1[0] && hist) std_(a.t1[comp], e, y);
+    if (wall) {
+        const double yn = last ? ac + k_ * kSixth : y + (a.stage == 3 ? k_ : k_ * 0.5);
+        std_(last ? a.eb[comp] : a.eo[comp], e, z_wall_edge<I>(a, comp, wall > 0, e, in, yw, y, yn));
+        if (a.stage == 1) std_(a.eacc[comp], e, yw);
+        if (a.keep) std_(a.t1[comp], e, yw);
+        return;
+    }
+    // the base value before the combine overwrites it, for the Mur walls
+    // (transfer_pointer, EMdynamic_AbsorbingBoundary.cpp:3-56); each edge's
+    // own thread reads and then writes its base
+    if (a.keep && hist) std_(a.t1[comp], e, y);
     rk_state<I>(a.stage, e, k_, y, ac, a.eb[comp], a.eacc[comp], a.eo[comp]);
 }
 

@@ -149,7 +149,13 @@ struct EmArgs {
     const double* dma1[3];
     const double* dma2[3];
     const double* jishe[2];     // inverse spin Hall current Jx, Jy, null when off
-    double* t1[3];              // stage 4 with Mur walls: E of the planes the walls read, kept before the combine
+    double* t1[3];              // Mur walls: E of the planes the walls read, kept before the combine
+    int32_t keep;               // this stage keeps them
+    // the z walls applied by their own edges' threads (z_wall_edge), with x
+    // and y periodic and nz >= 2
+    int32_t zwall;
+    int32_t wall_zero[2];       // the bottom / top wall is held at zero
+    double wall_cf[2];          // Mur coefficients of the bottom / top wall
     int64_t nx, ny, nz;
     double dt, ce, rdt;         // time step, dt / eps0, 1 / dt
     double rdx, rdy, rdz;       // 1/dx, 1/dy, 1/dz
@@ -415,6 +421,7 @@ struct FeStageArgs {
     const double* strain0[6];   // static strain added to strain, or null
     const double* eigen0[6];    // static eigenstrain added to eigen, with strain0
     const double* ecell[3];     // electrodynamic E at the cells, null when uncoupled
+    const double* es[3];        // or the E store it is taken from, null when ecell is given or uncoupled
     const double* flexo[3];     // flexoelectric force of the stage, null when off
     int64_t nx, ny, nz;
     double dt;
@@ -719,6 +726,11 @@ struct gf_ctx {
     bool fe_defer = false;
     bool fe_pending = false;
     gf::FeStageArgs fe_args{};
+    // and, with no walls but z ones and nothing but the ferroelectric reading
+    // the cell fields, the stage's z walls and cell E too: the cell arrays
+    // are stale until gf_step's end then
+    bool em_lean = false;
+    bool cells_stale = false;
     int e_sel = 0, h_sel = 0, em_next_stage = 1;
     double cf_top_half = 0, cf_bot_half = 0, cf_x_half = 0, cf_y_half = 0;
     double cf_top = 0, cf_bot = 0, cf_x = 0, cf_y = 0;

@@ -107,25 +107,34 @@ def test_fe_em_stages(flags):
     o.close()
 
 
-@pytest.mark.parametrize("shape", [(1, 1, 9), (1, 2, 255), (2, 9, 64), (3, 5, 17), (8, 8, 12)])
-def test_fe_em_steps_at_group_edges(shape):
+@pytest.mark.parametrize("shape,flags", [((1, 1, 9), 0), ((1, 2, 255), FLAG_PEC_Z), ((2, 9, 64), 0),
+                                         ((3, 5, 17), FLAG_1D_ABC | FLAG_1D_ABC_EM_ONLYTOP), ((8, 8, 12), 0),
+                                         ((4, 6, 16), "periodic"), ((4, 6, 16), FLAG_PLANE_EM)])
+def test_fe_em_steps_at_group_edges(shape, flags):
     """gf_step runs the ferroelectric cells, the edges and the faces as whole
-    workgroups of one launch: grids whose three counts leave each kind's last
-    workgroup nearly empty, nearly full or alone, against the oracle (the
-    per-stage bound)."""
+    workgroups of one launch, with the z walls applied by their own edges and
+    the cells' E taken from the store (not beside a plane source): grids whose
+    three counts leave each kind's last workgroup nearly empty, nearly full or
+    alone, each kind of z wall and none, against the oracle (the per-stage
+    bound)."""
     from oracle.oracle import Oracle
-    prob, p, q = fe_film(shape=shape)
-    say("case fe + em steps", shape)
+    prob, p, q = fe_film(shape=shape, flags=0 if flags == "periodic" else flags)
+    if flags == "periodic":
+        prob.periodic = (True, True, True)
+    if flags == FLAG_PLANE_EM:
+        prob.planeEM_E, prob.planeEM_E_freq, prob.planeEM_source_z = (1e6, 2e6, 0.0), (1e12, 2e12, 1e12), 2
+    say("case fe + em steps", shape, flags)
     g, o = Context(prob), Oracle(prob)
     E = random_yee(shape, FIELD_E_EM, 1e6, 4)
     H = random_yee(shape, FIELD_H_EM, 3e3, 5)
     for fid, val in ((FIELD_P, p), (FIELD_Q, q), (FIELD_E_EM, E), (FIELD_H_EM, H)):
         g.upload(fid, val)
         o.set(fid, val)
-    g.step(3)
-    o.step(3)
-    for fid in (FIELD_P, FIELD_Q, FIELD_E_EM, FIELD_H_EM, FIELD_E_CELL):
-        assert rel(g.download(fid), o.get(fid)) <= 1e-12, fid
+    for steps in (1, 2):
+        g.step(steps)
+        o.step(steps)
+        for fid in (FIELD_P, FIELD_Q, FIELD_E_EM, FIELD_H_EM, FIELD_E_CELL, FIELD_H_CELL):
+            assert rel(g.download(fid), o.get(fid)) <= 1e-12, (fid, steps)
     g.close()
     o.close()
 
