@@ -1071,6 +1071,7 @@ gf_status gf_destroy(gf_ctx* c) {
         if (c->pec[a]) hipFree(c->pec[a]);
     if (c->jf_spatial) hipFree(c->jf_spatial);
     if (c->red_partial) hipFree(c->red_partial);
+    if (c->red_host) hipHostFree(c->red_host);
     if (c->d_code) hipFree(c->d_code);
     if (c->d_fm_ids) hipFree(c->d_fm_ids);
     if (c->d_mats) hipFree(c->d_mats);
@@ -1218,15 +1219,15 @@ static gf_status em_transfer(gf_ctx* c, int id, double* host, size_t count, bool
     size_t tot = 0;
     for (int q = 0; q < np; q++) tot += static_cast<size_t>(sizes[q]);
     if (count != tot) return set_error(c, GF_ERR_ARG, "count must be " + std::to_string(tot) + " for this field");
+    if (!up) return download_parts(c, parts, sizes, np, host);
     size_t o = 0;
     gf_status st = GF_OK;
     for (int q = 0; q < np && !st; q++) {
         const size_t b = sizeof(double) * static_cast<size_t>(sizes[q]);
-        st = up ? hip_check(c, hipMemcpyAsync(parts[q], host + o, b, hipMemcpyHostToDevice, c->stream), "upload")
-                : hip_check(c, hipMemcpyAsync(host + o, parts[q], b, hipMemcpyDeviceToHost, c->stream), "download");
+        st = hip_check(c, hipMemcpyAsync(parts[q], host + o, b, hipMemcpyHostToDevice, c->stream), "upload");
         o += static_cast<size_t>(sizes[q]);
     }
-    if (!st && up) {
+    if (!st) {
         // EMdynamic_initialize.cpp:376-404: the stores start equal to the
         // fields and the cell fields follow them
         if (id == GF_FIELD_E_EM) { c->e_sel = 0; c->em_next_stage = 1; st = em_cells(c, true, false); }
@@ -1241,7 +1242,7 @@ static gf_status em_transfer(gf_ctx* c, int id, double* host, size_t count, bool
         }
     }
     if (st) return st;
-    return hip_check(c, hipStreamSynchronize(c->stream), up ? "upload sync" : "download sync");
+    return hip_check(c, hipStreamSynchronize(c->stream), "upload sync");
 }
 
 gf_status gf_set_material(gf_ctx* c, int index, const gf_material* m) {
@@ -1355,12 +1356,8 @@ gf_status gf_download(gf_ctx* c, int id, double* host, size_t count) {
         if (st) return st;
     }
     if (id == GF_FIELD_HSTAT && (st = demag_materialize_h(c))) return st;
-    for (int a = 0; a < 3; a++) {
-        st = hip_check(c, hipMemcpyAsync(host + a * c->n, f[a], sizeof(double) * c->n, hipMemcpyDeviceToHost, c->stream),
-                       "download");
-        if (st) return st;
-    }
-    return hip_check(c, hipStreamSynchronize(c->stream), "download sync");
+    const int64_t n3[3] = {c->n, c->n, c->n};
+    return download_parts(c, f, n3, 3, host);
 }
 
 // global.cpp:513-549 (H drive table; t advances every call)
@@ -2203,23 +2200,25 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
 
 gf_status gf_average(gf_ctx* c, int id, double out[3]) {
     if (!c || !out) return GF_ERR_ARG;
-    gf_status st;
+    gf_status st = GF_OK;
     if (id != GF_FIELD_M && id != GF_FIELD_M_AFM1 && id != GF_FIELD_M_AFM2 && id != GF_FIELD_P)
         return set_error(c, GF_ERR_ARG, "average is defined for m, m_AFM1, m_AFM2, p");
     double** f = field_for(c, id, false, &st);
     if (!f) return st;
     const double* ff[3] = {f[0], f[1], f[2]};
-    st = hip_check(c, launch_sum3(ff, c->n, c->red_partial, c->red_blocks, c->stream), "sum");
-    if (st) return st;
-    std::vector<double> part(static_cast<size_t>(3 * c->red_blocks));
-    st = hip_check(c, hipMemcpyAsync(part.data(), c->red_partial, sizeof(double) * part.size(), hipMemcpyDeviceToHost,
-                                     c->stream), "sum copy");
+    // the partial sums go straight to host memory: no copy after the launch
+    const size_t sums = static_cast<size_t>(3 * c->red_blocks);
+    if (!c->red_host)
+        st = hip_check(c, hipHostMalloc(reinterpret_cast<void**>(&c->red_host), sizeof(double) * sums,
+                                        hipHostMallocDefault), "hipHostMalloc sums");
+    if (!st) st = hip_check(c, launch_sum3(ff, c->n, c->red_host, c->red_blocks, c->stream), "sum");
     if (!st) st = hip_check(c, hipStreamSynchronize(c->stream), "sum sync");
     if (st) return st;
+    const double* part = c->red_host;
     const double cnt = static_cast<double>(id == GF_FIELD_M ? c->nfm : (id == GF_FIELD_P ? c->nfe : c->nafm));
     for (int a = 0; a < 3; a++) {
         double s = 0.;
-        for (int64_t b = 0; b < c->red_blocks; b++) s += part[static_cast<size_t>(3 * b + a)];
+        for (int64_t b = 0; b < c->red_blocks; b++) s += part[3 * b + a];
         out[a] = s / cnt;
     }
     return GF_OK;

@@ -604,6 +604,18 @@ struct TimerSlot {
 
 }  // namespace gf
 
+namespace gf {
+// The pinned slots of download_parts live while any context does.
+void host_slots_retain();
+void host_slots_release();
+struct HostSlotsUser {
+    HostSlotsUser() { host_slots_retain(); }
+    ~HostSlotsUser() { host_slots_release(); }
+    HostSlotsUser(const HostSlotsUser&) = delete;
+    HostSlotsUser& operator=(const HostSlotsUser&) = delete;
+};
+}  // namespace gf
+
 struct gf_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -770,7 +782,9 @@ struct gf_ctx {
     double* e0t0[6] = {};           // static crystal-frame eigenstrain at t0 (elastodynamics), on first use
     // reduction scratch
     double* red_partial = nullptr;
+    double* red_host = nullptr;     // pinned, on first use: the partial sums of an average
     int64_t red_blocks = 0;
+    gf::HostSlotsUser slots_user;
 
     // Which buffer holds the store the next stage reads: 0 = m, 1 = a, 2 = b.
     int mag_store_sel = 0;
@@ -826,6 +840,10 @@ std::string stage_io_conflict(const AfmStageArgs& a);
 std::string stage_io_conflict(const FeStageArgs& a);
 // true when cell indices of an n-cell grid fit 32-bit byte offsets (gf_llg.hip)
 bool narrow(int64_t n);
+
+// device to host copies of whole fields (gf_hostio.hip): the parts of count[p]
+// doubles at src[p], one after another into host; waits for the stream
+gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* count, int parts, double* host);
 
 // launchers (gf_llg.hip)
 // ids: when set, the count FM cells the stage runs over (else all n cells)
