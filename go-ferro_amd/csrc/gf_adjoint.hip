@@ -84,7 +84,9 @@ struct AdjPointArgs {
     double* gb1;
     double* ghdrive[3];            // may be null
     int64_t nx, ny, nz;
-    double dx, dy, dz;
+    CellDiv div;
+    double idx, idy, idz;          // 1/dx, 1/dy, 1/dz
+    double ih2[3];                 // 1/dx^2, 1/dy^2, 1/dz^2
     double hext[3];
     double drive_s;
     double Tg2c[3][3];
@@ -131,8 +133,8 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
+    I x, y, z;
+    cell_xyz(a.div, id, ny, nz, x, y, z);
 
     // read before the cell's code is known (every index is in bounds)
     const uint32_t own = ldu(a.code, id);
@@ -154,7 +156,7 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const double mgx = yc[0], mgy = yc[1], mgz = yc[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil st = stencil_core<true>(mgx, mgy, mgz, nv, ncd, a.mats, own, kFmSurfShift, -1, a.dx, a.dy, a.dz,
+    const Stencil st = stencil_core<true>(mgx, mgy, mgz, nv, ncd, a.mats, own, kFmSurfShift, -1, a.idx, a.idy, a.idz,
                                           M.Aex, M.Aex_self, M.dmi_slope);
     // exchange and interfacial DMI (zero without it) of the forward stage
     const double hex0 = M.exch * st.ex[0] + M.dmi_pos * st.d[2], hex1 = M.exch * st.ex[1] + M.dmi_pos * st.d[3];
@@ -163,11 +165,10 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     // non-surface face's difference weighted by d(coefficient)/dAex
     double exd0 = 0., exd1 = 0., exd2 = 0.;
     {
-        const double ih2[3] = {1. / (a.dx * a.dx), 1. / (a.dy * a.dy), 1. / (a.dz * a.dz)};
         const uint32_t mi = own & kMatMask;
         for (int f = 0; f < 6; f++) {
             if ((own >> (kFmSurfShift + f)) & 1u) continue;
-            const double w = dcoef_dA(a.mats, mi, ncd[f] & kMatMask, static_cast<uint32_t>(a.mat)) * ih2[f >> 1];
+            const double w = dcoef_dA(a.mats, mi, ncd[f] & kMatMask, static_cast<uint32_t>(a.mat)) * a.ih2[f >> 1];
             exd0 += w * (nv[f][0] - mgx);
             exd1 += w * (nv[f][1] - mgy);
             exd2 += w * (nv[f][2] - mgz);
@@ -253,7 +254,7 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     {
         const double s = M.dmi_slope;
         const double ga = M.dmi_neg * hb2 * 0.5, al = M.dmi_pos * hb0 * 0.5, be = M.dmi_pos * hb1 * 0.5;
-        const double ix = 1. / a.dx, iy = 1. / a.dy;
+        const double ix = a.idx, iy = a.idy;
         const double kx = M.exch * M.Aex * s * ix, ky = M.exch * M.Aex * s * iy;
         const bool sf[4] = {((own >> (kFmSurfShift + kXB)) & 1u) != 0, ((own >> (kFmSurfShift + kXF)) & 1u) != 0,
                             ((own >> (kFmSurfShift + kYB)) & 1u) != 0, ((own >> (kFmSurfShift + kYF)) & 1u) != 0};
@@ -325,7 +326,8 @@ struct AdjCombineArgs {
     double* kbar[3];
     double* ybar[3];               // mode 0 output
     int64_t nx, ny, nz;
-    double dx, dy, dz;
+    CellDiv div;
+    double idx, idy, idz;          // 1/dx, 1/dy, 1/dz
     int32_t mode;                  // 0: ybar only; 1..4: RK4 bookkeeping after stage `mode`
     int32_t lo[3], hi[3];          // probe box
     double g;                      // loss gradient per probe cell (mode 1)
@@ -339,8 +341,8 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
+    I x, y, z;
+    cell_xyz(a.div, id, ny, nz, x, y, z);
     // Everything the cell reads, before its code is known and before the
     // first write (every index is in bounds).
     // the exchange part of the transposed Jacobian: the field at cell i is
@@ -372,7 +374,7 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     // slope (+), one above in its backward slope (-)
     double yd[3] = {0., 0., 0.};
     {
-        const double ih[2] = {1. / a.dx, 1. / a.dy};
+        const double ih[2] = {a.idx, a.idy};
         for (int f = 0; f < 4; f++) {
             if (((own >> (kFmSurfShift + f)) & 1u) || !(ncd[f] & kIsFM)) continue;
             // the neighbour's own constants; its record is read only when it is another
@@ -393,7 +395,7 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
         for (int c = 0; c < 3; c++) nv[f][c] = e * nv[f][c];
     }
     const Stencil st = stencil_core<false>(M.exch * hb[0], M.exch * hb[1], M.exch * hb[2], nv, ncd, a.mats, own,
-                                           kFmSurfShift, -1, a.dx, a.dy, a.dz, M.Aex, M.Aex_self, 0.);
+                                           kFmSurfShift, -1, a.idx, a.idy, a.idz, M.Aex, M.Aex_self, 0.);
     const bool probe = x >= static_cast<I>(a.lo[0]) && x <= static_cast<I>(a.hi[0]) && y >= static_cast<I>(a.lo[1]) &&
                        y <= static_cast<I>(a.hi[1]) && z >= static_cast<I>(a.lo[2]) && z <= static_cast<I>(a.hi[2]);
     for (int c = 0; c < 3; c++) {
@@ -546,7 +548,10 @@ void stage_point_args(gf_ctx* c, int material, AdjPointArgs& p) {
     for (int i = 0; i < 6; i++) strain[i] = sa.strain[i];
     for (int i = 0; i < 6; i++) p.strain[i] = strain[i];
     for (int i = 0; i < 3; i++) { p.hnu[i] = sa.hnu[i]; p.hdrive[i] = sa.hdrive[i]; }
-    p.nx = c->nx; p.ny = c->ny; p.nz = c->nz; p.dx = c->dx; p.dy = c->dy; p.dz = c->dz;
+    p.nx = c->nx; p.ny = c->ny; p.nz = c->nz;
+    p.div = make_cell_div(c->ny, c->nz);
+    p.idx = 1. / c->dx; p.idy = 1. / c->dy; p.idz = 1. / c->dz;
+    p.ih2[0] = 1. / (c->dx * c->dx); p.ih2[1] = 1. / (c->dy * c->dy); p.ih2[2] = 1. / (c->dz * c->dz);
     std::memcpy(p.Tg2c, c->Tg2c, sizeof(p.Tg2c));
     std::memcpy(p.Tc2g, c->Tc2g, sizeof(p.Tc2g));
     p.rotate = sa.rotate;
@@ -591,7 +596,9 @@ gf_status combine(gf_ctx* c, int mode, double* const* mbar, double* const* hbar,
         a.kbar[i] = kbar ? kbar[i] : nullptr; a.ybar[i] = ybar ? ybar[i] : nullptr;
         a.lo[i] = lo[i]; a.hi[i] = hi[i];
     }
-    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz;
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
+    a.div = make_cell_div(c->ny, c->nz);
+    a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     a.mode = mode; a.g = g;
     if (narrow(c->n)) hipLaunchKernelGGL(adj_combine_kernel<uint32_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, a);
     else hipLaunchKernelGGL(adj_combine_kernel<int64_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, a);

@@ -550,6 +550,7 @@ gf_status elastic_strain(gf_ctx* c) {
     for (int i = 0; i < 6; i++) { a.eg[i] = c->eg[i]; a.ec[i] = c->ec[i]; }
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz;
     a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
+    a.div = make_cell_div(c->ny, c->nz);
     for (int i = 0; i < 3; i++) a.per[i] = c->per[i];
     a.rotate = (c->flags & GF_FLAG_ORIENT_ROTATE) ? 1 : 0;
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
@@ -1411,7 +1412,9 @@ StageArgs fm_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
         a.hdrive[i] = c->hdrive[i];
         a.hcell[i] = em_m ? c->Hcell[i] : nullptr;
     }
-    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz;
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
+    a.div = make_cell_div(c->ny, c->nz);
+    a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
     std::memcpy(a.Tc2g, c->Tc2g, sizeof(a.Tc2g));
     a.rotate = (c->flags & GF_FLAG_ORIENT_ROTATE) ? 1 : 0;
@@ -1462,7 +1465,9 @@ AfmStageArgs afm_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
         a.out1[i] = o1[i]; a.out2[i] = o2[i];
         a.hstat[i] = hstat_live(c) ? c->hstat[i] : nullptr;
     }
-    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz;
+    a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
+    a.div = make_cell_div(c->ny, c->nz);
+    a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
     std::memcpy(a.Tc2g, c->Tc2g, sizeof(a.Tc2g));
     a.rotate = (c->flags & GF_FLAG_ORIENT_ROTATE) ? 1 : 0;
@@ -1628,6 +1633,7 @@ FeStageArgs fe_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
         a.flexo[i] = c->d_flexo ? c->flexo_force[i] : nullptr;
     }
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dt = c->dt;
+    a.div = make_cell_div(c->ny, c->nz);
     const double h[3] = {c->dx, c->dy, c->dz};
     for (int i = 0; i < 3; i++) a.rh2[i] = (1. / h[i]) * (1. / h[i]);
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
@@ -1856,6 +1862,7 @@ gf_status gf_elastic_stage(gf_ctx* c, int stage) {
         for (int i = 0; i < 6; i++) { a.eg[i] = c->eg[i]; a.ec[i] = c->ec[i]; }
         a.nx = c->nx; a.ny = c->ny; a.nz = c->nz; a.dx = c->dx; a.dy = c->dy; a.dz = c->dz;
         a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
+        a.div = make_cell_div(c->ny, c->nz);
         for (int i = 0; i < 3; i++) a.per[i] = c->per[i];
         a.rotate = rotate;
         std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));

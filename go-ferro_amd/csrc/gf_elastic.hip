@@ -56,16 +56,14 @@ __device__ __forceinline__ void rot_voigt(const double T[3][3], const double v[6
 }
 
 // ---------------------------------------------------------------- strain
-// (i, j, k) of cell id = (i ny + j) nz + k, by 32-bit divisions when the
-// index and ny nz fit 32 bits (64-bit divisions are emulated and slow).
-__device__ __forceinline__ void cell_ijk(int64_t id, int64_t ny, int64_t nz, int64_t& i, int64_t& j, int64_t& k) {
-    const int64_t nyz = ny * nz;
-    if (((id | nyz) >> 32) == 0) {
-        const uint32_t u = static_cast<uint32_t>(id), q = static_cast<uint32_t>(nyz), z = static_cast<uint32_t>(nz);
-        const uint32_t ii = u / q, r = u - ii * q, jj = r / z;
-        i = ii; j = jj; k = r - jj * z;
+// (i, j, k) of cell id, with 32-bit arithmetic when the grid is narrow.
+__device__ __forceinline__ void cell_ijk(const ElStrainArgs& a, int64_t id, int64_t& i, int64_t& j, int64_t& k) {
+    if (a.nx * a.ny * a.nz < (int64_t{1} << 28)) {
+        uint32_t x, y, z;
+        cell_xyz(a.div, static_cast<uint32_t>(id), static_cast<uint32_t>(a.ny), static_cast<uint32_t>(a.nz), x, y, z);
+        i = x; j = y; k = z;
     } else {
-        i = id / nyz; j = (id - i * nyz) / nz; k = id - i * nyz - j * nz;
+        cell_xyz(a.div, id, a.ny, a.nz, i, j, k);
     }
 }
 
@@ -169,7 +167,7 @@ __global__ void __launch_bounds__(256) el_strain_kernel(ElStrainArgs a) {
     const int64_t id = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
     if (id >= a.nx * a.ny * a.nz) return;
     int64_t i, j, k;
-    cell_ijk(id, a.ny, a.nz, i, j, k);
+    cell_ijk(a, id, i, j, k);
     double g[6][3], e[6];
     cell_grad(a, id, i, j, k, g);
     grad_out(a, i, j, k, g);
@@ -340,7 +338,7 @@ __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
     const int64_t id = static_cast<int64_t>(xcd_group(blockIdx.x, gridDim.x)) * blockDim.x + threadIdx.x;
     if (id >= a.s.nx * a.s.ny * a.s.nz) return;
     int64_t i, j, k;
-    cell_ijk(id, a.s.ny, a.s.nz, i, j, k);
+    cell_ijk(a.s, id, i, j, k);
     double g[6][3], e[6], e0[6] = {0., 0., 0., 0., 0., 0.}, sc[6];
     const uint32_t code = a.s.code[id];
     // the eigenstrain first: its loads then go out with the store's, before
@@ -397,7 +395,8 @@ __device__ __forceinline__ void el_force_group(const ElStageArgs& a, double* cta
     const I nx = static_cast<I>(f.nx), ny = static_cast<I>(f.ny), nz = static_cast<I>(f.nz);
     const I id = static_cast<I>(group) * kGroup + static_cast<I>(threadIdx.x);
     if (id >= nx * ny * nz) return;
-    const I cl = id / nz, k = id - cl * nz, i = cl / ny, j = cl - i * ny;
+    I i, j, k;
+    cell_xyz(a.s.div, id, ny, nz, i, j, k);
     const int stage = f.stage;
     const I ib = i == 0 ? nx - 1 : i - 1, iff = i == nx - 1 ? 0 : i + 1;
     const I jb = j == 0 ? ny - 1 : j - 1, jf = j == ny - 1 ? 0 : j + 1;

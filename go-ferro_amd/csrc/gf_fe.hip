@@ -62,7 +62,8 @@ __device__ __forceinline__ void fe_cell(const FeStageArgs& a, I id) {
     if (own & kIsFE) {
         const DevMaterial& M = a.mats[(own & kMatMask) - 1];
         const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-        const I l = id / nz, k = id - l * nz, i = l / ny, j = l - i * ny;
+        I i, j, k;
+        cell_xyz(a.div, id, ny, nz, i, j, k);
         const double c[3] = {ldd(a.pstore[0], id), ldd(a.pstore[1], id), ldd(a.pstore[2], id)};
         // Laplacian, mirror value across a surface face (ferroelectric_solver.cpp:4-131)
         double lap[3] = {0., 0., 0.};

@@ -129,8 +129,8 @@ __device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn
     double mx = mgx, my = mgy, mz = mgz;
     if (!kLean && a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
 
-    const Stencil st = stencil_core<true>(mgx, mgy, mgz, in.v, in.cd, mats, in.own, kFmSurfShift, -1, a.dx, a.dy,
-                                          a.dz, M.Aex, M.Aex_self, M.dmi_slope);
+    const Stencil st = stencil_core<true>(mgx, mgy, mgz, in.v, in.cd, mats, in.own, kFmSurfShift, -1, a.idx, a.idy,
+                                          a.idz, M.Aex, M.Aex_self, M.dmi_slope);
 
     // magnetocrystalline anisotropy (magnetic_solver.cpp:124-141)
     double hac0 = 0., hac1 = 0., hac2 = 0.;
@@ -199,8 +199,8 @@ __device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn
 template <class I, bool kLanes = false>
 __device__ __forceinline__ void fm_point(const StageArgs& a, I id) {
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
+    I x, y, z;
+    cell_xyz(a.div, id, ny, nz, x, y, z);
     FmIn in;
     fm_load<I, kLanes>(a, id, x, y, z, in);
     // a null Hstat is zero (no statics, nothing uploaded)

@@ -118,6 +118,48 @@ __device__ __forceinline__ uint32_t lane_down(uint32_t v) {
     return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), 0x130, 0xf, 0xf, false));
 }
 
+// Quotients by nz and ny of the 32-bit cell indices of grids narrow() accepts
+// (id < 2^28) as a multiplication each: q = hi32(id m) >> s with
+// s = ceil(log2 d) - 1 and m = ceil(2^(32+s) / d), which is exact while
+// id (m d - 2^(32+s)) < 2^(32+s): id < 2^28 and m d - 2^(32+s) < d <= 2^(s+1).
+// d = 1 has m = 0.  A 32-bit division is about 20 instructions here, and the
+// stages are half bound by their instructions: with this and the reciprocal
+// spacings passed in, 100x84x30 film 8.84 -> 8.58 ms for 40 steps, the elastic
+// stage of 128x128x64 39.4 -> 38.7 ms for 60.
+struct CellDiv {
+    uint32_t mz, sz, my, sy;
+};
+inline void cell_div_one(int64_t d, uint32_t& m, uint32_t& s) {
+    m = 0; s = 0;
+    if (d < 2 || d >= (int64_t{1} << 28)) return;   // wider axes belong to the 64-bit form
+    while ((int64_t{2} << s) < d) s++;
+    m = static_cast<uint32_t>(((uint64_t{1} << (32 + s)) + static_cast<uint64_t>(d) - 1) / static_cast<uint64_t>(d));
+}
+inline CellDiv make_cell_div(int64_t ny, int64_t nz) {
+    CellDiv d;
+    cell_div_one(nz, d.mz, d.sz);
+    cell_div_one(ny, d.my, d.sy);
+    return d;
+}
+__host__ __device__ __forceinline__ uint32_t cell_div_apply(uint32_t id, uint32_t m, uint32_t s) {
+    return m ? static_cast<uint32_t>((static_cast<uint64_t>(id) * m) >> 32) >> s : id;
+}
+// (x, y, z) of cell id = (x ny + y) nz + z
+__device__ __forceinline__ void cell_xyz(const CellDiv& d, uint32_t id, uint32_t ny, uint32_t nz, uint32_t& x,
+                                         uint32_t& y, uint32_t& z) {
+    const uint32_t col = cell_div_apply(id, d.mz, d.sz);
+    z = id - col * nz;
+    x = cell_div_apply(col, d.my, d.sy);
+    y = col - x * ny;
+}
+__device__ __forceinline__ void cell_xyz(const CellDiv&, int64_t id, int64_t ny, int64_t nz, int64_t& x, int64_t& y,
+                                         int64_t& z) {
+    const int64_t col = id / nz;
+    z = id - col * nz;
+    x = col / ny;
+    y = col - x * ny;
+}
+
 // Workgroup b of a launch of G, renumbered so that each XCD (workgroups are
 // dealt to the 8 XCDs round-robin) takes a contiguous range of the cells: a
 // cell's x and y neighbours are then mostly in its own XCD's L2.  Elastic
@@ -256,6 +298,7 @@ struct ElStrainArgs {
     double* eg[6];
     double* ec[6];          // may equal eg (no rotation)
     int64_t nx, ny, nz;
+    CellDiv div;
     double dx, dy, dz;
     double idx, idy, idz;   // 1/dx, 1/dy, 1/dz
     int32_t per[3];
@@ -425,6 +468,7 @@ struct FeStageArgs {
     const double* flexo[3];     // flexoelectric force of the stage, null when off
     int64_t nx, ny, nz;
     double dt;
+    CellDiv div;
     double rh2[3];              // 1 / spacing^2
     double eext[3];
     double Tg2c[3][3];
@@ -449,7 +493,8 @@ struct StageArgs {
     const double* hcell[3];     // electrodynamic H at the cells, null when uncoupled
     double* dm_out[3];          // k of this stage, null unless Faraday's law needs it
     int64_t nx, ny, nz;
-    double dx, dy, dz;
+    CellDiv div;
+    double idx, idy, idz;       // 1/dx, 1/dy, 1/dz
     double hext[3];
     double drive_s;             // sin(2 pi f t) of the shaped drive at the stage time
     double Tg2c[3][3];
@@ -479,7 +524,8 @@ struct AfmStageArgs {
     double* dm_out1[3];         // k of this stage per sublattice, null unless needed
     double* dm_out2[3];
     int64_t nx, ny, nz;
-    double dx, dy, dz;
+    CellDiv div;
+    double idx, idy, idz;       // 1/dx, 1/dy, 1/dz
     double hext[3];
     double Tg2c[3][3];
     double Tc2g[3][3];

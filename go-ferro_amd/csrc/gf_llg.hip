@@ -207,8 +207,8 @@ __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, Fused
 template <class I, bool kLanes = false>
 __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) {
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    const I col = id / nz, z = id - col * nz;
-    const I x = col / ny, y = col - x * ny;
+    I x, y, z;
+    cell_xyz(a.div, id, ny, nz, x, y, z);
     const P3 s1 = {{a.store1[0], a.store1[1], a.store1[2]}}, s2 = {{a.store2[0], a.store2[1], a.store2[2]}};
     const P3 st = sub == 0 ? s1 : s2;
     const P3 other = sub == 0 ? s2 : s1;
@@ -241,8 +241,8 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
     GMat& M = mat_of(a.mats, own);
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil s = stencil_core<false>(mgx, mgy, mgz, v, cd, (GMat*)a.mats, own, kAfmSurfShift, sub, a.dx, a.dy,
-                                          a.dz, M.aAex[sub], M.aAex_self[sub], 0.);
+    const Stencil s = stencil_core<false>(mgx, mgy, mgz, v, cd, (GMat*)a.mats, own, kAfmSurfShift, sub, a.idx, a.idy,
+                                          a.idz, M.aAex[sub], M.aAex_self[sub], 0.);
     // uniaxial anisotropy 2K1 (u.m) u (magnetic_AFM_solver.cpp:148-154)
     const double udotm = mx * M.u[0] + my * M.u[1] + mz * M.u[2];
     const double hac0 = 2. * M.aK1n[sub] * udotm * M.u[0];

@@ -112,16 +112,15 @@ __device__ __forceinline__ double face_coef(MP mats, uint32_t mat, uint32_t nc, 
 }
 
 // The stencil of get_m_spatial_derivative_local from the cell's store
-// (c0, c1, c2) and its gathered neighbours; see gather6.
+// (c0, c1, c2) and its gathered neighbours; see gather6.  ix, iy and iz are
+// the reciprocal spacings: each quotient moves by at most an ulp against the
+// reference's c/dx.
 template <bool kDmi, class MP>
 __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2, const double (&v)[6][3],
                                                 const uint32_t (&cd)[6], MP mats, uint32_t own,
-                                                int surf_shift, int sub, double dx, double dy, double dz, double A,
+                                                int surf_shift, int sub, double ix, double iy, double iz, double A,
                                                 double A_self, double slope) {
     const uint32_t mat = own & kMatMask;
-    // one reciprocal per spacing instead of a division per difference: each
-    // quotient moves by at most an ulp against the reference's c/dx
-    const double ix = 1. / dx, iy = 1. / dy, iz = 1. / dz;
     Stencil r;
     double bw[3], fw[3], ab, af;
     // x faces
@@ -181,19 +180,6 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
     }
     for (int a = 0; a < 3; a++) r.ex[a] = r.ex[a] + af * (fw[a] * iz) + ab * (-bw[a] * iz);
     return r;
-}
-
-template <bool kDmi, class I>
-__device__ __forceinline__ Stencil stencil(const P3 s3, const uint32_t* code, const DevMaterial* mats,
-                                           uint32_t own, int surf_shift, int sub, I i, I j, I k,
-                                           I nx, I ny, I nz, double dx, double dy, double dz,
-                                           double A, double A_self, double slope) {
-    const I id = (i * ny + j) * nz + k;
-    const double c0 = ldd(s3.p[0], id), c1 = ldd(s3.p[1], id), c2 = ldd(s3.p[2], id);
-    double v[6][3];
-    uint32_t cd[6];
-    gather6<I>(s3, code, i, j, k, nx, ny, nz, v, cd);
-    return stencil_core<kDmi>(c0, c1, c2, v, cd, mats, own, surf_shift, sub, dx, dy, dz, A, A_self, slope);
 }
 
 // Magnetoelastic field of a crystal-frame strain, in the global frame:
