@@ -415,13 +415,20 @@ struct Shapes {
 
 // Pencils per workgroup.  z and y passes write their output transposed,
 // so their pencil count sets the length of the store runs (16 B each);
-// the x pass reads and writes whole rows, so it keeps one pencil per
-// component and more workgroups per CU (at 256x256x128 one pencil beat two
-// by 7% and eight y pencils matched four).  GOFERRO_FFT_PENCILS="z,y,x"
-// overrides the defaults (powers of two) for tuning sweeps.
+// the x pass reads and writes whole rows (x_pencils).  Eight y pencils make
+// whole 128 B lines of the y passes; sixteen only halved the number of workgroups (64x64x16, 20
+// steps: 2.40 ms with 16, 2.18 with 8, 2.30 with 4; 128x128x32 adjoint 74.8 and
+// 74.0 ms).  Lines of 256 and more keep to 1024 elements a workgroup while the
+// spectra stay in the caches (128x256x32, 40 steps: 18.3 ms with 8 pencils, 17.7
+// with 4), but not beyond (256x256x128: 108 ms with 8, 113 with 4: half lines).
+// GOFERRO_FFT_PENCILS="z,y,x" overrides the defaults (powers of two) for
+// tuning sweeps.
 Shapes shapes(const gf_ctx* c) {
     Shapes s;
-    int64_t bz = 2048, by = 2048, bx = 512, cz = 16, cy = 16, cx = 1;
+    const int64_t spectra = 3 * c->nx * c->ny * (c->nz / 2 + 1) * static_cast<int64_t>(sizeof(double2));
+    int64_t bz = 2048, by = spectra <= (int64_t{64} << 20) ? 1024 : 2048, bx = 1024, cy = 8;
+    int64_t cz = z_pencils(c->nx, c->ny);
+    int64_t cx = x_pencils(c->nx, c->ny);
     if (const char* env = std::getenv("GOFERRO_FFT_PENCILS")) {
         int z = 0, y = 0, x = 0;
         if (std::sscanf(env, "%d,%d,%d", &z, &y, &x) == 3 && z > 0 && y > 0 && x > 0) {

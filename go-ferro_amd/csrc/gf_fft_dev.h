@@ -29,6 +29,24 @@ template <> struct FftComplex<float2> {
     static __device__ __forceinline__ float2 make(float re, float im) { return make_float2(re, im); }
 };
 
+// y rows (pencils of each component) of an x pass's workgroup of 256 threads:
+// from rows of 128 points on, as many as give each thread a point of the
+// tensor product (two of 128: the pass 20.9 -> 18.9 us at 128x128x32, with three
+// elements a thread where one row leaves half of the threads a second one);
+// one row of 64 or fewer, since those leave threads idle either way and more
+// workgroups are the better split (64x64x16, 20 steps: 2.18 ms; two rows 2.26,
+// four 2.21).
+inline int x_pencils(int64_t nx, int64_t ny) {
+    int r = 1;
+    while (nx >= 128 && 2 * r * nx <= 256 && 2 * r <= ny) r *= 2;
+    return r;
+}
+
+// At most this many columns a workgroup of a z pass (three components): 32
+// where that leaves four workgroups per CU (128x128x32 adjoint: 71.9 -> 70.9 ms,
+// FP32 48.4 -> 47.2), else 16 (64x64x16: 24.4 ms, 25.3 with 32).
+inline int64_t z_pencils(int64_t nx, int64_t ny) { return 3 * nx * (ny / 32) >= 1024 ? 32 : 16; }
+
 __device__ __forceinline__ double2 fft_cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }

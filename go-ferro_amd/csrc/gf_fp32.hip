@@ -322,26 +322,30 @@ struct X32Args {
     int64_t nh;
     float den;                     // -dx*dy*dz
     int nx, ny, lognx;
+    int rows, logr;                // y rows per workgroup
     int adjoint;                   // conjugate transpose of the tensor
 };
 
 // x forward transform, tensor product (magnetostatic_solver.cpp:163-177,
-// spectra xx, yy, zz, xy, yz, zx, yx, zy, xz), x inverse, one y row of the
+// spectra xx, yy, zz, xy, yz, zx, yx, zy, xz), x inverse, `rows` y rows of the
 // three components per workgroup.
 __global__ void __launch_bounds__(kT) xconv32_kernel(X32Args a) {
     extern __shared__ float2 sm32[];
-    const int kz = blockIdx.y, y = blockIdx.x;
+    const int kz = blockIdx.y, pts = a.rows * a.nx;
     float2* tw = sm32;
     float2* buf = sm32 + (a.nx >> 1);
     const float2 tw0 = fft_twiddle_prefetch(a.tw, a.nx);
-    const int64_t row = (static_cast<int64_t>(kz) * a.ny + y) * a.nx;
+    // rows is a power of two dividing ny, and they are consecutive in memory:
+    // element i of component c, in memory and (bit-reversed in x) in LDS
+    const int64_t row = (static_cast<int64_t>(kz) * a.ny + static_cast<int64_t>(blockIdx.x) * a.rows) * a.nx;
+    const int logp = a.lognx + a.logr;
     fft_staged_load<kBatch32, float2>(
-        3 * a.nx, [&](int idx) { return a.data[(idx >> a.lognx) * a.nh + row + (idx & (a.nx - 1))]; },
-        [&](int idx, float2 v) { buf[fpad((idx >> a.lognx) * a.nx + fft_bitrev(idx & (a.nx - 1), a.lognx))] = v; });
+        3 * pts, [&](int idx) { return a.data[(idx >> logp) * a.nh + row + (idx & (pts - 1))]; },
+        [&](int idx, float2 v) { buf[fpad((idx & ~(a.nx - 1)) + fft_bitrev(idx & (a.nx - 1), a.lognx))] = v; });
     fft_twiddle_store(tw, a.tw, a.nx, tw0);
     __syncthreads();
-    fft_dit<4>(buf, 3, a.lognx, tw);
-    for (int x = threadIdx.x; x < a.nx; x += blockDim.x) {
+    fft_dit<4>(buf, 3 * a.rows, a.lognx, tw);
+    for (int x = threadIdx.x; x < pts; x += blockDim.x) {
         const int64_t g = row + x;
         float2 K[9];
         for (int q = 0; q < 9; q++) {
@@ -349,7 +353,7 @@ __global__ void __launch_bounds__(kT) xconv32_kernel(X32Args a) {
             const float2 v = a.kt[t * a.nh + g];
             K[q] = make_float2(v.x, a.adjoint ? -v.y : v.y);
         }
-        const float2 mx = buf[fpad(x)], my = buf[fpad(a.nx + x)], mz = buf[fpad(2 * a.nx + x)];
+        const float2 mx = buf[fpad(x)], my = buf[fpad(pts + x)], mz = buf[fpad(2 * pts + x)];
         auto cm = [](float2 p, float2 q) { return make_float2(p.x * q.x - p.y * q.y, p.x * q.y + p.y * q.x); };
         float2 t0 = cm(mx, K[0]), t1 = cm(my, K[3]), t2 = cm(mz, K[8]);
         const float2 hx = make_float2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
@@ -357,14 +361,13 @@ __global__ void __launch_bounds__(kT) xconv32_kernel(X32Args a) {
         const float2 hy = make_float2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
         t0 = cm(mz, K[2]); t1 = cm(mx, K[5]); t2 = cm(my, K[7]);
         const float2 hz = make_float2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
-        buf[fpad(x)] = hx; buf[fpad(a.nx + x)] = hy; buf[fpad(2 * a.nx + x)] = hz;
+        buf[fpad(x)] = hx; buf[fpad(pts + x)] = hy; buf[fpad(2 * pts + x)] = hz;
     }
     __syncthreads();
-    ifft_dif<4>(buf, 3, a.lognx, tw);
-    for (int idx = threadIdx.x; idx < 3 * a.nx; idx += blockDim.x) {
-        const int c = idx >> a.lognx, x = idx & (a.nx - 1);
-        a.data[c * a.nh + row + x] = buf[fpad(c * a.nx + fft_bitrev(x, a.lognx))];
-    }
+    ifft_dif<4>(buf, 3 * a.rows, a.lognx, tw);
+    for (int idx = threadIdx.x; idx < 3 * pts; idx += blockDim.x)
+        a.data[(idx >> logp) * a.nh + row + (idx & (pts - 1))] =
+            buf[fpad((idx & ~(a.nx - 1)) + fft_bitrev(idx & (a.nx - 1), a.lognx))];
 }
 
 struct ZI32Args {
@@ -681,8 +684,10 @@ gf_status conv32(gf_ctx* c, Adj32* s, const float* const* in, float* const* out,
     x.data = s->spb; x.kt = s->kt; x.tw = s->twx; x.nh = s->nh;
     x.den = static_cast<float>(-c->dx * c->dy * c->dz);
     x.nx = nx; x.ny = ny; x.lognx = ilog2i(nx); x.adjoint = adjoint ? 1 : 0;
-    const size_t lx = sizeof(float2) * static_cast<size_t>(nx / 2 + fft_lds_elems(3 * static_cast<int64_t>(nx)));
-    hipLaunchKernelGGL(xconv32_kernel, dim3(ny, nzh), dim3(kT), lx, c->stream, x);
+    x.rows = x_pencils(nx, ny);
+    x.logr = ilog2i(x.rows);
+    const size_t lx = sizeof(float2) * static_cast<size_t>(nx / 2 + fft_lds_elems(3 * static_cast<int64_t>(x.rows) * nx));
+    hipLaunchKernelGGL(xconv32_kernel, dim3(ny / x.rows, nzh), dim3(kT), lx, c->stream, x);
     y.in = s->spb; y.out = s->spa;
     hipLaunchKernelGGL(yinv32_kernel, gy, dim3(kT), ly, c->stream, y);
     ZI32Args zi{};
@@ -840,8 +845,8 @@ gf_status adjoint32_forward(gf_ctx* c, const gf_adjoint_desc* d, double* loss) {
     if (!st && s->ms) {
         s->nzh = c->nz / 2 + 1;
         s->nh = c->nx * c->ny * s->nzh;
-        s->pz = pencils_for(c->nz, 2048, 16, c->ny);
-        s->py = pencils_for(c->ny, 2048, 16, c->nx);
+        s->pz = pencils_for(c->nz, 2048, z_pencils(c->nx, c->ny), c->ny);
+        s->py = pencils_for(c->ny, 2048, 8, c->nx);
         st = twiddles32(c, &s->twx, c->nx);
         if (!st) st = twiddles32(c, &s->twy, c->ny);
         if (!st) st = twiddles32(c, &s->twz, c->nz);
