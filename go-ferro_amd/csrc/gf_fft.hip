@@ -186,7 +186,9 @@ struct XArgs {
     const double2* tw;
     int64_t nh, nhb;
     int kz0, kzb0;
-    double den;                 // -dx*dy*dz
+    double rden;                // 1 / (-dx*dy*dz): a product is within an ulp of the quotient, and six
+                                // divisions a point were 8% of the pass's instructions (256x256x128:
+                                // 159 -> 152 us)
     int nx, ny, nzh;
     int lognx, pencils, logp;
     int adjoint;                // 1: conjugate transpose of the tensor (adjoint convolution)
@@ -252,11 +254,11 @@ __global__ void __launch_bounds__(kThreads) xconv_kernel(XArgs a) {
             const double2 mx = buf[fpad(ix)], my = buf[fpad(iy)], mz = buf[fpad(iz)];
             auto K = [&](int q) { return make_double2(kr[q], ki[q]); };
             double2 t0 = cmul(mx, K(0)), t1 = cmul(my, K(3)), t2 = cmul(mz, K(8));
-            const double2 hx = make_double2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
+            const double2 hx = make_double2((t0.x + t1.x + t2.x) * a.rden, (t0.y + t1.y + t2.y) * a.rden);
             t0 = cmul(my, K(1)); t1 = cmul(mz, K(4)); t2 = cmul(mx, K(6));
-            const double2 hy = make_double2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
+            const double2 hy = make_double2((t0.x + t1.x + t2.x) * a.rden, (t0.y + t1.y + t2.y) * a.rden);
             t0 = cmul(mz, K(2)); t1 = cmul(mx, K(5)); t2 = cmul(my, K(7));
-            const double2 hz = make_double2((t0.x + t1.x + t2.x) / a.den, (t0.y + t1.y + t2.y) / a.den);
+            const double2 hz = make_double2((t0.x + t1.x + t2.x) * a.rden, (t0.y + t1.y + t2.y) * a.rden);
             buf[fpad(ix)] = hx; buf[fpad(iy)] = hy; buf[fpad(iz)] = hz;
         };
         if (first_ok) product(first, kr0, ki0);
@@ -626,7 +628,7 @@ static hipError_t run_x(gf_ctx* c, DemagPlan& d, bool conv, KzRange kr, bool adj
     a.data = d.spec_b; a.kre = d.kre; a.kim = d.kim; a.tw = d.twx.dev;
     a.nh = c->nx * c->ny * d.nzh;
     a.nhb = kr.nhb; a.kz0 = kr.k0; a.kzb0 = kr.kb0;
-    a.den = -c->dx * c->dy * c->dz;
+    a.rden = 1. / (-c->dx * c->dy * c->dz);
     a.nx = static_cast<int>(c->nx); a.ny = static_cast<int>(c->ny); a.nzh = static_cast<int>(d.nzh);
     a.lognx = ilog2(c->nx); a.pencils = sh.px; a.logp = ilog2(sh.px);
     dim3 grid(blocks_for(c->ny, sh.px), static_cast<unsigned>(kr.cnt));

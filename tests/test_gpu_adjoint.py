@@ -568,6 +568,21 @@ def test_fp32_sweep_tracks_fp64(demag, anis):
     g32.close()
 
 
+@pytest.mark.parametrize("shape", [(128, 8, 8), (128, 16, 4), (256, 8, 4), (16, 32, 8)])
+def test_fp32_passes_at_workgroup_edges(shape):
+    """x rows of 128 points two to a workgroup (and of 256, one), eight y lines
+    and 32 z columns: the loss and the drive gradient track the FP64 sweep's."""
+    say("case FP32 passes", shape)
+    prob = problem(shape=shape, rotate=False)
+    f = inputs(shape)
+    g64, L64, _, ghd64 = run_adjoint(prob, f, 6)
+    g32, L32, _, ghd32 = run_adjoint32(prob, f, 6)
+    assert abs(L32 - L64) <= 1e-5 * L64
+    assert np.linalg.norm(ghd32 - ghd64) <= 1e-5 * np.linalg.norm(ghd64)
+    g64.close()
+    g32.close()
+
+
 def test_fp32_checkpoints_and_state():
     """The FP32 gradients do not depend on the checkpoint spacing (the
     recomputed FP32 trajectory is bit-identical), and the sweep leaves the

@@ -31,6 +31,27 @@ def test_fm_mixed_materials_general_grid(shape, rotate):
     say("  worst stage store difference", worst)
 
 
+@pytest.mark.parametrize("shape", [(128, 1, 4), (128, 2, 8), (64, 4, 2), (4, 256, 4), (2, 512, 2), (16, 32, 8),
+                                   (256, 4, 4)])
+def test_power_of_two_passes_at_workgroup_edges(shape):
+    """The field of the power-of-two passes where their split changes: x rows
+    of 128 points two to a workgroup (and one, where there is only one), y
+    lines of 256 and 512 with four and two to a workgroup, z columns 32 and 16
+    to a workgroup."""
+    from oracle.oracle import Oracle
+    say("case power-of-two demag", shape)
+    prob, m = workloads.fm_film(shape)
+    g, o = Context(prob), Oracle(prob)
+    g.upload(FIELD_M, m)
+    o.set(FIELD_M, m)
+    g.demag()
+    o.demag()
+    hg, ho = g.download(FIELD_HSTAT), o.get(FIELD_HSTAT)
+    assert np.abs(hg - ho).max() <= 1e-12 * np.abs(ho).max()
+    g.close()
+    o.close()
+
+
 def test_fm_film_general_grid_fused_and_periodic():
     """The config-1 film physics on 20x12x16: periodic in x and y, the fused
     stage (nz = 16) with P = 4 columns dividing ny = 12."""
