@@ -141,13 +141,13 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const double yc[3] = {ldd(a.y[0], id), ldd(a.y[1], id), ldd(a.y[2], id)};
     const P3 sp = {{a.y[0], a.y[1], a.y[2]}};
     double nv[6][3];
-    uint32_t ncd[6];
-    gather6_lanes_load<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
+    const I nx = static_cast<I>(a.nx);
+    gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, nv);
     const double kb0 = ldd(a.kbar[0], id), kb1 = ldd(a.kbar[1], id), kb2 = ldd(a.kbar[2], id);
     const bool dem = a.hd[0] != nullptr;
     const double hd0 = dem ? ldd(a.hd[0], id) : 0., hd1 = dem ? ldd(a.hd[1], id) : 0.;
     const double hd2 = dem ? ldd(a.hd[2], id) : 0.;
-    gather6_lanes_shift<I>(z, nz, yc, own, nv, ncd);
+    gather6_lanes_shift<I>(z, nz, yc, nv);
     if (!(own & kIsFM)) {
         for (int c = 0; c < 3; c++) { std_(a.mbar[c], id, 0.); std_(a.hbar[c], id, 0.); }
         return;
@@ -156,8 +156,8 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const double mgx = yc[0], mgy = yc[1], mgz = yc[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil st = stencil_core<true>(mgx, mgy, mgz, nv, ncd, a.mats, own, kFmSurfShift, -1, a.idx, a.idy, a.idz,
-                                          M.Aex, M.Aex_self, M.dmi_slope);
+    const Stencil st = magnet_stencil<true, I>(yc, nv, a.code, (GMat*)a.mats, own, kFmSurfShift, -1, x, y, z, nx, ny, nz,
+                                               a.idx, a.idy, a.idz, M.Aex, M.Aex_self, M.dmi_slope);
     // exchange and interfacial DMI (zero without it) of the forward stage
     const double hex0 = M.exch * st.ex[0] + M.dmi_pos * st.d[2], hex1 = M.exch * st.ex[1] + M.dmi_pos * st.d[3];
     const double hex2 = M.exch * st.ex[2] + M.dmi_neg * (st.d[0] + st.d[1]);
@@ -168,7 +168,8 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
         const uint32_t mi = own & kMatMask;
         for (int f = 0; f < 6; f++) {
             if ((own >> (kFmSurfShift + f)) & 1u) continue;
-            const double w = dcoef_dA(a.mats, mi, ncd[f] & kMatMask, static_cast<uint32_t>(a.mat)) * a.ih2[f >> 1];
+            const uint32_t mj = own & kMixed ? ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz)) & kMatMask : mi;
+            const double w = dcoef_dA(a.mats, mi, mj, static_cast<uint32_t>(a.mat)) * a.ih2[f >> 1];
             exd0 += w * (nv[f][0] - mgx);
             exd1 += w * (nv[f][1] - mgy);
             exd2 += w * (nv[f][2] - mgz);
@@ -353,8 +354,8 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     const P3 sp = {{a.hbar[0], a.hbar[1], a.hbar[2]}};
     const double hb[3] = {ldd(a.hbar[0], id), ldd(a.hbar[1], id), ldd(a.hbar[2], id)};
     double nv[6][3];
-    uint32_t ncd[6];
-    gather6_lanes_load<I>(sp, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, nv, ncd);
+    const I nx = static_cast<I>(a.nx);
+    gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, nv);
     double mb[3], da[3], lam[3], acc[3];
     const bool dem = a.dadj[0] != nullptr, step = a.mode != 0, later = step && a.mode != 4;
     for (int c = 0; c < 3; c++) {
@@ -363,7 +364,7 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
         lam[c] = step ? ldd(a.lam[c], id) : 0.;
         acc[c] = later ? ldd(a.acc[c], id) : 0.;
     }
-    gather6_lanes_shift<I>(z, nz, hb, own, nv, ncd);
+    gather6_lanes_shift<I>(z, nz, hb, nv);
     if (!(own & kIsFM)) {
         if (a.mode == 0) for (int c = 0; c < 3; c++) std_(a.ybar[c], id, 0.);
         return;
@@ -376,11 +377,11 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     {
         const double ih[2] = {a.idx, a.idy};
         for (int f = 0; f < 4; f++) {
-            if (((own >> (kFmSurfShift + f)) & 1u) || !(ncd[f] & kIsFM)) continue;
-            // the neighbour's own constants; its record is read only when it is another
+            if ((own >> (kFmSurfShift + f)) & 1u) continue;   // else the neighbour is FM
+            // the neighbour's own constants; its record is read only when it can be another
             double dn = M.dmi_neg, dp = M.dmi_pos;
-            if ((ncd[f] ^ own) & kMatMask) {
-                GMat& Mn = mat_of(a.mats, ncd[f]);
+            if (own & kMixed) {
+                GMat& Mn = mat_of(a.mats, ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz)));
                 dn = Mn.dmi_neg; dp = Mn.dmi_pos;
             }
             const double w = ((f & 1) ? -1. : 1.) * ih[f >> 1];
@@ -390,12 +391,14 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
         }
     }
     for (int f = 0; f < 6; f++) {
-        double e = M.exch;
-        if ((ncd[f] ^ own) & kMatMask) e = (ncd[f] & kIsFM) ? mat_of(a.mats, ncd[f]).exch : 0.;
+        double e = M.exch;   // across a surface too: the value is not used there
+        if ((own & kMixed) && !((own >> (kFmSurfShift + f)) & 1u))
+            e = mat_of(a.mats, ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz))).exch;
         for (int c = 0; c < 3; c++) nv[f][c] = e * nv[f][c];
     }
-    const Stencil st = stencil_core<false>(M.exch * hb[0], M.exch * hb[1], M.exch * hb[2], nv, ncd, a.mats, own,
-                                           kFmSurfShift, -1, a.idx, a.idy, a.idz, M.Aex, M.Aex_self, 0.);
+    const double eh[3] = {M.exch * hb[0], M.exch * hb[1], M.exch * hb[2]};
+    const Stencil st = magnet_stencil<false, I>(eh, nv, a.code, (GMat*)a.mats, own, kFmSurfShift, -1, x, y, z, nx, ny, nz,
+                                                a.idx, a.idy, a.idz, M.Aex, M.Aex_self, 0.);
     const bool probe = x >= static_cast<I>(a.lo[0]) && x <= static_cast<I>(a.hi[0]) && y >= static_cast<I>(a.lo[1]) &&
                        y <= static_cast<I>(a.hi[1]) && z >= static_cast<I>(a.lo[2]) && z <= static_cast<I>(a.hi[2]);
     for (int c = 0; c < 3; c++) {

@@ -126,6 +126,40 @@ void build_surface_bits(gf_ctx* c, bool (*kind)(const gf_ctx*, int64_t), int shi
             }
 }
 
+// The codes as the device holds them: with kMixed set (one magnetic material
+// has no such cell).
+std::vector<uint32_t> device_codes(const gf_ctx* c) {
+    std::vector<uint32_t> out = c->host_code;
+    uint32_t seen = 0;
+    bool several = false;
+    for (size_t i = 0; i < out.size() && !several; i++) {
+        if (!(out[i] & (kIsFM | kIsAFM))) continue;
+        const uint32_t t = out[i] & kMatMask;
+        several = seen && t != seen;
+        seen = t;
+    }
+    if (!several) return out;
+    const int64_t n3[3] = {c->nx, c->ny, c->nz}, step[3] = {c->ny * c->nz, c->nz, 1};
+    int64_t q[3];
+    for (q[0] = 0; q[0] < n3[0]; q[0]++)
+        for (q[1] = 0; q[1] < n3[1]; q[1]++)
+            for (q[2] = 0; q[2] < n3[2]; q[2]++) {
+                const int64_t id = q[0] * step[0] + q[1] * step[1] + q[2];
+                const uint32_t own = c->host_code[static_cast<size_t>(id)];
+                if (!(own & (kIsFM | kIsAFM))) continue;
+                for (int f = 0; f < 6; f++) {
+                    const bool fm = (own & kIsFM) && !((own >> (kFmSurfShift + f)) & 1u);
+                    const bool afm = (own & kIsAFM) && !((own >> (kAfmSurfShift + f)) & 1u);
+                    if (!fm && !afm) continue;
+                    const int ax = f >> 1;
+                    const int64_t to = f & 1 ? (q[ax] == n3[ax] - 1 ? 0 : q[ax] + 1) : (q[ax] == 0 ? n3[ax] - 1 : q[ax] - 1);
+                    const uint32_t nb = c->host_code[static_cast<size_t>(id + (to - q[ax]) * step[ax])];
+                    if ((nb ^ own) & kMatMask) out[static_cast<size_t>(id)] |= kMixed;
+                }
+            }
+    return out;
+}
+
 DevMaterial make_dev_material(const gf_material& m, double dt) {
     DevMaterial d{};
     d.is_fm = m.if_FM ? 1 : 0;
@@ -909,7 +943,7 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
     if (!st) st = hip_check(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
     if (!st) st = hip_check(c, hipMalloc(&c->d_code, sizeof(uint32_t) * c->n), "hipMalloc code");
     if (!st)
-        st = hip_check(c, hipMemcpy(c->d_code, c->host_code.data(), sizeof(uint32_t) * c->n, hipMemcpyHostToDevice),
+        st = hip_check(c, hipMemcpy(c->d_code, device_codes(c).data(), sizeof(uint32_t) * c->n, hipMemcpyHostToDevice),
                        "copy code");
     if (!st && c->any_fm && c->nfm < c->n && c->n <= INT64_C(0xffffffff)) {
         // the FM cells in index order: the unfused FM stage runs over them

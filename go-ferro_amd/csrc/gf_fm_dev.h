@@ -13,39 +13,27 @@ namespace {
 // gather6 for launches whose active lanes hold consecutive cells along z
 // (lane i of a wave at cell id0 + i, and a lane without a cell only past
 // the grid's last cell): a cell's z neighbours are then the store values
-// and codes of the lanes next to it, moved with DPP wave shifts, except at
-// a column end (k = 0 or nz - 1, where the neighbour wraps or the face is a
-// surface) or a wave edge, where they are loaded.  A lane next to one
-// without a cell is at a column end.  Two parts: the loads, and after the
-// cell's other loads have been issued, the lane shifts of its own store c
-// and code own.
+// of the lanes next to it, moved with DPP wave shifts, except at a column
+// end (k = 0 or nz - 1, where the neighbour wraps or the face is a surface)
+// or a wave edge, where they are loaded.  A lane next to one without a cell
+// is at a column end.  Two parts: the loads, and after the cell's other
+// loads have been issued, the lane shifts of its own store c.
 template <class I>
-__device__ __forceinline__ void gather6_lanes_load(const P3 s3, const uint32_t* code, I x, I y, I z, I nx, I ny,
-                                                   I nz, double (&v)[6][3], uint32_t (&cd)[6]) {
-    const I nb[4] = {((x == 0 ? nx - 1 : x - 1) * ny + y) * nz + z, ((x == nx - 1 ? 0 : x + 1) * ny + y) * nz + z,
-                     (x * ny + (y == 0 ? ny - 1 : y - 1)) * nz + z, (x * ny + (y == ny - 1 ? 0 : y + 1)) * nz + z};
+__device__ __forceinline__ void gather6_lanes_load(const P3 s3, I x, I y, I z, I nx, I ny, I nz, double (&v)[6][3]) {
 #pragma unroll
     for (int f = 0; f < 4; f++) {
-        for (int q = 0; q < 3; q++) v[f][q] = ldd(s3.p[q], nb[f]);
-        cd[f] = ldu(code, nb[f]);
+        const I nb = face_nb<I>(f, x, y, z, nx, ny, nz);
+        for (int q = 0; q < 3; q++) v[f][q] = ldd(s3.p[q], nb);
     }
     const int lane = static_cast<int>(threadIdx.x & 63u);
-    const bool gm = lane == 0 || z == 0, gp = lane == 63 || z == nz - 1;
-    if (gm) {
-        const I zm = (x * ny + y) * nz + (z == 0 ? nz - 1 : z - 1);
-        for (int q = 0; q < 3; q++) v[4][q] = ldd(s3.p[q], zm);
-        cd[4] = ldu(code, zm);
-    }
-    if (gp) {
-        const I zp = (x * ny + y) * nz + (z == nz - 1 ? 0 : z + 1);
-        for (int q = 0; q < 3; q++) v[5][q] = ldd(s3.p[q], zp);
-        cd[5] = ldu(code, zp);
-    }
+    if (lane == 0 || z == 0)
+        for (int q = 0; q < 3; q++) v[4][q] = ldd(s3.p[q], face_nb<I>(4, x, y, z, nx, ny, nz));
+    if (lane == 63 || z == nz - 1)
+        for (int q = 0; q < 3; q++) v[5][q] = ldd(s3.p[q], face_nb<I>(5, x, y, z, nx, ny, nz));
 }
 
 template <class I>
-__device__ __forceinline__ void gather6_lanes_shift(I z, I nz, const double (&c)[3], uint32_t own, double (&v)[6][3],
-                                                    uint32_t (&cd)[6]) {
+__device__ __forceinline__ void gather6_lanes_shift(I z, I nz, const double (&c)[3], double (&v)[6][3]) {
     const int lane = static_cast<int>(threadIdx.x & 63u);
     const bool gm = lane == 0 || z == 0, gp = lane == 63 || z == nz - 1;
     for (int q = 0; q < 3; q++) {
@@ -53,9 +41,6 @@ __device__ __forceinline__ void gather6_lanes_shift(I z, I nz, const double (&c)
         if (!gm) v[4][q] = dn;
         if (!gp) v[5][q] = up;
     }
-    const uint32_t cdn = lane_up(own), cup = lane_down(own);
-    if (!gm) cd[4] = cdn;
-    if (!gp) cd[5] = cup;
 }
 
 // Every global input of one FM cell of a stage except the static field:
@@ -66,7 +51,6 @@ struct FmIn {
     uint32_t own;
     double c[3];        // stage store at the cell
     double v[6][3];     // stage store at the six face neighbours (gather6)
-    uint32_t cd[6];     // their codes
     double m[3];        // m at the start of the step
     double acc[3];      // RK accumulator (read at stages 2-4)
 };
@@ -78,13 +62,13 @@ __device__ __forceinline__ void fm_load(const StageArgs& a, I id, I x, I y, I z,
     const P3 sp = {{a.store[0], a.store[1], a.store[2]}};
     for (int c = 0; c < 3; c++) in.c[c] = ldd(a.store[c], id);
     const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    if (kLanes) gather6_lanes_load<I>(sp, a.code, x, y, z, nx, ny, nz, in.v, in.cd);
-    else gather6<I>(sp, a.code, x, y, z, nx, ny, nz, in.v, in.cd);
+    if (kLanes) gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, in.v);
+    else gather6<I>(sp, x, y, z, nx, ny, nz, in.v);
     // at stage 1 the stage store is m itself: read it once
     const bool same = a.base[0] == a.store[0] && a.base[1] == a.store[1] && a.base[2] == a.store[2];
     for (int c = 0; c < 3; c++) in.m[c] = same ? in.c[c] : ldd_nt(a.base[c], id);
     for (int c = 0; c < 3; c++) in.acc[c] = a.stage > 1 ? ldd_nt(a.acc[c], id) : 0.;
-    if (kLanes) gather6_lanes_shift<I>(z, nz, in.c, in.own, in.v, in.cd);
+    if (kLanes) gather6_lanes_shift<I>(z, nz, in.c, in.v);
 }
 
 // RK update of one component (see the file comment) from its preloaded m
@@ -119,18 +103,19 @@ __device__ __forceinline__ double rk_store(int stage, I id, int c, double k, dou
 // prescribed bottom layer) for contexts that have none of them: their
 // pointers and the rotation matrices then occupy no scalar registers
 // across the cell loop.  mats is the material table, in global memory
-// (GMat) or a workgroup's LDS copy (LMat).  bottom: the cell is at k = 0.
+// (GMat) or a workgroup's LDS copy (LMat).  (x, y, z) are the cell's.
 template <bool kLean, class I, class MT>
-__device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn& in, I id, double hs0, double hs1,
-                                        double hs2, double& n0, double& n1, double& n2, bool bottom) {
+__device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn& in, I id, I x, I y, I z, double hs0,
+                                        double hs1, double hs2, double& n0, double& n1, double& n2) {
     MT& M = mats[(in.own & kMatMask) - 1];
 
     const double mgx = in.c[0], mgy = in.c[1], mgz = in.c[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (!kLean && a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
 
-    const Stencil st = stencil_core<true>(mgx, mgy, mgz, in.v, in.cd, mats, in.own, kFmSurfShift, -1, a.idx, a.idy,
-                                          a.idz, M.Aex, M.Aex_self, M.dmi_slope);
+    const Stencil st = magnet_stencil<true, I>(in.c, in.v, a.code, mats, in.own, kFmSurfShift, -1, x, y, z,
+                                               static_cast<I>(a.nx), static_cast<I>(a.ny), static_cast<I>(a.nz), a.idx,
+                                               a.idy, a.idz, M.Aex, M.Aex_self, M.dmi_slope);
 
     // magnetocrystalline anisotropy (magnetic_solver.cpp:124-141)
     double hac0 = 0., hac1 = 0., hac2 = 0.;
@@ -188,7 +173,7 @@ __device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn
     }
     // update_prescribed_m{_half,_full,} over the update (magnetic_solver.cpp:
     // 1526-1609, 1891-1957); the accumulator keeps the LLG increment
-    const bool pres = !kLean && a.prescribe && bottom;
+    const bool pres = !kLean && a.prescribe && z == 0;
     n0 = rk_store(a.stage, id, 0, k0, in.m[0], in.acc[0], a.acc, a.out, pres, a.presc_m[0]);
     n1 = rk_store(a.stage, id, 1, k1, in.m[1], in.acc[1], a.acc, a.out, pres, a.presc_m[1]);
     n2 = rk_store(a.stage, id, 2, k2, in.m[2], in.acc[2], a.acc, a.out, pres, a.presc_m[2]);
@@ -209,7 +194,7 @@ __device__ __forceinline__ void fm_point(const StageArgs& a, I id) {
     const double hs2 = hs ? ldd(a.hstat[2], id) : 0.;
     if (!(in.own & kIsFM)) return;
     double n0, n1, n2;
-    fm_cell<false, I>(a, (GMat*)a.mats, in, id, hs0, hs1, hs2, n0, n1, n2, z == 0);
+    fm_cell<false, I>(a, (GMat*)a.mats, in, id, x, y, z, hs0, hs1, hs2, n0, n1, n2);
 }
 
 }  // namespace

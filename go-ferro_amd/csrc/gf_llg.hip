@@ -165,10 +165,12 @@ __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, Fused
             double Ms;
             if (kLean) {
                 LMat* tab = (LMat*)ltab;
-                fm_cell<kLean, I>(a, tab, in, id, *h0, *h1, *h2, n0, n1, n2, k == 0);
+                fm_cell<kLean, I>(a, tab, in, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), *h0, *h1, *h2, n0,
+                                  n1, n2);
                 Ms = tab[(in.own & kMatMask) - 1].Ms;
             } else {
-                fm_cell<kLean, I>(a, (GMat*)a.mats, in, id, *h0, *h1, *h2, n0, n1, n2, k == 0);
+                fm_cell<kLean, I>(a, (GMat*)a.mats, in, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), *h0, *h1,
+                                  *h2, n0, n1, n2);
                 Ms = mat_of(a.mats, in.own).Ms;
             }
             mx = Ms * n0; my = Ms * n1; mz = Ms * n2;
@@ -216,11 +218,12 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
     double* const* acc = sub == 0 ? a.acc1 : a.acc2;
     double* const* out = sub == 0 ? a.out1 : a.out2;
     const uint32_t own = ldu(a.code, id);
-    const double mgx = ldd(st.p[0], id), mgy = ldd(st.p[1], id), mgz = ldd(st.p[2], id);
+    const double c3[3] = {ldd(st.p[0], id), ldd(st.p[1], id), ldd(st.p[2], id)};
+    const double mgx = c3[0], mgy = c3[1], mgz = c3[2];
+    const I nx = static_cast<I>(a.nx);
     double v[6][3];
-    uint32_t cd[6];
-    if (kLanes) gather6_lanes_load<I>(st, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, v, cd);
-    else gather6<I>(st, a.code, x, y, z, static_cast<I>(a.nx), ny, nz, v, cd);
+    if (kLanes) gather6_lanes_load<I>(st, x, y, z, nx, ny, nz, v);
+    else gather6<I>(st, x, y, z, nx, ny, nz, v);
     const double o0 = ldd(other.p[0], id), o1 = ldd(other.p[1], id), o2 = ldd(other.p[2], id);
     // a null Hstat is zero (no statics, nothing uploaded)
     const bool hs = a.hstat[0] != nullptr;
@@ -233,16 +236,13 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
     mb[1] = same ? mgy : ldd_nt(base[1], id);
     mb[2] = same ? mgz : ldd_nt(base[2], id);
     for (int c = 0; c < 3; c++) ac[c] = a.stage > 1 ? ldd_nt(acc[c], id) : 0.;
-    if (kLanes) {
-        const double c3[3] = {mgx, mgy, mgz};
-        gather6_lanes_shift<I>(z, nz, c3, own, v, cd);
-    }
+    if (kLanes) gather6_lanes_shift<I>(z, nz, c3, v);
     if (!(own & kIsAFM)) return;
     GMat& M = mat_of(a.mats, own);
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil s = stencil_core<false>(mgx, mgy, mgz, v, cd, (GMat*)a.mats, own, kAfmSurfShift, sub, a.idx, a.idy,
-                                          a.idz, M.aAex[sub], M.aAex_self[sub], 0.);
+    const Stencil s = magnet_stencil<false, I>(c3, v, a.code, (GMat*)a.mats, own, kAfmSurfShift, sub, x, y, z, nx, ny,
+                                               nz, a.idx, a.idy, a.idz, M.aAex[sub], M.aAex_self[sub], 0.);
     // uniaxial anisotropy 2K1 (u.m) u (magnetic_AFM_solver.cpp:148-154)
     const double udotm = mx * M.u[0] + my * M.u[1] + mz * M.u[2];
     const double hac0 = 2. * M.aK1n[sub] * udotm * M.u[0];

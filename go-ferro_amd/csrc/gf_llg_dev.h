@@ -77,26 +77,28 @@ struct P3 {
     const double* p[3];
 };
 
-// The six face neighbours of cell (i, j, k) in the order x-, x+, y-, y+,
-// z-, z+, with the reference's wrap (used or not, every index is in
-// bounds), and their cell codes.  Loaded whether or not a face is a
+// Face neighbour f of cell (i, j, k) in the order x-, x+, y-, y+, z-, z+,
+// with the reference's wrap (used or not, the index is in bounds).
+template <class I>
+__device__ __forceinline__ I face_nb(int f, I i, I j, I k, I nx, I ny, I nz) {
+    switch (f) {
+    case 0: return ((i == 0 ? nx - 1 : i - 1) * ny + j) * nz + k;
+    case 1: return ((i == nx - 1 ? 0 : i + 1) * ny + j) * nz + k;
+    case 2: return (i * ny + (j == 0 ? ny - 1 : j - 1)) * nz + k;
+    case 3: return (i * ny + (j == ny - 1 ? 0 : j + 1)) * nz + k;
+    case 4: return (i * ny + j) * nz + (k == 0 ? nz - 1 : k - 1);
+    default: return (i * ny + j) * nz + (k == nz - 1 ? 0 : k + 1);
+    }
+}
+
+// The store at the six face neighbours.  Loaded whether or not a face is a
 // surface, so that the loads do not wait for the cell's own code.
 template <class I>
-__device__ __forceinline__ void gather6(const P3 s3, const uint32_t* code, I i, I j, I k, I nx, I ny, I nz,
-                                        double (&v)[6][3], uint32_t (&cd)[6]) {
-    I nb[6];
-    nb[0] = ((i == 0 ? nx - 1 : i - 1) * ny + j) * nz + k;
-    nb[1] = ((i == nx - 1 ? 0 : i + 1) * ny + j) * nz + k;
-    nb[2] = (i * ny + (j == 0 ? ny - 1 : j - 1)) * nz + k;
-    nb[3] = (i * ny + (j == ny - 1 ? 0 : j + 1)) * nz + k;
-    nb[4] = (i * ny + j) * nz + (k == 0 ? nz - 1 : k - 1);
-    nb[5] = (i * ny + j) * nz + (k == nz - 1 ? 0 : k + 1);
+__device__ __forceinline__ void gather6(const P3 s3, I i, I j, I k, I nx, I ny, I nz, double (&v)[6][3]) {
 #pragma unroll
     for (int f = 0; f < 6; f++) {
-        v[f][0] = ldd(s3.p[0], nb[f]);
-        v[f][1] = ldd(s3.p[1], nb[f]);
-        v[f][2] = ldd(s3.p[2], nb[f]);
-        cd[f] = ldu(code, nb[f]);
+        const I nb = face_nb<I>(f, i, j, k, nx, ny, nz);
+        for (int q = 0; q < 3; q++) v[f][q] = ldd(s3.p[q], nb);
     }
 }
 
@@ -114,13 +116,12 @@ __device__ __forceinline__ double face_coef(MP mats, uint32_t mat, uint32_t nc, 
 // The stencil of get_m_spatial_derivative_local from the cell's store
 // (c0, c1, c2) and its gathered neighbours; see gather6.  ix, iy and iz are
 // the reciprocal spacings: each quotient moves by at most an ulp against the
-// reference's c/dx.
-template <bool kDmi, class MP>
-__device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2, const double (&v)[6][3],
-                                                const uint32_t (&cd)[6], MP mats, uint32_t own,
-                                                int surf_shift, int sub, double ix, double iy, double iz, double A,
-                                                double A_self, double slope) {
-    const uint32_t mat = own & kMatMask;
+// reference's c/dx.  coef(f) is the coefficient of a face that is not a
+// surface, A that of one that is.
+template <bool kDmi, class Coef>
+__device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2, const double (&v)[6][3], uint32_t own,
+                                                int surf_shift, double ix, double iy, double iz, double A, double slope,
+                                                Coef coef) {
     Stencil r;
     double bw[3], fw[3], ab, af;
     // x faces
@@ -130,7 +131,7 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
         ab = A;
     } else {
         bw[0] = (c0 - v[0][0]) * ix; bw[1] = (c1 - v[0][1]) * ix; bw[2] = (c2 - v[0][2]) * ix;
-        ab = face_coef(mats, mat, cd[0], sub, A, A_self);
+        ab = coef(0);
     }
     if ((own >> (surf_shift + kXF)) & 1u) {
         if (kDmi) { fw[0] = -slope * c2; fw[1] = 0.; fw[2] = slope * c0; }
@@ -138,7 +139,7 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
         af = A;
     } else {
         fw[0] = (v[1][0] - c0) * ix; fw[1] = (v[1][1] - c1) * ix; fw[2] = (v[1][2] - c2) * ix;
-        af = face_coef(mats, mat, cd[1], sub, A, A_self);
+        af = coef(1);
     }
     r.d[0] = (bw[0] + fw[0]) * 0.5;
     r.d[2] = (bw[2] + fw[2]) * 0.5;
@@ -150,7 +151,7 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
         ab = A;
     } else {
         bw[0] = (c0 - v[2][0]) * iy; bw[1] = (c1 - v[2][1]) * iy; bw[2] = (c2 - v[2][2]) * iy;
-        ab = face_coef(mats, mat, cd[2], sub, A, A_self);
+        ab = coef(2);
     }
     if ((own >> (surf_shift + kYF)) & 1u) {
         if (kDmi) { fw[0] = 0.; fw[1] = -slope * c2; fw[2] = slope * c1; }
@@ -158,7 +159,7 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
         af = A;
     } else {
         fw[0] = (v[3][0] - c0) * iy; fw[1] = (v[3][1] - c1) * iy; fw[2] = (v[3][2] - c2) * iy;
-        af = face_coef(mats, mat, cd[3], sub, A, A_self);
+        af = coef(3);
     }
     r.d[1] = (bw[1] + fw[1]) * 0.5;
     r.d[3] = (bw[2] + fw[2]) * 0.5;
@@ -169,17 +170,30 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
         ab = A;
     } else {
         bw[0] = (c0 - v[4][0]) * iz; bw[1] = (c1 - v[4][1]) * iz; bw[2] = (c2 - v[4][2]) * iz;
-        ab = face_coef(mats, mat, cd[4], sub, A, A_self);
+        ab = coef(4);
     }
     if ((own >> (surf_shift + kZF)) & 1u) {
         fw[0] = 0.; fw[1] = 0.; fw[2] = 0.;
         af = A;
     } else {
         fw[0] = (v[5][0] - c0) * iz; fw[1] = (v[5][1] - c1) * iz; fw[2] = (v[5][2] - c2) * iz;
-        af = face_coef(mats, mat, cd[5], sub, A, A_self);
+        af = coef(5);
     }
     for (int a = 0; a < 3; a++) r.ex[a] = r.ex[a] + af * (fw[a] * iz) + ab * (-bw[a] * iz);
     return r;
+}
+
+// stencil_core with the coefficients of a cell at (x, y, z): the material's
+// own (A_self), and only where kMixed says so those of the neighbours' codes.
+template <bool kDmi, class I, class MP>
+__device__ __forceinline__ Stencil magnet_stencil(const double (&c)[3], const double (&v)[6][3], const uint32_t* code,
+                                                  MP mats, uint32_t own, int surf_shift, int sub, I x, I y, I z, I nx,
+                                                  I ny, I nz, double ix, double iy, double iz, double A, double A_self,
+                                                  double slope) {
+    return stencil_core<kDmi>(c[0], c[1], c[2], v, own, surf_shift, ix, iy, iz, A, slope, [&](int f) {
+        if (!(own & kMixed)) return A_self;
+        return face_coef(mats, own & kMatMask, ldu(code, face_nb<I>(f, x, y, z, nx, ny, nz)), sub, A, A_self);
+    });
 }
 
 // Magnetoelastic field of a crystal-frame strain, in the global frame:

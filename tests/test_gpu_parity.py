@@ -141,6 +141,22 @@ def test_afm_stages_with_demag():
     compare_stages(prob, {FIELD_M_AFM1: m1, FIELD_M_AFM2: m2}, nsteps=2, afm=True, fm=False)
 
 
+@pytest.mark.parametrize("shape,periodic", [((6, 7, 5), (True, False, True)), ((3, 4, 70), (False, True, False)),
+                                            ((1, 1, 9), (True, True, True))])
+def test_interfaces_of_magnets_of_both_kinds(shape, periodic):
+    """Two ferromagnets and two antiferromagnets side by side, with vacuum: only
+    cells at an interface read their neighbours' codes (harmonic-mean faces),
+    at walls, across periodic wraps and past a wave's length."""
+    prob, m1, m2 = workloads.afm_block(shape)
+    other = workloads.afm_block(shape, Aex=3e-12)[0].materials[0]
+    fm, m = mixed_fm_problem(shape=shape, flags=0, rotate=False)
+    prob.materials = [prob.materials[0], other] + list(fm.materials[:2])
+    prob.material_cell = np.random.default_rng(31).choice(np.arange(5, dtype=np.uint32), size=shape,
+                                                          p=[0.06, 0.3, 0.24, 0.22, 0.18])
+    prob.periodic = periodic
+    compare_stages(prob, {FIELD_M: m, FIELD_M_AFM1: m1, FIELD_M_AFM2: m2}, nsteps=2, afm=True)
+
+
 def test_fm_and_afm_together():
     shape = (8, 8, 8)
     prob_fm, m = workloads.fm_film(shape)
