@@ -430,7 +430,7 @@ Shapes shapes(const gf_ctx* c) {
     const int64_t spectra = 3 * c->nx * c->ny * (c->nz / 2 + 1) * static_cast<int64_t>(sizeof(double2));
     int64_t bz = 2048, by = spectra <= (int64_t{64} << 20) ? 1024 : 2048, bx = 1024, cy = 8;
     int64_t cz = z_pencils(c->nx, c->ny);
-    int64_t cx = x_pencils(c->nx, c->ny);
+    int64_t cx = x_pencils(c->nx, c->ny, c->nz / 2 + 1);
     if (const char* env = std::getenv("GOFERRO_FFT_PENCILS")) {
         int z = 0, y = 0, x = 0;
         if (std::sscanf(env, "%d,%d,%d", &z, &y, &x) == 3 && z > 0 && y > 0 && x > 0) {

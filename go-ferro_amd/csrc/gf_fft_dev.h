@@ -31,14 +31,15 @@ template <> struct FftComplex<float2> {
 
 // y rows (pencils of each component) of an x pass's workgroup of 256 threads:
 // from rows of 128 points on, as many as give each thread a point of the
-// tensor product (two of 128: the pass 20.9 -> 18.9 us at 128x128x32, with three
-// elements a thread where one row leaves half of the threads a second one);
-// one row of 64 or fewer, since those leave threads idle either way and more
-// workgroups are the better split (64x64x16, 20 steps: 2.18 ms; two rows 2.26,
-// four 2.21).
-inline int x_pencils(int64_t nx, int64_t ny) {
+// tensor product, where that leaves four workgroups per CU (two rows of 128:
+// the pass 20.9 -> 19.3 us at 128x128x32, three elements a thread where one row
+// leaves half of the threads a second one; 128x256x32, 40 steps 18.95 -> 18.30
+// ms), else one: 128x64x32 adjoint 15.5 ms, with two rows 16.1; 128x32x8 7.7 and
+// 8.0.  Rows of 64 or fewer leave threads idle either way (64x64x16, 20 steps:
+// 2.18 ms; two rows 2.26, four 2.21).
+inline int x_pencils(int64_t nx, int64_t ny, int64_t nzh) {
     int r = 1;
-    while (nx >= 128 && 2 * r * nx <= 256 && 2 * r <= ny) r *= 2;
+    while (nx >= 128 && 2 * r * nx <= 256 && 2 * r <= ny && ny * nzh >= 2048 * r) r *= 2;
     return r;
 }
 

@@ -684,7 +684,7 @@ gf_status conv32(gf_ctx* c, Adj32* s, const float* const* in, float* const* out,
     x.data = s->spb; x.kt = s->kt; x.tw = s->twx; x.nh = s->nh;
     x.den = static_cast<float>(-c->dx * c->dy * c->dz);
     x.nx = nx; x.ny = ny; x.lognx = ilog2i(nx); x.adjoint = adjoint ? 1 : 0;
-    x.rows = x_pencils(nx, ny);
+    x.rows = x_pencils(nx, ny, nzh);
     x.logr = ilog2i(x.rows);
     const size_t lx = sizeof(float2) * static_cast<size_t>(nx / 2 + fft_lds_elems(3 * static_cast<int64_t>(x.rows) * nx));
     hipLaunchKernelGGL(xconv32_kernel, dim3(ny / x.rows, nzh), dim3(kT), lx, c->stream, x);

@@ -568,10 +568,10 @@ def test_fp32_sweep_tracks_fp64(demag, anis):
     g32.close()
 
 
-@pytest.mark.parametrize("shape", [(128, 8, 8), (128, 16, 4), (256, 8, 4), (16, 32, 8)])
+@pytest.mark.parametrize("shape", [(128, 128, 32), (128, 16, 4), (256, 8, 4), (16, 32, 8)])
 def test_fp32_passes_at_workgroup_edges(shape):
-    """x rows of 128 points two to a workgroup (and of 256, one), eight y lines
-    and 32 z columns: the loss and the drive gradient track the FP64 sweep's."""
+    """x rows of 128 points two to a workgroup (and one, where there are few, or
+    of 256), eight y lines and 32 z columns: the loss and the drive gradient track the FP64 sweep's."""
     say("case FP32 passes", shape)
     prob = problem(shape=shape, rotate=False)
     f = inputs(shape)

@@ -31,11 +31,11 @@ def test_fm_mixed_materials_general_grid(shape, rotate):
     say("  worst stage store difference", worst)
 
 
-@pytest.mark.parametrize("shape", [(128, 1, 4), (128, 2, 8), (64, 4, 2), (4, 256, 4), (2, 512, 2), (16, 32, 8),
+@pytest.mark.parametrize("shape", [(128, 1, 4), (128, 128, 32), (64, 4, 2), (4, 256, 4), (2, 512, 2), (16, 32, 8),
                                    (256, 4, 4)])
 def test_power_of_two_passes_at_workgroup_edges(shape):
     """The field of the power-of-two passes where their split changes: x rows
-    of 128 points two to a workgroup (and one, where there is only one), y
+    of 128 points two to a workgroup (and one, where there are few), y
     lines of 256 and 512 with four and two to a workgroup, z columns 32 and 16
     to a workgroup."""
     from oracle.oracle import Oracle
