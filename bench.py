@@ -351,13 +351,13 @@ def bench_coupled(which: str, steps: int) -> dict:
     # compulsory bytes per stage of the state each class owns (fused RK4: 17 double
     # accesses per state component per step = 4.25 per stage) plus its cross reads.
     # The elastic class is its two launches (strain, eigenstrain and stress parts; then
-    # the stress divergence and updates): u, v state, the strain written for the
-    # magnets, the m store read for the eigenstrain.  The EM class is one launch
+    # the stress divergence and updates, with the magnet's stage): u, v state, the
+    # strain written for the magnets, the m store read for the eigenstrain.  The EM class is one launch
     # for Ampere, Faraday and the ferroelectric stage (gf_step runs them together).
     if which == "magnetoelastic":
         nmag = n * 16 // 64
-        per = {"elastic_stage": n * (6 * 4.25 * 8 + 4 + 6 * 8) + nmag * 3 * 8,
-               "mag_stage": nmag * (3 * 4.25 * 8 + 6 * 8 + 4 + 24)}
+        per = {"elastic_stage": n * (6 * 4.25 * 8 + 4 + 6 * 8) + nmag * 3 * 8 +
+               nmag * (3 * 4.25 * 8 + 6 * 8 + 4 + 24)}
     else:
         nfe = n * 200 // 1024
         ne = 6.77 * n

@@ -1710,20 +1710,22 @@ gf_status gf_mag_stage(gf_ctx* c, int stage) {
     if (stage == 4 && c->spin_on && !c->any_afm)
         if (gf_status e = spin_save(c, 0)) return e;
     hipEvent_t ev = nullptr;
-    timer_begin(c, GF_K_MAG_STAGE, &ev);
+    const bool with_force = c->el_pending;
+    c->el_pending = false;
+    if (with_force) ev = c->el_event;
+    else timer_begin(c, GF_K_MAG_STAGE, &ev);
     gf_status st;
     if (c->demag.fused) {
         st = hip_check(c, launch_mag_stage_fused(a, f, c->demag.h_in_spec, c->stream), "mag stage");
         if (!st) c->demag.m_in_spec = true;
     } else {
-        if (c->el_pending)
+        if (with_force)
             st = hip_check(c, launch_el_force_mag(c->el_args, a, c->d_fm_ids, c->d_fm_ids ? c->n_fm_ids : c->n,
                                                   c->stream), "elastic force and mag stage");
         else
             st = hip_check(c, launch_mag_stage(a, c->n, c->stream, c->d_fm_ids, c->n_fm_ids), "mag stage");
-        c->el_pending = false;
     }
-    timer_end(c, GF_K_MAG_STAGE, ev);
+    timer_end(c, with_force ? GF_K_ELASTIC_STAGE : GF_K_MAG_STAGE, ev);
     if (st) return st;
     c->mag_in_sel = c->mag_store_sel;
     c->mag_store_sel = out_sel;
@@ -1957,10 +1959,11 @@ gf_status gf_elastic_stage(gf_ctx* c, int stage) {
         if (!st && c->el_defer) {
             c->el_args = sa;
             c->el_pending = true;
-        } else if (!st) {
-            st = hip_check(c, launch_el_force(sa, c->stream), "elastic force");
+            c->el_event = ev;   // the stage's time ends with the magnet's launch
+        } else {
+            if (!st) st = hip_check(c, launch_el_force(sa, c->stream), "elastic force");
+            timer_end(c, GF_K_ELASTIC_STAGE, ev);
         }
-        timer_end(c, GF_K_ELASTIC_STAGE, ev);
         // the store just written is the stage's u store from here on
         if (!st) std::swap(c->us, c->us_alt);
     }

@@ -785,6 +785,7 @@ struct gf_ctx {
     bool el_defer = false;
     bool el_pending = false;
     gf::ElStageArgs el_args{};
+    hipEvent_t el_event = nullptr;   // the elastic stage's timer, when kernel timing is on
     // gf_step with a ferroelectric and electrodynamics: the FE stage's
     // launch is deferred and runs in the EM stage's Ampere/Faraday launch
     bool fe_defer = false;
