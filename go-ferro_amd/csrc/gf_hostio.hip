@@ -7,9 +7,10 @@
 // of 1 MiB, and from 8 MiB on several threads move them on, each with two
 // slots of its own, so that the faults run in parallel and a slot's copy
 // overlaps the move of the other: 40 steps of that film with the read-back
-// 121 -> 108 ms.  One slot and one wait also serve a small field better than a
-// copy per component (16x16x8, one step with its average and read-back: 161 ->
-// 127 us, with the average's partial sums written to pinned memory).
+// 121 -> 108 ms.  A field of up to one slot takes one wait and one move where
+// the direct copies wait for each component: 16x16x8, one step with its average
+// (whose partial sums go to pinned memory) and read-back 148 -> 107 us; 30x20x30
+// antiferromagnet, 10 steps 344 -> 335 us (369 with an event per component).
 //
 // The slots are shared by the process's contexts: at most kSlots of them,
 // allocated when first needed and given back with the last context.  One
@@ -75,6 +76,46 @@ hipError_t move_chunks(const std::vector<Chunk>& chunks, int w, int workers, hip
     return e;
 }
 
+hipError_t move_large(const std::vector<Chunk>& chunks, int workers, int device, hipStream_t s) {
+    // the work queued before is waited for once, not by every thread
+    hipError_t e = workers > 1 ? hipStreamSynchronize(s) : hipSuccess;
+    if (e != hipSuccess) return e;
+    std::atomic<int> failed{hipSuccess};
+    std::vector<std::thread> pool;
+    auto work = [&](int w) {
+        hipError_t r = w ? hipSetDevice(device) : hipSuccess;
+        if (r == hipSuccess) r = move_chunks(chunks, w, workers, s);
+        if (r != hipSuccess) failed = static_cast<int>(r);
+    };
+    int started = 1;
+    try {
+        pool.reserve(static_cast<size_t>(workers));
+        for (; started < workers; started++) pool.emplace_back(work, started);
+    } catch (const std::system_error&) {
+        // no more threads: this one does what they would have
+    }
+    work(0);
+    for (int w = started; w < workers; w++) work(w);
+    for (std::thread& t : pool) t.join();
+    return static_cast<hipError_t>(failed.load());
+}
+
+// A field of at most one slot: its parts into it, one wait, one move.
+hipError_t move_small(const std::vector<Chunk>& chunks, hipStream_t s) {
+    char*& slot = g_slot[0];
+    hipError_t e = hipSuccess;
+    if (!slot) e = hipHostMalloc(reinterpret_cast<void**>(&slot), kSlotBytes, hipHostMallocPortable);
+    size_t o = 0;
+    for (const Chunk& k : chunks) {
+        if (e == hipSuccess) e = hipMemcpyAsync(slot + o, k.src, k.bytes, hipMemcpyDeviceToHost, s);
+        o += k.bytes;
+    }
+    const hipError_t w = hipStreamSynchronize(s);   // also after a failure: no copy into the slot is left behind
+    if (e == hipSuccess) e = w;
+    if (e == hipSuccess) std::memcpy(chunks[0].dst, slot, o);   // the parts lie one after another there too
+    return e;
+}
+
 }  // namespace
 
 void host_slots_retain() {
@@ -107,30 +148,8 @@ gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* cou
                 chunks.push_back({from + o, dst + o, std::min(kSlotBytes, bytes - o)});
             dst += bytes;
         }
-        const int workers = total < kThreadsFrom ? 1 : kThreads;
-        // the work queued before is waited for once, not by every thread
-        if (workers > 1) {
-            const gf_status st = hip_check(c, hipStreamSynchronize(c->stream), "download sync");
-            if (st) return st;
-        }
-        std::atomic<int> failed{hipSuccess};
-        std::vector<std::thread> pool;
-        auto work = [&](int w) {
-            hipError_t r = w ? hipSetDevice(c->device) : hipSuccess;
-            if (r == hipSuccess) r = move_chunks(chunks, w, workers, c->stream);
-            if (r != hipSuccess) failed = static_cast<int>(r);
-        };
-        int started = 1;
-        try {
-            pool.reserve(static_cast<size_t>(workers));
-            for (; started < workers; started++) pool.emplace_back(work, started);
-        } catch (const std::system_error&) {
-            // no more threads: this one does what they would have
-        }
-        work(0);
-        for (int w = started; w < workers; w++) work(w);
-        for (std::thread& t : pool) t.join();
-        e = static_cast<hipError_t>(failed.load());
+        e = total <= kSlotBytes ? move_small(chunks, c->stream)
+                                : move_large(chunks, total < kThreadsFrom ? 1 : kThreads, c->device, c->stream);
     }
     if (e != hipSuccess) {
         double* dst = host;

@@ -18,10 +18,10 @@ def film(n, seed):
     return prob, np.random.default_rng(seed).standard_normal((3, 1, 1, n))
 
 
-# one double; a component of exactly one slot and one more and one fewer
-# double; the field just below, at and above the threads' threshold; many
+# one double; a field of just one slot and one cell more; a component of
+# exactly one slot and one more and one fewer double; the field just below, at and above the threads' threshold; many
 # slots with an odd tail
-@pytest.mark.parametrize("n", [1, 131071, 131072, 131073, 349525, 349526, 1400011])
+@pytest.mark.parametrize("n", [1, 43690, 43691, 131071, 131072, 131073, 349525, 349526, 1400011])
 def test_field_comes_back_whole(n):
     print("case download", n, file=sys.stderr, flush=True)
     prob, m = film(n, n)
