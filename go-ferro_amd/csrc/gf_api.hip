@@ -2209,7 +2209,8 @@ gf_status gf_step(gf_ctx* c, int64_t nsteps) {
                  !(c->flags & GF_FLAG_PLANE_EM) && (c->em_periodic_all || em_only_z_walls(c));
     // and the elastic force inside the FM stage's (Mur planes follow the
     // force at once, so it is not deferred with them)
-    c->el_defer = c->el_on && c->any_fm && !c->demag.fused && !(c->flags & GF_FLAG_1D_ABC) && narrow(c->n);
+    c->el_defer = c->el_on && c->any_fm && !c->demag.fused && !(c->flags & GF_FLAG_1D_ABC) &&
+                  el_narrow(c->nx, c->ny, c->nz, true);
     for (int64_t s = 0; s < nsteps; s++) {
         gf_status st = gf_time_advance(c);
         for (int stage = 1; stage <= 4 && !st; stage++) {

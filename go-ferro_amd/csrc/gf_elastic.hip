@@ -656,7 +656,8 @@ hipError_t launch_el_prep(const ElStageArgs& a, hipStream_t s) {
 
 hipError_t launch_el_force(const ElStageArgs& a, hipStream_t s) {
     // 32-bit element offsets where they reach
-    const auto force = narrow(a.f.nx * a.f.ny * a.f.nz) ? el_force_kernel<uint32_t> : el_force_kernel<int64_t>;
+    const bool small = el_narrow(a.f.nx, a.f.ny, a.f.nz, a.f.liao);
+    const auto force = small ? el_force_kernel<uint32_t> : el_force_kernel<int64_t>;
     const size_t lds = el_lds(a);
     const hipError_t e = allow_lds(reinterpret_cast<const void*>(force), lds);
     if (e != hipSuccess) return e;
@@ -664,7 +665,7 @@ hipError_t launch_el_force(const ElStageArgs& a, hipStream_t s) {
     return hipGetLastError();
 }
 
-// Grids of fewer than 2^28 cells (narrow); ids and count as launch_mag_stage.
+// Grids that el_narrow accepts; ids and count as launch_mag_stage.
 hipError_t launch_el_force_mag(const ElStageArgs& a, const StageArgs& m, const uint32_t* ids, int64_t count,
                                hipStream_t s) {
     const size_t lds = el_lds(a);

@@ -898,6 +898,13 @@ bool narrow(int64_t n);
 // doubles at src[p], one after another into host; waits for the stream
 gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* count, int parts, double* host);
 
+// true when the elastic force may use 32-bit byte offsets: for the cell arrays
+// and, with the Liao plane, for a history slot of 12 nx ny elements.  A grid of
+// five planes along z has a slot larger than its cell arrays.
+inline bool el_narrow(int64_t nx, int64_t ny, int64_t nz, bool liao) {
+    return narrow(nx * ny * nz) && (!liao || 3 * kHistPlanes * nx * ny <= (int64_t{1} << 29));
+}
+
 // launchers (gf_llg.hip)
 // ids: when set, the count FM cells the stage runs over (else all n cells)
 hipError_t launch_mag_stage(const StageArgs& a, int64_t n, hipStream_t s, const uint32_t* ids = nullptr,
