@@ -39,11 +39,13 @@ __global__ void __launch_bounds__(256) mag_stage_kernel(StageArgs a) {
 }
 
 // The same over a list of the FM cells: a layered magnet fills whole
-// waves instead of loading the inputs of every non-magnetic cell first.
-__global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs a, const uint32_t* ids, uint32_t count) {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+// waves instead of loading the inputs of every non-magnetic cell first.  The
+// list is of 32-bit indices on every grid that has one (up to 2^32 cells).
+template <class I>
+__global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs a, const uint32_t* ids, I count) {
+    const I t = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (t >= count) return;
-    fm_point<uint32_t>(a, ldu(ids, t));
+    fm_point<I>(a, static_cast<I>(ldu(ids, t)));
 }
 
 // The FM stage fused with the z transforms of the FFT magnetostatics, for
@@ -426,9 +428,11 @@ bool narrow(int64_t n) { return n < (int64_t{1} << 28); }
 
 hipError_t launch_mag_stage(const StageArgs& a, int64_t n, hipStream_t s, const uint32_t* ids, int64_t count) {
     if (ids) {
-        if (count > 0)
-            hipLaunchKernelGGL(mag_stage_list_kernel, dim3(static_cast<unsigned>((count + 255) / 256)), dim3(256), 0, s,
-                               a, ids, static_cast<uint32_t>(count));
+        const dim3 grid(static_cast<unsigned>((count + 255) / 256));
+        if (count > 0 && narrow(n))
+            hipLaunchKernelGGL(mag_stage_list_kernel<uint32_t>, grid, dim3(256), 0, s, a, ids, static_cast<uint32_t>(count));
+        else if (count > 0)
+            hipLaunchKernelGGL(mag_stage_list_kernel<int64_t>, grid, dim3(256), 0, s, a, ids, count);
         return hipGetLastError();
     }
     const int64_t blocks = (n + 255) / 256;

@@ -22,10 +22,13 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("rule", ["elastic_force"])
+@pytest.mark.parametrize("rule", ["elastic_force", "magnet_list", "cell_div"])
 def test_offset_rule(driver, rule):
     """elastic_force: the cell arrays and, with the Liao plane, a history slot
     of 12 nx ny elements stay within 32-bit byte offsets, and no grid that
-    does is refused the 32-bit form."""
+    does is refused the 32-bit form.  magnet_list: the stage over a list of FM
+    cells uses 64-bit offsets from 2^28 cells on.  cell_div: the multiplications
+    that stand for divisions of a cell index by an axis length are exact up to
+    the largest index the 32-bit kernels take."""
     out = subprocess.run([str(driver), rule], capture_output=True, text=True, timeout=60)
     assert out.returncode == 0, out.stdout + out.stderr
