@@ -15,14 +15,13 @@
 // The slots are shared by the process's contexts: at most kSlots of them,
 // allocated when first needed and given back with the last context.  One
 // call holds them at a time; a call that finds them held (another thread's)
-// copies directly, as does one whose slot cannot be allocated.
+// copies directly, as does one that cannot allocate a slot or an event.  What
+// a copy, or the work queued before it, fails with is the call's error.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
 #include <mutex>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 #include "gf_internal.h"
 
@@ -34,86 +33,153 @@ constexpr size_t kSlotBytes = size_t{1} << 20;
 constexpr int kThreads = 8;
 constexpr int kSlots = 2 * kThreads;
 constexpr size_t kThreadsFrom = size_t{8} << 20;
+constexpr int kParts = 9;         // most arrays of a field
 
 std::mutex g_slots_lock;          // held while the slots are used or freed
 std::mutex g_users_lock;
 int64_t g_users = 0;              // contexts alive
 char* g_slot[kSlots] = {};
 
+// The parts of a field one after another in host memory, as chunks of at most
+// a slot.
 struct Chunk {
     const char* src;
     char* dst;
     size_t bytes;
 };
+struct Chunks {
+    const double* const* src;
+    const int64_t* count;
+    int parts;
+    double* host;
+    int first[kParts + 1] = {};   // of a part; the last is the number of all
 
-// Chunks w, w + workers, ... through the slots w, w + workers, ... below
-// 2 * workers.
-hipError_t move_chunks(const std::vector<Chunk>& chunks, int w, int workers, hipStream_t s) {
-    hipEvent_t ev[2] = {nullptr, nullptr};
-    hipError_t e = hipSuccess;
-    auto send = [&](size_t i, int b) {
-        char*& slot = g_slot[w + b * workers];
-        if (!slot) e = hipHostMalloc(reinterpret_cast<void**>(&slot), kSlotBytes, hipHostMallocPortable);
-        if (e == hipSuccess && !ev[b]) e = hipEventCreateWithFlags(&ev[b], hipEventDisableTiming);
-        if (e == hipSuccess) e = hipMemcpyAsync(slot, chunks[i].src, chunks[i].bytes, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(ev[b], s);
-    };
-    const size_t n = chunks.size(), step = static_cast<size_t>(workers);
-    for (int b = 0; b < 2 && e == hipSuccess; b++) {
-        const size_t i = static_cast<size_t>(w) + static_cast<size_t>(b) * step;
-        if (i < n) send(i, b);
+    Chunks(const double* const* s, const int64_t* n, int p, double* h) : src(s), count(n), parts(p), host(h) {
+        for (int q = 0; q < p; q++) first[q + 1] = first[q] + static_cast<int>((bytes(q) + kSlotBytes - 1) / kSlotBytes);
     }
-    int b = 0;
-    for (size_t i = static_cast<size_t>(w); i < n && e == hipSuccess; i += step, b ^= 1) {
-        if ((e = hipEventSynchronize(ev[b])) != hipSuccess) break;
-        std::memcpy(chunks[i].dst, g_slot[w + b * workers], chunks[i].bytes);
-        if (i + 2 * step < n) send(i + 2 * step, b);
+    size_t bytes(int part) const { return sizeof(double) * static_cast<size_t>(count[part]); }
+    int size() const { return first[parts]; }
+    Chunk operator[](int i) const {
+        int q = 0;
+        char* dst = reinterpret_cast<char*>(host);
+        for (; i >= first[q + 1]; q++) dst += bytes(q);
+        const size_t o = static_cast<size_t>(i - first[q]) * kSlotBytes;
+        return {reinterpret_cast<const char*>(src[q]) + o, dst + o, std::min(kSlotBytes, bytes(q) - o)};
+    }
+};
+
+// The context's device while events are made for its stream, and the
+// caller's again after it.
+struct OnDevice {
+    int was = -1;
+    explicit OnDevice(int device) {
+        if (hipGetDevice(&was) != hipSuccess || was == device || hipSetDevice(device) != hipSuccess) was = -1;
+    }
+    ~OnDevice() {
+        if (was >= 0) (void)hipSetDevice(was);
+    }
+};
+
+struct Events {
+    hipEvent_t e[kSlots] = {};
+    bool make(int n) {
+        for (int i = 0; i < n; i++)
+            if (hipEventCreateWithFlags(&e[i], hipEventDisableTiming) != hipSuccess) return false;
+        return true;
+    }
+    ~Events() {
+        for (hipEvent_t v : e)
+            if (v) (void)hipEventDestroy(v);
+    }
+};
+
+// The first n slots, allocated where they are not yet.
+bool have_slots(int n) {
+    for (int i = 0; i < n; i++)
+        if (!g_slot[i] && hipHostMalloc(reinterpret_cast<void**>(&g_slot[i]), kSlotBytes, hipHostMallocPortable) != hipSuccess) {
+            g_slot[i] = nullptr;
+            return false;
+        }
+    return true;
+}
+
+// Chunks w, w + workers, ... through the slots w and w + workers.
+hipError_t move_chunks(const Chunks& chunks, const Events& ev, int w, int workers, hipStream_t s) {
+    hipError_t e = hipSuccess;
+    auto send = [&](int i, int b) {
+        const Chunk k = chunks[i];
+        e = hipMemcpyAsync(g_slot[b], k.src, k.bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = hipEventRecord(ev.e[b], s);
+    };
+    const int n = chunks.size();
+    for (int i = w; i < n && i < 2 * workers && e == hipSuccess; i += workers) send(i, i);
+    int b = w;
+    for (int i = w; i < n && e == hipSuccess; i += workers, b = b == w ? w + workers : w) {
+        if ((e = hipEventSynchronize(ev.e[b])) != hipSuccess) break;
+        const Chunk k = chunks[i];
+        std::memcpy(k.dst, g_slot[b], k.bytes);
+        if (i + 2 * workers < n) send(i + 2 * workers, b);
     }
     // no copy into a slot is left behind when a call fails
-    if (e != hipSuccess) hipStreamSynchronize(s);
-    for (hipEvent_t v : ev)
-        if (v) hipEventDestroy(v);
+    if (e != hipSuccess) (void)hipStreamSynchronize(s);
     return e;
 }
 
-hipError_t move_large(const std::vector<Chunk>& chunks, int workers, int device, hipStream_t s) {
+hipError_t move_large(const Chunks& chunks, const Events& ev, int workers, int device, hipStream_t s) {
     // the work queued before is waited for once, not by every thread
     hipError_t e = workers > 1 ? hipStreamSynchronize(s) : hipSuccess;
     if (e != hipSuccess) return e;
     std::atomic<int> failed{hipSuccess};
-    std::vector<std::thread> pool;
     auto work = [&](int w) {
         hipError_t r = w ? hipSetDevice(device) : hipSuccess;
-        if (r == hipSuccess) r = move_chunks(chunks, w, workers, s);
-        if (r != hipSuccess) failed = static_cast<int>(r);
+        if (r == hipSuccess) r = move_chunks(chunks, ev, w, workers, s);
+        int none = hipSuccess;
+        if (r != hipSuccess) failed.compare_exchange_strong(none, static_cast<int>(r));
     };
+    std::thread pool[kThreads];
     int started = 1;
     try {
-        pool.reserve(static_cast<size_t>(workers));
-        for (; started < workers; started++) pool.emplace_back(work, started);
-    } catch (const std::system_error&) {
+        for (; started < workers; started++) pool[started] = std::thread(work, started);
+    } catch (...) {
         // no more threads: this one does what they would have
     }
     work(0);
     for (int w = started; w < workers; w++) work(w);
-    for (std::thread& t : pool) t.join();
+    for (std::thread& t : pool)
+        if (t.joinable()) t.join();
     return static_cast<hipError_t>(failed.load());
 }
 
 // A field of at most one slot: its parts into it, one wait, one move.
-hipError_t move_small(const std::vector<Chunk>& chunks, hipStream_t s) {
-    char*& slot = g_slot[0];
+hipError_t move_small(const Chunks& chunks, hipStream_t s) {
+    char* const slot = g_slot[0];
     hipError_t e = hipSuccess;
-    if (!slot) e = hipHostMalloc(reinterpret_cast<void**>(&slot), kSlotBytes, hipHostMallocPortable);
     size_t o = 0;
-    for (const Chunk& k : chunks) {
-        if (e == hipSuccess) e = hipMemcpyAsync(slot + o, k.src, k.bytes, hipMemcpyDeviceToHost, s);
+    for (int i = 0; i < chunks.size() && e == hipSuccess; i++) {
+        const Chunk k = chunks[i];
+        e = hipMemcpyAsync(slot + o, k.src, k.bytes, hipMemcpyDeviceToHost, s);
         o += k.bytes;
     }
     const hipError_t w = hipStreamSynchronize(s);   // also after a failure: no copy into the slot is left behind
     if (e == hipSuccess) e = w;
-    if (e == hipSuccess) std::memcpy(chunks[0].dst, slot, o);   // the parts lie one after another there too
+    if (e == hipSuccess) std::memcpy(chunks.host, slot, o);   // the parts lie one after another there too
     return e;
+}
+
+// Through the slots, with the result in *e; false, with nothing copied, when
+// a slot or an event cannot be had.
+bool through_slots(gf_ctx* c, const Chunks& chunks, size_t total, hipError_t* e) {
+    if (total <= kSlotBytes) {
+        if (!have_slots(1)) return false;
+        *e = move_small(chunks, c->stream);
+        return true;
+    }
+    const int workers = total < kThreadsFrom ? 1 : kThreads, slots = std::min(2 * workers, chunks.size());
+    const OnDevice here(c->device);
+    Events ev;
+    if (!have_slots(slots) || !ev.make(slots)) return false;
+    *e = move_large(chunks, ev, workers, c->device, c->stream);
+    return true;
 }
 
 }  // namespace
@@ -128,43 +194,30 @@ void host_slots_release() {
     if (--g_users > 0) return;
     std::lock_guard<std::mutex> h(g_slots_lock);
     for (char*& p : g_slot) {
-        if (p) hipHostFree(p);
+        if (p) (void)hipHostFree(p);
         p = nullptr;
     }
 }
 
 gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* count, int parts, double* host) {
-    std::unique_lock<std::mutex> held(g_slots_lock, std::try_to_lock);
+    const Chunks chunks(src, count, parts, host);
     size_t total = 0;
-    for (int p = 0; p < parts; p++) total += sizeof(double) * static_cast<size_t>(count[p]);
-    hipError_t e = hipErrorOutOfMemory;
+    for (int p = 0; p < parts; p++) total += chunks.bytes(p);
+    std::unique_lock<std::mutex> held(g_slots_lock, std::try_to_lock);
+    hipError_t e = hipSuccess;
     if (held.owns_lock()) {
-        std::vector<Chunk> chunks;
-        char* dst = reinterpret_cast<char*>(host);
-        for (int p = 0; p < parts; p++) {
-            const char* from = reinterpret_cast<const char*>(src[p]);
-            const size_t bytes = sizeof(double) * static_cast<size_t>(count[p]);
-            for (size_t o = 0; o < bytes; o += kSlotBytes)
-                chunks.push_back({from + o, dst + o, std::min(kSlotBytes, bytes - o)});
-            dst += bytes;
-        }
-        e = total <= kSlotBytes ? move_small(chunks, c->stream)
-                                : move_large(chunks, total < kThreadsFrom ? 1 : kThreads, c->device, c->stream);
+        // an error of a copy or of the work before it is the call's
+        if (through_slots(c, chunks, total, &e)) return hip_check(c, e, "download");
+        (void)hipGetLastError();   // what made the slots unusable is not the next launch's error
     }
-    if (e != hipSuccess) {
-        double* dst = host;
-        e = hipSuccess;
-        hipGetLastError();   // what made the slots unusable is not the next launch's error
-        for (int p = 0; p < parts && e == hipSuccess; p++) {
-            e = hipMemcpyAsync(dst, src[p], sizeof(double) * static_cast<size_t>(count[p]), hipMemcpyDeviceToHost,
-                               c->stream);
-            dst += count[p];
-        }
-        const gf_status st = hip_check(c, e, "download");
-        if (st) return st;
-        return hip_check(c, hipStreamSynchronize(c->stream), "download sync");
+    double* dst = host;
+    for (int p = 0; p < parts && e == hipSuccess; p++) {
+        e = hipMemcpyAsync(dst, src[p], chunks.bytes(p), hipMemcpyDeviceToHost, c->stream);
+        dst += count[p];
     }
-    return GF_OK;
+    const gf_status st = hip_check(c, e, "download");
+    if (st) return st;
+    return hip_check(c, hipStreamSynchronize(c->stream), "download sync");
 }
 
 }  // namespace gf
