@@ -27,6 +27,8 @@ size_t g_done = 0;
 int g_mallocs = 0, g_frees = 0, g_events = 0;
 size_t g_to_slots = 0;             // copies whose destination a slot is
 hipError_t g_last = hipSuccess;
+hipMemoryType g_type = hipMemoryTypeUnregistered;   // of the caller's buffer
+bool g_known = true;                                // the runtime answers for it
 thread_local int t_device = 0;
 
 // The call that fails: the `at`-th of the named kind from now on, every
@@ -111,6 +113,11 @@ hipError_t hipStreamSynchronize(hipStream_t) {
     finish(g_queue.size());
     return hipSuccess;
 }
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t* a, const void*) {
+    if (!g_known) return g_last = hipErrorInvalidValue;
+    a->type = g_type;
+    return hipSuccess;
+}
 hipError_t hipGetDevice(int* d) { *d = t_device; return hipSuccess; }
 hipError_t hipSetDevice(int d) { t_device = d; return hipSuccess; }
 hipError_t hipGetLastError() {
@@ -184,6 +191,8 @@ void clear() {
     g_last = hipSuccess;
     g_new_in = -1;
     g_thread_in = -1;
+    g_type = hipMemoryTypeUnregistered;
+    g_known = true;
 }
 
 int bad(const char* what, const Field& f, int k) {
@@ -200,6 +209,7 @@ int whole() {
             for (int r = 0; r < 3; r++) {
                 clear();
                 t_device = device;
+                g_known = r != 1;
                 if (f.read(c) || !f.whole() || g_last || g_done != g_queue.size()) return bad("whole", f, r);
                 if (t_device != device || g_events) return bad("left behind", f, r);
             }
@@ -207,6 +217,22 @@ int whole() {
         }
         if (g_mallocs != g_frees) return bad("slots not given back", f, g_mallocs - g_frees);
     }
+    return 0;
+}
+
+// A buffer the caller pinned, or a device's: one copy a part, straight into it.
+int known() {
+    for (hipMemoryType type : {hipMemoryTypeHost, hipMemoryTypeDevice, hipMemoryTypeManaged})
+        for (const auto& n : kFields) {
+            Field f(n);
+            gf_ctx c;
+            c.device = t_device = 1;
+            clear();
+            g_type = type;
+            const int before = g_mallocs;
+            if (f.read(c) || !f.whole() || g_to_slots || g_mallocs != before || g_queue.size() != n.size())
+                return bad("known memory", f, type);
+        }
     return 0;
 }
 
@@ -293,6 +319,7 @@ int contended() {
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "whole") return whole();
+    if (what == "known") return known();
     if (what == "unavailable") return unavailable();
     if (what == "errors") return errors();
     if (what == "host_limits") return host_limits();

@@ -1,6 +1,7 @@
 """Reading fields back: the copies go through pinned slots of 1 MiB and, from
 8 MiB on, several threads; a call that finds the slots held by another
-thread's copies directly.  Bytes must be those uploaded, whatever the path."""
+thread's, or whose buffer the caller pinned, copies directly.  Bytes must be those uploaded, whatever the path."""
+import ctypes
 import sys
 import threading
 
@@ -57,3 +58,20 @@ def test_threads_read_their_own_contexts():
     for c, _ in ctxs:
         c.close()
     assert not bad
+
+
+@pytest.mark.parametrize("n", [1, 43691, 349526, 1400011])
+def test_pinned_buffer_comes_back_whole(n):
+    """A buffer from the HIP runtime the library links, by its own allocator."""
+    print("case pinned download", n, file=sys.stderr, flush=True)
+    prob, m = film(n, n)
+    c = Context(prob)
+    c.upload(FIELD_M, m)
+    hip = ctypes.CDLL("libamdhip64.so.7")
+    ptr = ctypes.c_void_p()
+    assert hip.hipHostMalloc(ctypes.byref(ptr), ctypes.c_size_t(24 * n), ctypes.c_uint(0)) == 0
+    out = ctypes.cast(ptr, ctypes.POINTER(ctypes.c_double))
+    assert c.lib.gf_download(c._h, FIELD_M, out, 3 * n) == 0
+    np.testing.assert_array_equal(np.ctypeslib.as_array(out, (3 * n,)), m.ravel())
+    assert hip.hipHostFree(ptr) == 0
+    c.close()
