@@ -139,6 +139,67 @@ def test_fe_em_steps_at_group_edges(shape, flags):
     o.close()
 
 
+def current_and_conductor(shape, periodic_z=False, flags=0):
+    """A ferroelectric between two conductors that end at the z walls, with a
+    current box over the cells of one wall: the edges next to that wall, which
+    its own threads evaluate once more, see all three."""
+    prob, p, q = fe_film(shape=shape, flags=flags, source=False)
+    prob.materials = [prob.materials[0], Material.make(r_permittivity=3.0, conductivity=2e5, **EM_MAT),
+                      Material.make(r_permittivity=7.0, conductivity=5e4, **EM_MAT)]
+    cell = prob.material_cell
+    nz = shape[2]
+    cell[:, :, :nz // 3] = 2
+    cell[:, :, 2 * nz // 3:] = 3
+    if periodic_z:
+        prob.periodic = (True, True, True)
+    prob.flags |= FLAG_JF_INPUT
+    prob.Jf_input_type, prob.Jf_input_component, prob.Jf_input_amp, prob.Jf_input_freq = 1, "y", 2e12, 5e16
+    prob.Jf_input_sigma, prob.num_Jf_cycles = 5e-16, 3
+    prob.Jfin_lo, prob.Jfin_hi = (0, 0, nz - 2), (shape[0] - 1, max(shape[1] - 2, 0), nz - 1)
+    return prob, p, q
+
+
+@pytest.mark.parametrize("shape,periodic_z,flags", [((4, 5, 12), False, 0), ((1, 2, 7), False, 0),
+                                                    ((3, 4, 9), False, FLAG_PEC_Z), ((3, 2, 6), True, 0),
+                                                    ((2, 3, 8), False, FLAG_1D_ABC | FLAG_1D_ABC_EM_ONLYTOP)])
+def test_fe_em_steps_with_current_and_conductor(shape, periodic_z, flags):
+    """gf_step's one launch with a free current and conductors at the walls,
+    against the oracle (the per-stage bound); the oracle without either of
+    them is far from it, so that both count."""
+    from oracle.oracle import Oracle
+    say("case fe + em steps with current and conductor", shape, periodic_z, flags)
+    E = random_yee(shape, FIELD_E_EM, 1e6, 4)
+    H = random_yee(shape, FIELD_H_EM, 3e3, 5)
+
+    def start(kind, change=None):
+        prob, p, q = current_and_conductor(shape, periodic_z, flags)
+        if change:
+            change(prob)
+        c = kind(prob)
+        for fid, val in ((FIELD_P, p), (FIELD_Q, q), (FIELD_E_EM, E), (FIELD_H_EM, H)):
+            (c.upload if kind is Context else c.set)(fid, val)
+        return c
+
+    def no_current(prob):
+        prob.flags &= ~FLAG_JF_INPUT
+
+    def no_conductor(prob):
+        for mat in prob.materials[1:]:
+            mat.conductivity = 0.0
+
+    g, o = start(Context), start(Oracle)
+    others = [start(Oracle, no_current), start(Oracle, no_conductor)]
+    for steps in (1, 2):
+        for c in (g, o, *others):
+            c.step(steps)
+        for fid in (FIELD_P, FIELD_Q, FIELD_E_EM, FIELD_H_EM, FIELD_E_CELL, FIELD_H_CELL):
+            assert rel(g.download(fid), o.get(fid)) <= 1e-12, (fid, steps)
+    for c in others:
+        assert rel(c.get(FIELD_E_EM), o.get(FIELD_E_EM)) > 1e-4
+    for c in (g, o, *others):
+        c.close()
+
+
 def boxed_media(shape=(8, 10, 12), flags=0, jf_type=1, plane=True):
     """Non-periodic in every direction: Mur (or PEC) walls on all six faces,
     a conductor, a Drude metal with two poles, a PEC inclusion, a plane
