@@ -13,7 +13,13 @@
 // antiferromagnet, 10 steps 344 -> 335 us (369 with an event per component).
 //
 // The slots are shared by the process's contexts: at most kSlots of them,
-// allocated when first needed and given back with the last context.  One
+// allocated when they pay and given back with the last context.  A slot takes
+// about 0.1 ms to allocate and free again, and saves 26 us of a field of up to
+// 48 KB, about 20 us of a MB of a larger one: a program that reads one field
+// and ends is slower for it (12.6 MB: first read-back 0.79 -> 1.54 ms, end of
+// the context 4.4 -> 5.3 ms).  So slots come with the fourth read-back of up to a
+// slot, or once the larger ones have moved kPays bytes for each slot they
+// need; what came before copied directly.  One
 // call holds them at a time; a call that finds them held (another thread's)
 // copies directly, as does one into memory the runtime knows (which the caller
 // pinned: 201 MB in 3.6 ms, 6.6 through the slots; 1.4 MB 53 and 82 us) and one that cannot allocate a slot or an event.  What
@@ -35,11 +41,15 @@ constexpr int kThreads = 8;
 constexpr int kSlots = 2 * kThreads;
 constexpr size_t kThreadsFrom = size_t{8} << 20;
 constexpr int kParts = 9;         // most arrays of a field
+constexpr int kPaysCalls = 4;
+constexpr size_t kPays = size_t{4} << 20;
 
 std::mutex g_slots_lock;          // held while the slots are used or freed
 std::mutex g_users_lock;
 int64_t g_users = 0;              // contexts alive
 char* g_slot[kSlots] = {};
+int g_small_reads = 0;            // read-backs since the slots were last given back
+size_t g_large_bytes = 0;
 
 // The parts of a field one after another in host memory, as chunks of at most
 // a slot.
@@ -94,8 +104,16 @@ struct Events {
     }
 };
 
-// The first n slots, allocated where they are not yet.
-bool have_slots(int n) {
+// The first n slots for a field of `total` bytes, allocated where they are not
+// yet; false when they do not pay yet or cannot be had.
+bool have_slots(int n, size_t total) {
+    if (g_slot[n - 1]) return true;
+    if (total <= kSlotBytes) {
+        if (++g_small_reads < kPaysCalls) return false;
+    } else {
+        g_large_bytes += total;
+        if (g_large_bytes / static_cast<size_t>(n) < kPays) return false;
+    }
     for (int i = 0; i < n; i++)
         if (!g_slot[i] && hipHostMalloc(reinterpret_cast<void**>(&g_slot[i]), kSlotBytes, hipHostMallocPortable) != hipSuccess) {
             g_slot[i] = nullptr;
@@ -168,17 +186,17 @@ hipError_t move_small(const Chunks& chunks, hipStream_t s) {
 }
 
 // Through the slots, with the result in *e; false, with nothing copied, when
-// a slot or an event cannot be had.
+// they do not pay yet or a slot or an event cannot be had.
 bool through_slots(gf_ctx* c, const Chunks& chunks, size_t total, hipError_t* e) {
     if (total <= kSlotBytes) {
-        if (!have_slots(1)) return false;
+        if (!have_slots(1, total)) return false;
         *e = move_small(chunks, c->stream);
         return true;
     }
     const int workers = total < kThreadsFrom ? 1 : kThreads, slots = std::min(2 * workers, chunks.size());
     const OnDevice here(c->device);
     Events ev;
-    if (!have_slots(slots) || !ev.make(slots)) return false;
+    if (!have_slots(slots, total) || !ev.make(slots)) return false;
     *e = move_large(chunks, ev, workers, c->device, c->stream);
     return true;
 }
@@ -206,6 +224,8 @@ void host_slots_release() {
         if (p) (void)hipHostFree(p);
         p = nullptr;
     }
+    g_small_reads = 0;
+    g_large_bytes = 0;
 }
 
 gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* count, int parts, double* host) {

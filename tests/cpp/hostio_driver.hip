@@ -200,22 +200,56 @@ int bad(const char* what, const Field& f, int k) {
     return 1;
 }
 
+// Reads until a read goes through the slots, and counts the reads before it.
+int warm(Field& f, gf_ctx& c) {
+    for (int k = 0; k < 16; k++) {
+        clear();
+        if (f.read(c) || !f.whole() || g_last) return -1;
+        if (g_to_slots) return k;
+    }
+    return -1;
+}
+
 int whole() {
     for (const auto& n : kFields) {
         Field f(n);
         for (int device : {0, 1}) {   // the caller's current device, the context's or not
             gf_ctx c;
-            c.device = 1;
+            c.device = t_device = 1;
+            if (warm(f, c) < 0) return bad("no slot used", f, device);
             for (int r = 0; r < 3; r++) {
                 clear();
                 t_device = device;
                 g_known = r != 1;
                 if (f.read(c) || !f.whole() || g_last || g_done != g_queue.size()) return bad("whole", f, r);
                 if (t_device != device || g_events) return bad("left behind", f, r);
+                if (g_to_slots == 0) return bad("no slot used", f, device);
             }
-            if (g_to_slots == 0) return bad("no slot used", f, device);
         }
         if (g_mallocs != g_frees) return bad("slots not given back", f, g_mallocs - g_frees);
+    }
+    return 0;
+}
+
+// One read-back, or a few small ones, allocate nothing; the slots come when
+// the rule says so, serve other contexts and go with the last one.
+int pays() {
+    for (const auto& n : kFields) {
+        Field f(n);
+        const size_t bytes = sizeof(double) * f.want.size();
+        const int before = g_mallocs;
+        {
+            gf_ctx a, b;
+            a.device = b.device = t_device = 1;
+            const int reads = warm(f, a);
+            int chunks = 0;
+            for (int64_t k : n) chunks += static_cast<int>((sizeof(double) * k + gf::kSlotBytes - 1) / gf::kSlotBytes);
+            const size_t slots = bytes <= gf::kSlotBytes ? 1 : std::min(bytes < gf::kThreadsFrom ? 2 : gf::kSlots, chunks);
+            const int want = bytes <= gf::kSlotBytes ? 3 : static_cast<int>((slots * gf::kPays + bytes - 1) / bytes) - 1;
+            if (reads != want || g_mallocs - before != static_cast<int>(slots)) return bad("pays", f, reads);
+            if (warm(f, b) != 0) return bad("another context", f, 0);
+        }
+        if (g_frees != g_mallocs) return bad("given back", f, 0);
     }
     return 0;
 }
@@ -244,9 +278,11 @@ int unavailable() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                clear();
-                g_fail = {what, at, true, hipErrorOutOfMemory};
-                if (f.read(c) || !f.whole() || g_last || g_events) return bad(what, f, at);
+                for (int r = 0; r < 12; r++) {
+                    clear();
+                    g_fail = {what, at, true, hipErrorOutOfMemory};
+                    if (f.read(c) || !f.whole() || g_last || g_events) return bad(what, f, at);
+                }
             }
     return 0;
 }
@@ -256,12 +292,11 @@ int unavailable() {
 int errors() {
     for (const char* what : {"hipMemcpyAsync", "hipEventRecord", "hipEventSynchronize", "hipStreamSynchronize"})
         for (const auto& n : kFields)
-            for (int at = 0; at < 40; at += 1 + at / 4) {
+            for (int at = 0; at < 40; at += 1 + at / 2) {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                clear();
-                if (f.read(c)) return bad("first", f, at);
+                if (warm(f, c) < 0) return bad("no slot used", f, at);
                 clear();
                 g_fail = {what, at, false, hipErrorLaunchFailure};
                 const gf_status st = f.read(c);
@@ -281,6 +316,7 @@ int host_limits() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
+                if (warm(f, c) < 0) return bad("no slot used", f, at);
                 clear();
                 *limit = at;
                 const gf_status st = f.read(c);
@@ -296,8 +332,7 @@ int contended() {
         Field f(n);
         gf_ctx c;
         c.device = t_device = 1;
-        clear();
-        if (f.read(c)) return bad("first", f, 0);
+        if (warm(f, c) < 0) return bad("no slot used", f, 0);
         clear();
         std::atomic<int> step{0};
         std::thread other([&] {
@@ -319,6 +354,7 @@ int contended() {
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "whole") return whole();
+    if (what == "pays") return pays();
     if (what == "known") return known();
     if (what == "unavailable") return unavailable();
     if (what == "errors") return errors();
