@@ -2251,15 +2251,18 @@ gf_status gf_average(gf_ctx* c, int id, double out[3]) {
     double** f = field_for(c, id, false, &st);
     if (!f) return st;
     const double* ff[3] = {f[0], f[1], f[2]};
-    // the partial sums go straight to host memory: no copy after the launch
-    const size_t sums = static_cast<size_t>(3 * c->red_blocks);
-    if (!c->red_host)
-        st = hip_check(c, hipHostMalloc(reinterpret_cast<void**>(&c->red_host), sizeof(double) * sums,
-                                        hipHostMallocDefault), "hipHostMalloc sums");
-    if (!st) st = hip_check(c, launch_sum3(ff, c->n, c->red_host, c->red_blocks, c->stream), "sum");
+    double* const pinned = host_sums(c);
+    const double* part = pinned;
+    std::vector<double> copied;
+    st = hip_check(c, launch_sum3(ff, c->n, pinned ? pinned : c->red_partial, c->red_blocks, c->stream), "sum");
+    if (!st && !pinned) {
+        copied.resize(static_cast<size_t>(3 * c->red_blocks));
+        part = copied.data();
+        st = hip_check(c, hipMemcpyAsync(copied.data(), c->red_partial, sizeof(double) * copied.size(),
+                                         hipMemcpyDeviceToHost, c->stream), "sum copy");
+    }
     if (!st) st = hip_check(c, hipStreamSynchronize(c->stream), "sum sync");
     if (st) return st;
-    const double* part = c->red_host;
     const double cnt = static_cast<double>(id == GF_FIELD_M ? c->nfm : (id == GF_FIELD_P ? c->nfe : c->nafm));
     for (int a = 0; a < 3; a++) {
         double s = 0.;

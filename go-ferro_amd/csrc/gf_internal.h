@@ -835,7 +835,8 @@ struct gf_ctx {
     double* e0t0[6] = {};           // static crystal-frame eigenstrain at t0 (elastodynamics), on first use
     // reduction scratch
     double* red_partial = nullptr;
-    double* red_host = nullptr;     // pinned, on first use: the partial sums of an average
+    double* red_host = nullptr;     // pinned: the partial sums of an average (host_sums)
+    int32_t red_calls = 0;          // averages without it
     int64_t red_blocks = 0;
     gf::HostSlotsUser slots_user;
 
@@ -897,6 +898,9 @@ bool narrow(int64_t n);
 // device to host copies of whole fields (gf_hostio.hip): the parts of count[p]
 // doubles at src[p], one after another into host; waits for the stream
 gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* count, int parts, double* host);
+// the context's pinned memory for an average's partial sums, or null when it
+// does not pay yet or cannot be had (gf_hostio.hip)
+double* host_sums(gf_ctx* c);
 
 // true when the elastic force may use 32-bit byte offsets: for the cell arrays
 // and, with the Liao plane, for a history slot of 12 nx ny elements.  A grid of

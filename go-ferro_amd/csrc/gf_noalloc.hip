@@ -1,7 +1,8 @@
 // gf_noalloc.hip — an averaging entry point that allocates nothing.
 //
-// gf_average reduces a field with per-block partial sums in a buffer the
-// context allocates, copies the partials to the host and waits.  Callers
+// gf_average reduces a field to per-block partial sums in memory of the
+// context (device memory copied to the host, or pinned memory allocated when
+// averages recur) and waits for them.  Callers
 // that cannot allocate or wait (code under HIP graph capture, serving loops
 // that forbid hipMalloc) use gf_average_noalloc instead: the same sum3
 // kernel writes its partials into `scratch`, a file-scope device array of

@@ -349,12 +349,34 @@ int contended() {
     return 0;
 }
 
+// Pinned sums from the fourth average on; null, with no error left, while
+// they cannot be had.
+int sums() {
+    for (int fails = 0; fails < 3; fails++) {
+        gf_ctx c;
+        c.red_blocks = 7;
+        clear();
+        g_fail = {"hipHostMalloc", 0, true, hipErrorOutOfMemory};
+        for (int call = 1; call <= 40; call++) {
+            if (call == 4 * fails + 1) g_fail = Fail{};
+            const double* p = gf::host_sums(&c);
+            if ((p != nullptr) != (call >= 4 * (fails + 1)) || g_last) {
+                std::printf("sums: call %d after %d failures\n", call, fails);
+                return 1;
+            }
+        }
+        hipHostFree(c.red_host);
+    }
+    return 0;
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::string what = argc > 1 ? argv[1] : "";
     if (what == "whole") return whole();
     if (what == "pays") return pays();
+    if (what == "sums") return sums();
     if (what == "known") return known();
     if (what == "unavailable") return unavailable();
     if (what == "errors") return errors();

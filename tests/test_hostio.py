@@ -17,12 +17,12 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("case", ["whole", "pays", "known", "unavailable", "errors", "host_limits", "contended"])
+@pytest.mark.parametrize("case", ["whole", "pays", "sums", "known", "unavailable", "errors", "host_limits", "contended"])
 def test_read_back(driver, case):
     """whole: every byte, read only after it was waited for, from contexts of
     the caller's current device and of another; the slots given back with the
     last context.  pays: no slot is allocated before it saves what it costs.
-    known: memory the caller pinned is copied to directly.
+    sums: the same of an average's pinned sums.  known: memory the caller pinned is copied to directly.
     unavailable: no slot or event to be had is a direct copy.
     errors: a copy, record or wait that fails is the call's error.  host_limits:
     allocations or threads that fail are no exception.  contended: another
