@@ -126,19 +126,19 @@ void build_surface_bits(gf_ctx* c, bool (*kind)(const gf_ctx*, int64_t), int shi
             }
 }
 
-// The codes as the device holds them: with kMixed set (one magnetic material
-// has no such cell).
-std::vector<uint32_t> device_codes(const gf_ctx* c) {
-    std::vector<uint32_t> out = c->host_code;
+// The codes as the device holds them, with kMixed set; left empty where they
+// are the host's (one magnetic material has no such cell).
+void device_codes(const gf_ctx* c, std::vector<uint32_t>& out) {
     uint32_t seen = 0;
     bool several = false;
-    for (size_t i = 0; i < out.size() && !several; i++) {
-        if (!(out[i] & (kIsFM | kIsAFM))) continue;
-        const uint32_t t = out[i] & kMatMask;
+    for (size_t i = 0; i < c->host_code.size() && !several; i++) {
+        if (!(c->host_code[i] & (kIsFM | kIsAFM))) continue;
+        const uint32_t t = c->host_code[i] & kMatMask;
         several = seen && t != seen;
         seen = t;
     }
-    if (!several) return out;
+    if (!several) return;
+    out = c->host_code;
     const int64_t n3[3] = {c->nx, c->ny, c->nz}, step[3] = {c->ny * c->nz, c->nz, 1};
     int64_t q[3];
     for (q[0] = 0; q[0] < n3[0]; q[0]++)
@@ -157,7 +157,6 @@ std::vector<uint32_t> device_codes(const gf_ctx* c) {
                     if ((nb ^ own) & kMatMask) out[static_cast<size_t>(id)] |= kMixed;
                 }
             }
-    return out;
 }
 
 DevMaterial make_dev_material(const gf_material& m, double dt) {
@@ -871,6 +870,7 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
         return GF_ERR_ALLOC;
     }
     gf_status st = GF_OK;
+    std::vector<uint32_t> mixed;   // the device's codes where they differ from the host's
     try {
         c->nx = d->nx; c->ny = d->ny; c->nz = d->nz; c->n = d->nx * d->ny * d->nz;
         c->dx = d->dx; c->dy = d->dy; c->dz = d->dz;
@@ -917,6 +917,7 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
         if (c->any_fe) build_surface_bits(c, is_fe, kFeSurfShift);
         if (c->any_fm) build_surface_bits(c, is_fm, kFmSurfShift);
         if (c->any_afm) build_surface_bits(c, is_afm, kAfmSurfShift);
+        device_codes(c, mixed);
         if (c->flags & GF_FLAG_EMDYNAMIC) {
             const std::string why = em_unsupported(c, d);
             if (!why.empty()) {
@@ -943,8 +944,8 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
     if (!st) st = hip_check(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
     if (!st) st = hip_check(c, hipMalloc(&c->d_code, sizeof(uint32_t) * c->n), "hipMalloc code");
     if (!st)
-        st = hip_check(c, hipMemcpy(c->d_code, device_codes(c).data(), sizeof(uint32_t) * c->n, hipMemcpyHostToDevice),
-                       "copy code");
+        st = hip_check(c, hipMemcpy(c->d_code, (mixed.empty() ? c->host_code : mixed).data(), sizeof(uint32_t) * c->n,
+                                    hipMemcpyHostToDevice), "copy code");
     if (!st && c->any_fm && c->nfm < c->n && c->n <= INT64_C(0xffffffff)) {
         // the FM cells in index order: the unfused FM stage runs over them
         // alone (material kinds cannot change after set-up)
