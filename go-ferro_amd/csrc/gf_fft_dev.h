@@ -29,18 +29,18 @@ template <> struct FftComplex<float2> {
     static __device__ __forceinline__ float2 make(float re, float im) { return make_float2(re, im); }
 };
 
-// y rows (pencils of each component) of an x pass's workgroup of 256 threads:
-// from rows of 128 points on, as many as give each thread a point of the
-// tensor product, where that leaves four workgroups per CU (two rows of 128:
-// the pass 20.9 -> 19.3 us at 128x128x32, three elements a thread where one row
-// leaves half of the threads a second one; 128x256x32, 40 steps 18.95 -> 18.30
-// ms), else one: 128x64x32 adjoint 15.5 ms, with two rows 16.1; 128x32x8 7.7 and
-// 8.0.  Rows of 64 or fewer leave threads idle either way (64x64x16, 20 steps:
-// 2.18 ms; two rows 2.26, four 2.21).
+// y rows (pencils of each component) of an x pass's workgroup of 256 threads.
+// One, but two where a row is half of the threads and two leave four
+// workgroups per CU: one row of 128 gives half of the threads a second element
+// of three, two rows give each thread three and a point of the tensor product
+// (128x128x32: the pass 20.9 -> 19.3 us; 128x256x32, 40 steps 18.95 -> 18.30 ms;
+// with fewer workgroups 128x64x32 adjoint 15.5 ms, 16.1 with two; 128x32x8 7.7
+// and 8.0).  A row of 256 fills them alone (256x128x64: 670 us a step, 691 with
+// two).  Rows of 64 and 32 keep one, as they had: on small grids that is no worse
+// (64x64x16: 90 us a step with one, 94 with two, 90 with four), on wide ones it is
+// (64x256x128: 801, 723 and 693 us; 32x512x128: 1039, 849 and 779).
 inline int x_pencils(int64_t nx, int64_t ny, int64_t nzh) {
-    int r = 1;
-    while (nx >= 128 && 2 * r * nx <= 256 && 2 * r <= ny && ny * nzh >= 2048 * r) r *= 2;
-    return r;
+    return 2 * nx == 256 && ny >= 2 && ny * nzh >= 2048 ? 2 : 1;
 }
 
 // At most this many columns a workgroup of a z pass (three components): 32
