@@ -1,7 +1,7 @@
 // gf_fft_line.h — mixed-radix line transforms of the FFT passes, in
 // registers with LDS exchanges between the radix passes.
 //
-// A line of length n is a product of at most kMaxRadices radices of
+// A line of length n is a product of at most kMaxPasses radices of
 // {1..10, 12, 14, 15, 16}: two for most lengths up to 256, three up to 2048.
 // Each pass gives a thread one butterfly: R elements read together, the
 // R-point DFT in registers, R elements written (Stockham order: pass s of

@@ -327,7 +327,13 @@ const char* gf_last_error(const gf_ctx* ctx);
 /* Host <-> device copies of one field.  count is the number of doubles
  * (3*n for vector fields, see gf_field_size).  Uploading GF_FIELD_M also sets the stage store
  * to m, as initialize_device does (magnetic_initialize.cpp:1081-1097).
- * Both calls synchronise the context stream before returning. */
+ * Both calls synchronise the context stream before returning.
+ * gf_download copies directly into memory the runtime knows (hipHostMalloc);
+ * into ordinary memory it goes through pinned slots of 1 MiB that the process's
+ * contexts share, once they pay: at most 16, given back with the last context,
+ * with up to eight short-lived host threads from 8 MiB on.  One call holds the
+ * slots while it waits for its stream; calls of other threads meanwhile copy
+ * directly. */
 gf_status gf_upload(gf_ctx* ctx, int field_id, const double* host, size_t count);
 gf_status gf_download(gf_ctx* ctx, int field_id, double* host, size_t count);
 
