@@ -35,12 +35,15 @@ using em_dev::em_face;
 
 // Ampere and Faraday of a stage in one launch: both read only the stage
 // stores and write other arrays, so the edges and the faces are independent.
-template <class I>
+// kQ: a q store may be given (polarisation current).  Without what a launch
+// cannot meet (the z walls belong to the launch with the ferroelectric cells) the
+// kernel keeps to 72 VGPRs and 7 waves per SIMD.
+template <class I, bool kQ>
 __global__ void __launch_bounds__(em_dev::kEmGroup) em_eh_kernel(EmArgs a) {
     extern __shared__ double emtab[];
     const unsigned gE = em_dev::em_groups(em_dev::em_edges(a)), b = blockIdx.x;
     const I t = static_cast<I>(b < gE ? b : b - gE) * em_dev::kEmGroup + static_cast<I>(threadIdx.x);
-    if (b < gE) em_edge<I>(a, emtab, t);
+    if (b < gE) em_edge<I, kQ, false>(a, emtab, t);
     else if (t < static_cast<I>(em_dev::em_faces(a))) em_face<I>(a, t);
 }
 
@@ -230,8 +233,10 @@ hipError_t launch_em_eh(const EmArgs& a, hipStream_t s) {
     const int64_t nE = em_dev::em_edges(a), nH = em_dev::em_faces(a);
     const dim3 grid(em_dev::em_groups(nE) + em_dev::em_groups(nH)), block(em_dev::kEmGroup);
     const size_t lds = sizeof(double) * em_dev::kEmC * static_cast<size_t>(a.nmat);
-    if (narrow(nE + nH)) hipLaunchKernelGGL(em_eh_kernel<uint32_t>, grid, block, lds, s, a);
-    else hipLaunchKernelGGL(em_eh_kernel<int64_t>, grid, block, lds, s, a);
+    const auto eh = !narrow(nE + nH) ? em_eh_kernel<int64_t, true>
+                    : a.q[0]         ? em_eh_kernel<uint32_t, true>
+                                     : em_eh_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(eh, grid, block, lds, s, a);
     return hipGetLastError();
 }
 

@@ -95,7 +95,7 @@ __device__ __forceinline__ double edge_increment(const EmArgs& a, const double* 
             er = er + 1.;
         } else {
             const double* M = tab + (t - 1u) * kEmC;
-            if (a.q[0]) dP = dP + qv[q] * a.dt;
+            dP = dP + qv[q] * a.dt;
             er = er + M[0];
             cond = cond + M[1];
             pc = pc + M[2];
@@ -133,7 +133,7 @@ __device__ __forceinline__ double z_wall_edge(const EmArgs& a, int comp, bool to
 // A whole workgroup calls it, with e past the last edge in the last one's
 // spare threads: tab is the workgroup's material table, staged here after
 // the edge's own loads have been issued, so that both take one round trip.
-template <class I>
+template <class I, bool kQ, bool kWall>
 __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     const I nE = static_cast<I>(em_edges(a));
     const bool live = e < nE;
@@ -154,7 +154,7 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         const I l = e / (nz + 1), i = l / (ny + 1), j = l - i * (ny + 1);
         I k = e - l * (nz + 1);
         hist = (!a.per[1] && near(j, ny)) || (!a.per[2] && near(k, nz));
-        if (a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
+        if (kWall && a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
         const bool wj = j == 0 || j == ny, wk = k == 0 || k == nz;
         dead = (wj && !a.per[1]) || (wk && !a.per[2]);
         const I y1 = wj ? ny - 1 : j - 1, y3 = wj ? 0 : j, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
@@ -167,7 +167,7 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         const I l = e / (nz + 1), i = l / ny, j = l - i * ny;
         I k = e - l * (nz + 1);
         hist = (!a.per[0] && near(i, nx)) || (!a.per[2] && near(k, nz));
-        if (a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
+        if (kWall && a.zwall && (k == 0 || k == nz)) { wall = k == 0 ? -1 : 1; k = k == 0 ? 1 : nz - 1; }
         const bool wi = i == 0 || i == nx, wk = k == 0 || k == nz;
         dead = (wi && !a.per[0]) || (wk && !a.per[2]);
         const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
@@ -201,7 +201,7 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         cell[q] = C(ci[q], cj[q], ck[q]);
         tq[q] = ldu(a.code, cell[q]);
         hv[q] = ldd(a.hs[hf[q >> 1]], hp[q]);
-        if (a.q[0]) qv[q] = ldd(a.q[comp], cell[q]);
+        if (kQ && a.q[0]) qv[q] = ldd(a.q[comp], cell[q]);
     }
     load_emtab(tab, a.mats, a.nmat);
     if (!live) return;
@@ -223,18 +223,22 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     rk_state<I>(a.stage, e, k_, y, ac, a.eb[comp], a.eacc[comp], a.eo[comp]);
 }
 
-// dM of one cell next to a face (EMdynamic_solver.cpp:2290-2340); called
-// only where a magnetic increment is given.
+// What dM of one cell next to a face takes (EMdynamic_solver.cpp:2290-2340),
+// read only where a magnetic increment is given.
+struct CellDm {
+    uint32_t mat;
+    double f, f1, f2;
+};
 template <class I>
-__device__ __forceinline__ double cell_dm(const EmArgs& a, int comp, I id, double& count) {
-    const uint32_t t = ldu(a.code, id) & kMatMask;
-    if (!t) return 0.;
-    const DevMaterial& M = a.mats[t - 1];
-    const double f = a.dm[0] ? ldd(a.dm[comp], id) : 0.;
-    const double f1 = a.dma1[0] ? ldd(a.dma1[comp], id) : 0.;
-    const double f2 = a.dma2[0] ? ldd(a.dma2[comp], id) : 0.;
+__device__ __forceinline__ CellDm load_dm(const EmArgs& a, int comp, I id) {
+    return {ldu(a.code, id) & kMatMask, a.dm[0] ? ldd(a.dm[comp], id) : 0., a.dma1[0] ? ldd(a.dma1[comp], id) : 0.,
+            a.dma2[0] ? ldd(a.dma2[comp], id) : 0.};
+}
+__device__ __forceinline__ double cell_dm(const EmArgs& a, const CellDm& c, double& count) {
+    if (!c.mat) return 0.;
+    const DevMaterial& M = a.mats[c.mat - 1];
     if (M.is_fm || M.is_afm) count = count + 1.;
-    return f * M.Ms + f1 * M.aMs[0] + f2 * M.aMs[1];
+    return c.f * M.Ms + c.f1 * M.aMs[0] + c.f2 * M.aMs[1];
 }
 
 // Faraday on face f of the concatenated Hx|Hy|Hz grids, with its RK update;
@@ -275,13 +279,17 @@ __device__ __forceinline__ void em_face(const EmArgs& a, I f) {
         ep[0] = EY(i + 1, j, k); ep[1] = EY(i, j, k); ep[2] = EX(i, j + 1, k); ep[3] = EX(i, j, k);
         c1 = C(i, j, z1); c2 = C(i, j, z2);
     }
+    // the cells first: their materials' records are a second trip to memory
+    const bool mag = a.dm[0] || a.dma1[0];
+    CellDm m1{}, m2{};
+    if (mag) { m1 = load_dm<I>(a, comp, c1); m2 = load_dm<I>(a, comp, c2); }
     const double y = ldd(a.hb[comp], f), ac = a.stage > 1 ? ldd(a.hacc[comp], f) : 0.;
     double ev[4];
     for (int q = 0; q < 4; q++) ev[q] = ldd(a.es[ef[q >> 1]], ep[q]);
     double k_ = -a.dt / kMu0 * ((ev[0] - ev[1]) * re[0] - (ev[2] - ev[3]) * re[1]);
-    if (a.dm[0] || a.dma1[0]) {
+    if (mag) {
         double cnt = 0.;
-        const double d1 = cell_dm<I>(a, comp, c1, cnt), d2 = cell_dm<I>(a, comp, c2, cnt);
+        const double d1 = cell_dm(a, m1, cnt), d2 = cell_dm(a, m2, cnt);
         if (cnt < 0.5) cnt = 1.;
         k_ = k_ - (d1 + d2) / cnt;
     }

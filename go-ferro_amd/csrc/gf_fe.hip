@@ -179,7 +179,7 @@ __global__ void __launch_bounds__(em_dev::kEmGroup) fe_em_kernel(FeStageArgs f, 
     const unsigned b = blockIdx.x, first = b < gC ? 0u : (b < gC + gE ? gC : gC + gE);
     const I t = static_cast<I>(b - first) * em_dev::kEmGroup + static_cast<I>(threadIdx.x);
     if (b < gC) { if (t < static_cast<I>(f.nx * f.ny * f.nz)) fe_cell<I>(f, t); }
-    else if (b < gC + gE) em_dev::em_edge<I>(e, emtab, t);
+    else if (b < gC + gE) em_dev::em_edge<I, true, true>(e, emtab, t);
     else if (t < static_cast<I>(em_dev::em_faces(e))) em_dev::em_face<I>(e, t);
 }
 
