@@ -417,19 +417,21 @@ struct Shapes {
 
 // Pencils per workgroup.  z and y passes write their output transposed,
 // so their pencil count sets the length of the store runs (16 B each);
-// the x pass reads and writes whole rows (x_pencils).  Eight y pencils make
-// whole 128 B lines of the y passes; sixteen only halved the number of workgroups (64x64x16, 20
-// steps: 2.40 ms with 16, 2.18 with 8, 2.30 with 4; 128x128x32 adjoint 74.8 and
-// 74.0 ms).  Lines of 256 and more keep to 1024 elements a workgroup while the
-// spectra stay in the caches (128x256x32, 40 steps: 18.3 ms with 8 pencils, 17.7
-// with 4), but not beyond (256x256x128: 108 ms with 8, 113 with 4: half lines).
+// the x pass reads and writes whole rows (x_pencils, y_pencils, z_pencils).  y
+// lines of 256 keep to 1024 elements a workgroup while the spectra stay in the
+// caches (128x256x32, 40 steps: 18.3 ms with 8 pencils, 17.7 with 4), but not
+// beyond (256x256x128: 108 ms with 8, 113 with 4: half lines).  Longer ones take
+// 2048, else their runs fall below 64 B (256x512x8: 654 us a step with 4 pencils,
+// 701 with 2; 256x1024x8: 1346 with 2, 1541 with 1), unless that leaves less than
+// two workgroups per CU (4x1024x32: 309 us a step with 2, 299 with 1).
 // GOFERRO_FFT_PENCILS="z,y,x" overrides the defaults (powers of two) for
 // tuning sweeps.
 Shapes shapes(const gf_ctx* c) {
     Shapes s;
     const int64_t spectra = 3 * c->nx * c->ny * (c->nz / 2 + 1) * static_cast<int64_t>(sizeof(double2));
-    int64_t bz = 2048, by = spectra <= (int64_t{64} << 20) ? 1024 : 2048, bx = 1024, cy = 8;
-    int64_t cz = z_pencils(c->nx, c->ny);
+    const bool short_y = c->ny <= 256 || 3 * c->nx * c->ny * (c->nz / 2 + 1) < 512 * 2048;
+    int64_t bz = 2048, by = spectra <= (int64_t{64} << 20) && short_y ? 1024 : 2048, bx = 1024;
+    int64_t cz = z_pencils(c->nx, c->ny, c->nz), cy = y_pencils(c->nx, c->ny, c->nz / 2 + 1);
     int64_t cx = x_pencils(c->nx, c->ny, c->nz / 2 + 1);
     if (const char* env = std::getenv("GOFERRO_FFT_PENCILS")) {
         int z = 0, y = 0, x = 0;

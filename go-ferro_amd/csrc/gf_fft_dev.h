@@ -44,9 +44,22 @@ inline int x_pencils(int64_t nx, int64_t ny, int64_t nzh) {
 }
 
 // At most this many columns a workgroup of a z pass (three components): 32
-// where that leaves four workgroups per CU (128x128x32 adjoint: 71.9 -> 70.9 ms,
-// FP32 48.4 -> 47.2), else 16 (64x64x16: 24.4 ms, 25.3 with 32).
-inline int64_t z_pencils(int64_t nx, int64_t ny) { return 3 * nx * (ny / 32) >= 1024 ? 32 : 16; }
+// where that is at most four elements a thread and leaves four workgroups per CU
+// (128x128x32 adjoint: 71.9 -> 70.9 ms, FP32 48.4 -> 47.2), else 16 (64x64x16:
+// 24.4 ms, 25.3 with 32; the five passes of 256x256x64 253 us, 263 with 32).
+inline int64_t z_pencils(int64_t nx, int64_t ny, int64_t nz) {
+    return 32 * nz <= 1024 && 3 * nx * (ny / 32) >= 1024 ? 32 : 16;
+}
+
+// At most this many lines a workgroup of a y pass: eight make whole 128 B lines
+// of the transposed side (64x64x16, 20 steps: 2.40 ms with 16, 2.18 with 8, 2.30
+// with 4; 128x128x32 adjoint 74.8 and 74.0 ms), sixteen where they are at most
+// two elements a thread and leave two workgroups per CU (the five passes of
+// 512x8x64 45 us, 51 with 8; of 256x1x256 28 and 34; of 256x32x32 39.3 and 40.0;
+// but 64x32x16 19.7 and 19.3, and 64x8x64 93 us a step, 91 with 8).
+inline int64_t y_pencils(int64_t nx, int64_t ny, int64_t nzh) {
+    return 16 * ny <= 512 && 3 * (nx / 16) * nzh >= 512 ? 16 : 8;
+}
 
 __device__ __forceinline__ double2 fft_cmul(double2 a, double2 b) {
     return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);

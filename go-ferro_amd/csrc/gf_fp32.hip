@@ -845,8 +845,8 @@ gf_status adjoint32_forward(gf_ctx* c, const gf_adjoint_desc* d, double* loss) {
     if (!st && s->ms) {
         s->nzh = c->nz / 2 + 1;
         s->nh = c->nx * c->ny * s->nzh;
-        s->pz = pencils_for(c->nz, 2048, z_pencils(c->nx, c->ny), c->ny);
-        s->py = pencils_for(c->ny, 2048, 8, c->nx);
+        s->pz = pencils_for(c->nz, 2048, z_pencils(c->nx, c->ny, c->nz), c->ny);
+        s->py = pencils_for(c->ny, 2048, y_pencils(c->nx, c->ny, s->nzh), c->nx);
         st = twiddles32(c, &s->twx, c->nx);
         if (!st) st = twiddles32(c, &s->twy, c->ny);
         if (!st) st = twiddles32(c, &s->twz, c->nz);

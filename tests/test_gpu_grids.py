@@ -52,6 +52,24 @@ def test_power_of_two_passes_at_workgroup_edges(shape):
     o.close()
 
 
+@pytest.mark.parametrize("shape", [(256, 4, 64), (256, 1, 128), (128, 32, 32), (256, 512, 4), (2, 1024, 4), (32, 64, 64)])
+def test_power_of_two_passes_of_short_and_long_lines(shape):
+    """Short y lines sixteen to a workgroup, lines of 512 and more by the size of
+    the launch, z lines of 64 sixteen columns to a workgroup."""
+    from oracle.oracle import Oracle
+    say("case power-of-two demag, short and long lines", shape)
+    prob, m = workloads.fm_film(shape)
+    g, o = Context(prob), Oracle(prob)
+    g.upload(FIELD_M, m)
+    o.set(FIELD_M, m)
+    g.demag()
+    o.demag()
+    hg, ho = g.download(FIELD_HSTAT), o.get(FIELD_HSTAT)
+    assert np.abs(hg - ho).max() <= 1e-12 * np.abs(ho).max()
+    g.close()
+    o.close()
+
+
 def test_fm_film_general_grid_fused_and_periodic():
     """The config-1 film physics on 20x12x16: periodic in x and y, the fused
     stage (nz = 16) with P = 4 columns dividing ny = 12."""
