@@ -127,7 +127,7 @@ __device__ __forceinline__ void rot_t(const double T[3][3], double ix, double iy
 // before the cell's code is known, the z neighbours come from the adjacent
 // lanes, and the gradient accumulators are read together, not each after the
 // write of the one before.  128x128x32: 39.2 -> 34.9 us.
-template <class I>
+template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
@@ -142,12 +142,13 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const P3 sp = {{a.y[0], a.y[1], a.y[2]}};
     double nv[6][3];
     const I nx = static_cast<I>(a.nx);
-    gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, nv);
+    uint32_t cd[6];
+    gather6_lanes_load<kMixed, I>(sp, a.code, x, y, z, nx, ny, nz, nv, cd);
     const double kb0 = ldd(a.kbar[0], id), kb1 = ldd(a.kbar[1], id), kb2 = ldd(a.kbar[2], id);
     const bool dem = a.hd[0] != nullptr;
     const double hd0 = dem ? ldd(a.hd[0], id) : 0., hd1 = dem ? ldd(a.hd[1], id) : 0.;
     const double hd2 = dem ? ldd(a.hd[2], id) : 0.;
-    gather6_lanes_shift<I>(z, nz, yc, nv);
+    gather6_lanes_shift<kMixed, I>(z, nz, yc, own, nv, cd);
     if (!(own & kIsFM)) {
         for (int c = 0; c < 3; c++) { std_(a.mbar[c], id, 0.); std_(a.hbar[c], id, 0.); }
         return;
@@ -156,8 +157,8 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
     const double mgx = yc[0], mgy = yc[1], mgz = yc[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil st = magnet_stencil<true, I>(yc, nv, a.code, (GMat*)a.mats, own, kFmSurfShift, -1, x, y, z, nx, ny, nz,
-                                               a.idx, a.idy, a.idz, M.Aex, M.Aex_self, M.dmi_slope);
+    const Stencil st = magnet_stencil<true, kMixed>(yc, nv, cd, (GMat*)a.mats, own, kFmSurfShift, -1, a.idx, a.idy,
+                                                    a.idz, M.Aex, M.Aex_self, M.dmi_slope);
     // exchange and interfacial DMI (zero without it) of the forward stage
     const double hex0 = M.exch * st.ex[0] + M.dmi_pos * st.d[2], hex1 = M.exch * st.ex[1] + M.dmi_pos * st.d[3];
     const double hex2 = M.exch * st.ex[2] + M.dmi_neg * (st.d[0] + st.d[1]);
@@ -168,7 +169,7 @@ __global__ void __launch_bounds__(256) adj_point_kernel(AdjPointArgs a) {
         const uint32_t mi = own & kMatMask;
         for (int f = 0; f < 6; f++) {
             if ((own >> (kFmSurfShift + f)) & 1u) continue;
-            const uint32_t mj = own & kMixed ? ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz)) & kMatMask : mi;
+            const uint32_t mj = kMixed ? cd[f] & kMatMask : mi;
             const double w = dcoef_dA(a.mats, mi, mj, static_cast<uint32_t>(a.mat)) * a.ih2[f >> 1];
             exd0 += w * (nv[f][0] - mgx);
             exd1 += w * (nv[f][1] - mgy);
@@ -334,9 +335,9 @@ struct AdjCombineArgs {
     double g;                      // loss gradient per probe cell (mode 1)
 };
 
-// As adj_point_kernel; a neighbour's constants are read only when it is of
+// As adj_point_kernel; a neighbour's constants are read only where it can be of
 // another material.  128x128x32: 24.4 -> 22.4 us.
-template <class I>
+template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
@@ -355,7 +356,8 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     const double hb[3] = {ldd(a.hbar[0], id), ldd(a.hbar[1], id), ldd(a.hbar[2], id)};
     double nv[6][3];
     const I nx = static_cast<I>(a.nx);
-    gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, nv);
+    uint32_t cd[6];
+    gather6_lanes_load<kMixed, I>(sp, a.code, x, y, z, nx, ny, nz, nv, cd);
     double mb[3], da[3], lam[3], acc[3];
     const bool dem = a.dadj[0] != nullptr, step = a.mode != 0, later = step && a.mode != 4;
     for (int c = 0; c < 3; c++) {
@@ -364,7 +366,7 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
         lam[c] = step ? ldd(a.lam[c], id) : 0.;
         acc[c] = later ? ldd(a.acc[c], id) : 0.;
     }
-    gather6_lanes_shift<I>(z, nz, hb, nv);
+    gather6_lanes_shift<kMixed, I>(z, nz, hb, own, nv, cd);
     if (!(own & kIsFM)) {
         if (a.mode == 0) for (int c = 0; c < 3; c++) std_(a.ybar[c], id, 0.);
         return;
@@ -380,8 +382,8 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
             if ((own >> (kFmSurfShift + f)) & 1u) continue;   // else the neighbour is FM
             // the neighbour's own constants; its record is read only when it can be another
             double dn = M.dmi_neg, dp = M.dmi_pos;
-            if (own & kMixed) {
-                GMat& Mn = mat_of(a.mats, ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz)));
+            if (kMixed) {
+                GMat& Mn = mat_of(a.mats, cd[f]);
                 dn = Mn.dmi_neg; dp = Mn.dmi_pos;
             }
             const double w = ((f & 1) ? -1. : 1.) * ih[f >> 1];
@@ -392,13 +394,12 @@ __global__ void __launch_bounds__(256) adj_combine_kernel(AdjCombineArgs a) {
     }
     for (int f = 0; f < 6; f++) {
         double e = M.exch;   // across a surface too: the value is not used there
-        if ((own & kMixed) && !((own >> (kFmSurfShift + f)) & 1u))
-            e = mat_of(a.mats, ldu(a.code, face_nb<I>(f, x, y, z, nx, ny, nz))).exch;
+        if (kMixed && !((own >> (kFmSurfShift + f)) & 1u)) e = mat_of(a.mats, cd[f]).exch;
         for (int c = 0; c < 3; c++) nv[f][c] = e * nv[f][c];
     }
     const double eh[3] = {M.exch * hb[0], M.exch * hb[1], M.exch * hb[2]};
-    const Stencil st = magnet_stencil<false, I>(eh, nv, a.code, (GMat*)a.mats, own, kFmSurfShift, -1, x, y, z, nx, ny, nz,
-                                                a.idx, a.idy, a.idz, M.Aex, M.Aex_self, 0.);
+    const Stencil st = magnet_stencil<false, kMixed>(eh, nv, cd, (GMat*)a.mats, own, kFmSurfShift, -1, a.idx, a.idy,
+                                                     a.idz, M.Aex, M.Aex_self, 0.);
     const bool probe = x >= static_cast<I>(a.lo[0]) && x <= static_cast<I>(a.hi[0]) && y >= static_cast<I>(a.lo[1]) &&
                        y <= static_cast<I>(a.hi[1]) && z >= static_cast<I>(a.lo[2]) && z <= static_cast<I>(a.hi[2]);
     for (int c = 0; c < 3; c++) {
@@ -580,8 +581,10 @@ gf_status stage_vjp(gf_ctx* c, int material, int stage, double* const* y, double
     if (!h) for (int i = 0; i < 3; i++) p.hd[i] = c->hstat[i];   // uploaded static field, no convolution
     p.drive_s = sa.drive_s;
     p.galpha = gpar; p.gaex = gpar + c->n; p.gb1 = gpar + 2 * c->n;
-    if (narrow(c->n)) hipLaunchKernelGGL(adj_point_kernel<uint32_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, p);
-    else hipLaunchKernelGGL(adj_point_kernel<int64_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, p);
+    const auto point = !narrow(c->n)   ? adj_point_kernel<int64_t, true>
+                       : c->fm_mixed ? adj_point_kernel<uint32_t, true>
+                                     : adj_point_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(point, dim3(blocks256(c->n)), dim3(256), 0, c->stream, p);
     gf_status st = hip_check(c, hipGetLastError(), "adjoint point kernel");
     if (st) return st;
     if (h && dadj) return demag_adjoint(c, hbar, dadj);
@@ -603,8 +606,10 @@ gf_status combine(gf_ctx* c, int mode, double* const* mbar, double* const* hbar,
     a.div = make_cell_div(c->ny, c->nz);
     a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     a.mode = mode; a.g = g;
-    if (narrow(c->n)) hipLaunchKernelGGL(adj_combine_kernel<uint32_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, a);
-    else hipLaunchKernelGGL(adj_combine_kernel<int64_t>, dim3(blocks256(c->n)), dim3(256), 0, c->stream, a);
+    const auto join = !narrow(c->n)   ? adj_combine_kernel<int64_t, true>
+                      : c->fm_mixed ? adj_combine_kernel<uint32_t, true>
+                                    : adj_combine_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(join, dim3(blocks256(c->n)), dim3(256), 0, c->stream, a);
     return hip_check(c, hipGetLastError(), "adjoint combine kernel");
 }
 

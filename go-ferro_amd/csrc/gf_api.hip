@@ -126,39 +126,6 @@ void build_surface_bits(gf_ctx* c, bool (*kind)(const gf_ctx*, int64_t), int shi
             }
 }
 
-// The codes as the device holds them, with kMixed set; left empty where they
-// are the host's (one magnetic material has no such cell).
-void device_codes(const gf_ctx* c, std::vector<uint32_t>& out) {
-    uint32_t seen = 0;
-    bool several = false;
-    for (size_t i = 0; i < c->host_code.size() && !several; i++) {
-        if (!(c->host_code[i] & (kIsFM | kIsAFM))) continue;
-        const uint32_t t = c->host_code[i] & kMatMask;
-        several = seen && t != seen;
-        seen = t;
-    }
-    if (!several) return;
-    out = c->host_code;
-    const int64_t n3[3] = {c->nx, c->ny, c->nz}, step[3] = {c->ny * c->nz, c->nz, 1};
-    int64_t q[3];
-    for (q[0] = 0; q[0] < n3[0]; q[0]++)
-        for (q[1] = 0; q[1] < n3[1]; q[1]++)
-            for (q[2] = 0; q[2] < n3[2]; q[2]++) {
-                const int64_t id = q[0] * step[0] + q[1] * step[1] + q[2];
-                const uint32_t own = c->host_code[static_cast<size_t>(id)];
-                if (!(own & (kIsFM | kIsAFM))) continue;
-                for (int f = 0; f < 6; f++) {
-                    const bool fm = (own & kIsFM) && !((own >> (kFmSurfShift + f)) & 1u);
-                    const bool afm = (own & kIsAFM) && !((own >> (kAfmSurfShift + f)) & 1u);
-                    if (!fm && !afm) continue;
-                    const int ax = f >> 1;
-                    const int64_t to = f & 1 ? (q[ax] == n3[ax] - 1 ? 0 : q[ax] + 1) : (q[ax] == 0 ? n3[ax] - 1 : q[ax] - 1);
-                    const uint32_t nb = c->host_code[static_cast<size_t>(id + (to - q[ax]) * step[ax])];
-                    if ((nb ^ own) & kMatMask) out[static_cast<size_t>(id)] |= kMixed;
-                }
-            }
-}
-
 DevMaterial make_dev_material(const gf_material& m, double dt) {
     DevMaterial d{};
     d.is_fm = m.if_FM ? 1 : 0;
@@ -870,7 +837,6 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
         return GF_ERR_ALLOC;
     }
     gf_status st = GF_OK;
-    std::vector<uint32_t> mixed;   // the device's codes where they differ from the host's
     try {
         c->nx = d->nx; c->ny = d->ny; c->nz = d->nz; c->n = d->nx * d->ny * d->nz;
         c->dx = d->dx; c->dy = d->dy; c->dz = d->dz;
@@ -895,6 +861,7 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
             c->prescribe_e.assign(d->prescribe_Eext, d->prescribe_Eext + 4 * d->n_prescribe_Eext);
         c->host_mats.assign(d->materials, d->materials + d->n_materials);
         c->host_code.resize(static_cast<size_t>(c->n));
+        uint32_t fm = 0, afm = 0;   // the last cell's material of each kind
         for (int64_t i = 0; i < c->n; i++) {
             const uint32_t t = d->material_cell[i];
             if (t > static_cast<uint32_t>(d->n_materials)) {
@@ -904,8 +871,18 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
                 return GF_ERR_ARG;
             }
             uint32_t code = t;
-            if (t && d->materials[t - 1].if_FM) { code |= kIsFM; c->nfm++; }
-            if (t && d->materials[t - 1].if_AFM) { code |= kIsAFM; c->nafm++; }
+            if (t && d->materials[t - 1].if_FM) {
+                code |= kIsFM;
+                c->nfm++;
+                c->fm_mixed = c->fm_mixed || (fm && fm != t);
+                fm = t;
+            }
+            if (t && d->materials[t - 1].if_AFM) {
+                code |= kIsAFM;
+                c->nafm++;
+                c->afm_mixed = c->afm_mixed || (afm && afm != t);
+                afm = t;
+            }
             if (t && d->materials[t - 1].if_FE) { code |= kIsFE; c->nfe++; }
             c->host_code[static_cast<size_t>(i)] = code;
         }
@@ -917,7 +894,6 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
         if (c->any_fe) build_surface_bits(c, is_fe, kFeSurfShift);
         if (c->any_fm) build_surface_bits(c, is_fm, kFmSurfShift);
         if (c->any_afm) build_surface_bits(c, is_afm, kAfmSurfShift);
-        device_codes(c, mixed);
         if (c->flags & GF_FLAG_EMDYNAMIC) {
             const std::string why = em_unsupported(c, d);
             if (!why.empty()) {
@@ -944,8 +920,8 @@ gf_status gf_create(const gf_desc* d, gf_ctx** out) {
     if (!st) st = hip_check(c, hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking), "hipStreamCreate");
     if (!st) st = hip_check(c, hipMalloc(&c->d_code, sizeof(uint32_t) * c->n), "hipMalloc code");
     if (!st)
-        st = hip_check(c, hipMemcpy(c->d_code, (mixed.empty() ? c->host_code : mixed).data(), sizeof(uint32_t) * c->n,
-                                    hipMemcpyHostToDevice), "copy code");
+        st = hip_check(c, hipMemcpy(c->d_code, c->host_code.data(), sizeof(uint32_t) * c->n, hipMemcpyHostToDevice),
+                       "copy code");
     if (!st && c->any_fm && c->nfm < c->n && c->n <= INT64_C(0xffffffff)) {
         // the FM cells in index order: the unfused FM stage runs over them
         // alone (material kinds cannot change after set-up)
@@ -1449,6 +1425,7 @@ StageArgs fm_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
     }
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
     a.div = make_cell_div(c->ny, c->nz);
+    a.mixed = c->fm_mixed;
     a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
     std::memcpy(a.Tc2g, c->Tc2g, sizeof(a.Tc2g));
@@ -1502,6 +1479,7 @@ AfmStageArgs afm_stage_args(gf_ctx* c, int stage, int in_sel, int out_sel) {
     }
     a.nx = c->nx; a.ny = c->ny; a.nz = c->nz;
     a.div = make_cell_div(c->ny, c->nz);
+    a.mixed = c->afm_mixed;
     a.idx = 1. / c->dx; a.idy = 1. / c->dy; a.idz = 1. / c->dz;
     std::memcpy(a.Tg2c, c->Tg2c, sizeof(a.Tg2c));
     std::memcpy(a.Tc2g, c->Tc2g, sizeof(a.Tc2g));

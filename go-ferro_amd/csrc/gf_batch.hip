@@ -40,6 +40,7 @@ struct gf_batch {
     std::vector<BatchClock> clk;
 
     bool any_fm = false, any_afm = false, fm_narrow = true, afm_narrow = true;
+    bool fm_mixed = false, afm_mixed = false;
     int64_t fm_cells = 0, afm_cells = 0;
     uint32_t* d_fm_item = nullptr;   // workgroup slot -> instance
     uint32_t* d_fm_block0 = nullptr; // instance -> first slot
@@ -165,12 +166,12 @@ hipError_t launch_stage(gf_batch* b, int stage) {
     hipError_t e = hipSuccess;
     if (b->any_fm && b->fm_total) {
         const BatchLaunch L{b->d_fm_item, b->d_fm_block0, b->fm_total, grid_for(b->fm_total, b->grid_cap),
-                            static_cast<unsigned>(b->threads), b->cpt, b->fm_narrow};
+                            static_cast<unsigned>(b->threads), b->cpt, b->fm_narrow, b->fm_mixed};
         e = launch_mag_batch(b->d_fm, L, stage, b->stream);
     }
     if (e == hipSuccess && b->any_afm && b->afm_total) {
         const BatchLaunch L{b->d_afm_item, b->d_afm_block0, b->afm_total, grid_for(b->afm_total, b->grid_cap),
-                            static_cast<unsigned>(b->threads), b->cpt, b->afm_narrow};
+                            static_cast<unsigned>(b->threads), b->cpt, b->afm_narrow, b->afm_mixed};
         e = launch_afm_batch(b->d_afm, L, stage, b->stream);
     }
     return e;
@@ -279,11 +280,13 @@ gf_status gf_batch_create(gf_ctx* const* ctxs, int count, gf_batch** out) {
             b->any_fm = true;
             b->fm_cells += c->n;
             if (!narrow(c->n)) b->fm_narrow = false;
+            if (c->fm_mixed) b->fm_mixed = true;
         }
         if (c->any_afm) {
             b->any_afm = true;
             b->afm_cells += c->n;
             if (!narrow(c->n)) b->afm_narrow = false;
+            if (c->afm_mixed) b->afm_mixed = true;
         }
     }
     b->clk.resize(static_cast<size_t>(count));

@@ -571,6 +571,7 @@ __global__ void __launch_bounds__(kGroup) el_force_kernel(ElStageArgs a) {
 // cells are not FM) come first: their chain is the longer one.  On 70k cells
 // (45x38x41) each launch is mostly latency, and the magnet's 7.8 us hide in
 // the force's: 60 steps 7.66 -> 6.34 ms; 128x128x64: 45.5 -> 43.7 ms.
+template <bool kMixed>
 __global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, StageArgs m, const uint32_t* ids,
                                                               uint32_t count, unsigned mag_groups) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
@@ -580,8 +581,8 @@ __global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, Sta
     }
     const uint32_t t = blockIdx.x * kGroup + threadIdx.x;
     if (t >= count) return;
-    if (ids) fm_point<uint32_t>(m, ldu(ids, t));
-    else fm_point<uint32_t, true>(m, t);
+    if (ids) fm_point<uint32_t, false, kMixed>(m, ldu(ids, t));
+    else fm_point<uint32_t, true, kMixed>(m, t);
 }
 
 // -------------------------------------------------------------- boundary
@@ -669,11 +670,12 @@ hipError_t launch_el_force(const ElStageArgs& a, hipStream_t s) {
 hipError_t launch_el_force_mag(const ElStageArgs& a, const StageArgs& m, const uint32_t* ids, int64_t count,
                                hipStream_t s) {
     const size_t lds = el_lds(a);
-    const hipError_t e = allow_lds(reinterpret_cast<const void*>(el_force_mag_kernel), lds);
+    const auto both = m.mixed ? el_force_mag_kernel<true> : el_force_mag_kernel<false>;
+    const hipError_t e = allow_lds(reinterpret_cast<const void*>(both), lds);
     if (e != hipSuccess) return e;
     const unsigned mg = blocks_for(count);
-    hipLaunchKernelGGL(el_force_mag_kernel, dim3(mg + blocks_for(a.f.nx * a.f.ny * a.f.nz)), dim3(kGroup), lds, s, a, m,
-                       ids, static_cast<uint32_t>(count), mg);
+    hipLaunchKernelGGL(both, dim3(mg + blocks_for(a.f.nx * a.f.ny * a.f.nz)), dim3(kGroup), lds, s, a, m, ids,
+                       static_cast<uint32_t>(count), mg);
     return hipGetLastError();
 }
 

@@ -18,28 +18,35 @@ namespace {
 // or a wave edge, where they are loaded.  A lane next to one without a cell
 // is at a column end.  Two parts: the loads, and after the cell's other
 // loads have been issued, the lane shifts of its own store c.
-template <class I>
-__device__ __forceinline__ void gather6_lanes_load(const P3 s3, I x, I y, I z, I nx, I ny, I nz, double (&v)[6][3]) {
-#pragma unroll
-    for (int f = 0; f < 4; f++) {
+template <bool kMixed, class I>
+__device__ __forceinline__ void gather6_lanes_load(const P3 s3, const uint32_t* code, I x, I y, I z, I nx, I ny, I nz,
+                                                   double (&v)[6][3], uint32_t (&cd)[6]) {
+    auto face = [&](int f) {
         const I nb = face_nb<I>(f, x, y, z, nx, ny, nz);
         for (int q = 0; q < 3; q++) v[f][q] = ldd(s3.p[q], nb);
-    }
+        if (kMixed) cd[f] = ldu(code, nb);
+    };
+#pragma unroll
+    for (int f = 0; f < 4; f++) face(f);
     const int lane = static_cast<int>(threadIdx.x & 63u);
-    if (lane == 0 || z == 0)
-        for (int q = 0; q < 3; q++) v[4][q] = ldd(s3.p[q], face_nb<I>(4, x, y, z, nx, ny, nz));
-    if (lane == 63 || z == nz - 1)
-        for (int q = 0; q < 3; q++) v[5][q] = ldd(s3.p[q], face_nb<I>(5, x, y, z, nx, ny, nz));
+    if (lane == 0 || z == 0) face(4);
+    if (lane == 63 || z == nz - 1) face(5);
 }
 
-template <class I>
-__device__ __forceinline__ void gather6_lanes_shift(I z, I nz, const double (&c)[3], double (&v)[6][3]) {
+template <bool kMixed, class I>
+__device__ __forceinline__ void gather6_lanes_shift(I z, I nz, const double (&c)[3], uint32_t own, double (&v)[6][3],
+                                                    uint32_t (&cd)[6]) {
     const int lane = static_cast<int>(threadIdx.x & 63u);
     const bool gm = lane == 0 || z == 0, gp = lane == 63 || z == nz - 1;
     for (int q = 0; q < 3; q++) {
         const double dn = lane_up(c[q]), up = lane_down(c[q]);
         if (!gm) v[4][q] = dn;
         if (!gp) v[5][q] = up;
+    }
+    if (kMixed) {
+        const uint32_t dn = lane_up(own), up = lane_down(own);
+        if (!gm) cd[4] = dn;
+        if (!gp) cd[5] = up;
     }
 }
 
@@ -51,24 +58,25 @@ struct FmIn {
     uint32_t own;
     double c[3];        // stage store at the cell
     double v[6][3];     // stage store at the six face neighbours (gather6)
+    uint32_t cd[6];     // their codes, where they are read
     double m[3];        // m at the start of the step
     double acc[3];      // RK accumulator (read at stages 2-4)
 };
 
 // kLanes: the launch's lanes hold consecutive cells (see gather6_lanes).
-template <class I, bool kLanes = false>
+template <class I, bool kLanes, bool kMixed>
 __device__ __forceinline__ void fm_load(const StageArgs& a, I id, I x, I y, I z, FmIn& in) {
     in.own = ldu(a.code, id);
     const P3 sp = {{a.store[0], a.store[1], a.store[2]}};
     for (int c = 0; c < 3; c++) in.c[c] = ldd(a.store[c], id);
     const I nx = static_cast<I>(a.nx), ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
-    if (kLanes) gather6_lanes_load<I>(sp, x, y, z, nx, ny, nz, in.v);
-    else gather6<I>(sp, x, y, z, nx, ny, nz, in.v);
+    if (kLanes) gather6_lanes_load<kMixed, I>(sp, a.code, x, y, z, nx, ny, nz, in.v, in.cd);
+    else gather6<kMixed, I>(sp, a.code, x, y, z, nx, ny, nz, in.v, in.cd);
     // at stage 1 the stage store is m itself: read it once
     const bool same = a.base[0] == a.store[0] && a.base[1] == a.store[1] && a.base[2] == a.store[2];
     for (int c = 0; c < 3; c++) in.m[c] = same ? in.c[c] : ldd_nt(a.base[c], id);
     for (int c = 0; c < 3; c++) in.acc[c] = a.stage > 1 ? ldd_nt(a.acc[c], id) : 0.;
-    if (kLanes) gather6_lanes_shift<I>(z, nz, in.c, in.v);
+    if (kLanes) gather6_lanes_shift<kMixed, I>(z, nz, in.c, in.own, in.v, in.cd);
 }
 
 // RK update of one component (see the file comment) from its preloaded m
@@ -103,19 +111,18 @@ __device__ __forceinline__ double rk_store(int stage, I id, int c, double k, dou
 // prescribed bottom layer) for contexts that have none of them: their
 // pointers and the rotation matrices then occupy no scalar registers
 // across the cell loop.  mats is the material table, in global memory
-// (GMat) or a workgroup's LDS copy (LMat).  (x, y, z) are the cell's.
-template <bool kLean, class I, class MT>
-__device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn& in, I id, I x, I y, I z, double hs0,
-                                        double hs1, double hs2, double& n0, double& n1, double& n2) {
+// (GMat) or a workgroup's LDS copy (LMat).  z is the cell's.
+template <bool kLean, bool kMixed, class I, class MT>
+__device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn& in, I id, I z, double hs0, double hs1,
+                                        double hs2, double& n0, double& n1, double& n2) {
     MT& M = mats[(in.own & kMatMask) - 1];
 
     const double mgx = in.c[0], mgy = in.c[1], mgz = in.c[2];
     double mx = mgx, my = mgy, mz = mgz;
     if (!kLean && a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
 
-    const Stencil st = magnet_stencil<true, I>(in.c, in.v, a.code, mats, in.own, kFmSurfShift, -1, x, y, z,
-                                               static_cast<I>(a.nx), static_cast<I>(a.ny), static_cast<I>(a.nz), a.idx,
-                                               a.idy, a.idz, M.Aex, M.Aex_self, M.dmi_slope);
+    const Stencil st = magnet_stencil<true, kMixed>(in.c, in.v, in.cd, mats, in.own, kFmSurfShift, -1, a.idx, a.idy,
+                                                    a.idz, M.Aex, M.Aex_self, M.dmi_slope);
 
     // magnetocrystalline anisotropy (magnetic_solver.cpp:124-141)
     double hac0 = 0., hac1 = 0., hac2 = 0.;
@@ -181,20 +188,20 @@ __device__ __forceinline__ void fm_cell(const StageArgs& a, MT* mats, const FmIn
 
 // One FM cell of the unfused stage: coordinates from the linear index,
 // magnetostatic field from Hstat.
-template <class I, bool kLanes = false>
+template <class I, bool kLanes, bool kMixed>
 __device__ __forceinline__ void fm_point(const StageArgs& a, I id) {
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
     I x, y, z;
     cell_xyz(a.div, id, ny, nz, x, y, z);
     FmIn in;
-    fm_load<I, kLanes>(a, id, x, y, z, in);
+    fm_load<I, kLanes, kMixed>(a, id, x, y, z, in);
     // a null Hstat is zero (no statics, nothing uploaded)
     const bool hs = a.hstat[0] != nullptr;
     const double hs0 = hs ? ldd(a.hstat[0], id) : 0., hs1 = hs ? ldd(a.hstat[1], id) : 0.;
     const double hs2 = hs ? ldd(a.hstat[2], id) : 0.;
     if (!(in.own & kIsFM)) return;
     double n0, n1, n2;
-    fm_cell<false, I>(a, (GMat*)a.mats, in, id, x, y, z, hs0, hs1, hs2, n0, n1, n2);
+    fm_cell<false, kMixed, I>(a, (GMat*)a.mats, in, id, z, hs0, hs1, hs2, n0, n1, n2);
 }
 
 }  // namespace

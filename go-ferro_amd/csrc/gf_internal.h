@@ -38,12 +38,6 @@ constexpr uint32_t kIsFE = 1u << 10;
 constexpr int kFmSurfShift = 11;    // 6 bits: xb, xf, yb, yf, zb, zf
 constexpr int kAfmSurfShift = 17;   // 6 bits, same order
 constexpr int kFeSurfShift = 23;    // 6 bits, same order (FE_surf*, ferroelectric_initialize.cpp:74-308)
-// On the device only: a face of a magnet cell that is not a surface has a
-// neighbour of another material, so that its exchange coefficient is not the
-// material's own.  Elsewhere the stages read no neighbour's code.
-// Four loads and two lane shifts less a cell: 64x64x32 antiferromagnet, 100
-// steps 4.11 -> 4.04 ms; the fused stage of 256x256x128 338 -> 333 us.
-constexpr uint32_t kMixed = 1u << 29;
 enum Face { kXB = 0, kXF = 1, kYB = 2, kYF = 3, kZB = 4, kZF = 5 };
 
 // Per-material constants as the stage kernels need them.  Every entry is
@@ -501,6 +495,7 @@ struct StageArgs {
     int64_t nx, ny, nz;
     CellDiv div;
     double idx, idy, idz;       // 1/dx, 1/dy, 1/dz
+    int32_t mixed;              // more than one ferromagnet material: the neighbours' codes are read
     double hext[3];
     double drive_s;             // sin(2 pi f t) of the shaped drive at the stage time
     double Tg2c[3][3];
@@ -532,6 +527,7 @@ struct AfmStageArgs {
     int64_t nx, ny, nz;
     CellDiv div;
     double idx, idy, idz;       // 1/dx, 1/dy, 1/dz
+    int32_t mixed;              // as StageArgs, of the antiferromagnets
     double hext[3];
     double Tg2c[3][3];
     double Tc2g[3][3];
@@ -548,6 +544,7 @@ struct BatchLaunch {
     unsigned grid, threads;
     int cpt;
     bool narrow;
+    bool mixed;   // an instance has several materials of the kind
 };
 
 struct AdjState;
@@ -690,6 +687,7 @@ struct gf_ctx {
     std::vector<gf_material> host_mats;
     std::vector<uint32_t> host_code;
     bool any_fm = false, any_afm = false, any_fe = false;
+    bool fm_mixed = false, afm_mixed = false;   // cells of several materials of the kind
     int64_t nfm = 0, nafm = 0, nfe = 0;
     bool has_hnu = false;
     bool has_e0t0 = false;          // the static eigenstrain was written: the elastic stage subtracts it

@@ -30,22 +30,24 @@ constexpr int kSetupChunk = 4;
 static_assert(kLeanMats * sizeof(DevMaterial) / sizeof(double) <= kMatWordsPerThread * 256,
               "the lean stage's material records must fit the set-up loads of 256 threads");
 
-template <class I>
-__global__ void __launch_bounds__(256) mag_stage_kernel(StageArgs a) {
+template <class I, bool kMixed>
+__global__ void __launch_bounds__(256) mag_stage_kernel(StageArgs) {
+    const StageArgs& a = first_arg<StageArgs>();
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
-    fm_point<I, true>(a, id);
+    fm_point<I, true, kMixed>(a, id);
 }
 
 // The same over a list of the FM cells: a layered magnet fills whole
 // waves instead of loading the inputs of every non-magnetic cell first.  The
 // list is of 32-bit indices on every grid that has one (up to 2^32 cells).
-template <class I>
-__global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs a, const uint32_t* ids, I count) {
+template <class I, bool kMixed>
+__global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs, const uint32_t* ids, I count) {
+    const StageArgs& a = first_arg<StageArgs>();
     const I t = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (t >= count) return;
-    fm_point<I>(a, static_cast<I>(ldu(ids, t)));
+    fm_point<I, false, kMixed>(a, static_cast<I>(ldu(ids, t)));
 }
 
 // The FM stage fused with the z transforms of the FFT magnetostatics, for
@@ -64,7 +66,7 @@ __global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs a, const 
 // Workgroups are ordered so that each XCD takes a contiguous range of x
 // planes, keeping stencil neighbours in its L2.  The lean form also copies
 // the material records into LDS (at most kLeanMats of them).
-template <bool kHspec, bool kLean, class I>
+template <bool kHspec, bool kLean, bool kMixed, class I>
 __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, FusedZArgs f) {
     extern __shared__ double2 fsm[];
     const int nz = static_cast<int>(a.nz), ny = static_cast<int>(a.ny);
@@ -160,19 +162,17 @@ __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, Fused
         double* h2 = reinterpret_cast<double*>(cbuf + fpad(2 * pairs * nz + pos)) + part;
         const I id = (static_cast<I>(x) * static_cast<I>(ny) + static_cast<I>(y)) * static_cast<I>(nz) + static_cast<I>(k);
         FmIn in;
-        fm_load<I, true>(a, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), in);
+        fm_load<I, true, kMixed>(a, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), in);
         double mx = 0., my = 0., mz = 0.;
         if (in.own & kIsFM) {
             double n0, n1, n2;
             double Ms;
             if (kLean) {
                 LMat* tab = (LMat*)ltab;
-                fm_cell<kLean, I>(a, tab, in, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), *h0, *h1, *h2, n0,
-                                  n1, n2);
+                fm_cell<kLean, kMixed, I>(a, tab, in, id, static_cast<I>(k), *h0, *h1, *h2, n0, n1, n2);
                 Ms = tab[(in.own & kMatMask) - 1].Ms;
             } else {
-                fm_cell<kLean, I>(a, (GMat*)a.mats, in, id, static_cast<I>(x), static_cast<I>(y), static_cast<I>(k), *h0, *h1,
-                                  *h2, n0, n1, n2);
+                fm_cell<kLean, kMixed, I>(a, (GMat*)a.mats, in, id, static_cast<I>(k), *h0, *h1, *h2, n0, n1, n2);
                 Ms = mat_of(a.mats, in.own).Ms;
             }
             mx = Ms * n0; my = Ms * n1; mz = Ms * n2;
@@ -208,7 +208,7 @@ __global__ void __launch_bounds__(256) mag_stage_fused_kernel(StageArgs a, Fused
 // input of the sublattice is loaded before the cell's code is known (all
 // indices are in bounds), as for the FM cell, so one memory round trip
 // feeds the cell.
-template <class I, bool kLanes = false>
+template <class I, bool kLanes, bool kMixed>
 __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) {
     const I ny = static_cast<I>(a.ny), nz = static_cast<I>(a.nz);
     I x, y, z;
@@ -224,8 +224,9 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
     const double mgx = c3[0], mgy = c3[1], mgz = c3[2];
     const I nx = static_cast<I>(a.nx);
     double v[6][3];
-    if (kLanes) gather6_lanes_load<I>(st, x, y, z, nx, ny, nz, v);
-    else gather6<I>(st, x, y, z, nx, ny, nz, v);
+    uint32_t cd[6];
+    if (kLanes) gather6_lanes_load<kMixed, I>(st, a.code, x, y, z, nx, ny, nz, v, cd);
+    else gather6<kMixed, I>(st, a.code, x, y, z, nx, ny, nz, v, cd);
     const double o0 = ldd(other.p[0], id), o1 = ldd(other.p[1], id), o2 = ldd(other.p[2], id);
     // a null Hstat is zero (no statics, nothing uploaded)
     const bool hs = a.hstat[0] != nullptr;
@@ -238,13 +239,13 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
     mb[1] = same ? mgy : ldd_nt(base[1], id);
     mb[2] = same ? mgz : ldd_nt(base[2], id);
     for (int c = 0; c < 3; c++) ac[c] = a.stage > 1 ? ldd_nt(acc[c], id) : 0.;
-    if (kLanes) gather6_lanes_shift<I>(z, nz, c3, v);
+    if (kLanes) gather6_lanes_shift<kMixed, I>(z, nz, c3, own, v, cd);
     if (!(own & kIsAFM)) return;
     GMat& M = mat_of(a.mats, own);
     double mx = mgx, my = mgy, mz = mgz;
     if (a.rotate) rot(a.Tg2c, mgx, mgy, mgz, mx, my, mz);
-    const Stencil s = magnet_stencil<false, I>(c3, v, a.code, (GMat*)a.mats, own, kAfmSurfShift, sub, x, y, z, nx, ny,
-                                               nz, a.idx, a.idy, a.idz, M.aAex[sub], M.aAex_self[sub], 0.);
+    const Stencil s = magnet_stencil<false, kMixed>(c3, v, cd, (GMat*)a.mats, own, kAfmSurfShift, sub, a.idx, a.idy,
+                                                    a.idz, M.aAex[sub], M.aAex_self[sub], 0.);
     // uniaxial anisotropy 2K1 (u.m) u (magnetic_AFM_solver.cpp:148-154)
     const double udotm = mx * M.u[0] + my * M.u[1] + mz * M.u[2];
     const double hac0 = 2. * M.aK1n[sub] * udotm * M.u[0];
@@ -291,16 +292,18 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
 // (b / 8) % 2: the two sublattices of a cell block land on the same XCD
 // (workgroups are dealt to the 8 XCDs round-robin) one dispatch round
 // apart, so the second finds the shared reads (code, Hstat, the other
-// sublattice's store) in that XCD's L2.
-template <class I>
-__global__ void __launch_bounds__(256) afm_stage_kernel(AfmStageArgs a) {
+// sublattice's store) in that XCD's L2.  Over one material the by-value argument
+// is the faster one (64x64x32: 36.3 us a step, 37.9 through first_arg).
+template <class I, bool kMixed>
+__global__ void __launch_bounds__(256) afm_stage_kernel(AfmStageArgs byval) {
+    const AfmStageArgs& a = kMixed ? first_arg<AfmStageArgs>() : byval;
     const unsigned b = blockIdx.x;
     const unsigned blk = (b >> 4) * 8u + (b & 7u);
     const int sub = static_cast<int>((b >> 3) & 1u);
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blk) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
-    afm_point<I, true>(a, id, sub);
+    afm_point<I, true, kMixed>(a, id, sub);
 }
 
 // Batched stages: one launch covers every instance of a batch.  The stage
@@ -310,7 +313,7 @@ __global__ void __launch_bounds__(256) afm_stage_kernel(AfmStageArgs a) {
 // (b - L.block0[instance]) * L.cpt * blockDim.x, one cell per thread per
 // pass.  A grid smaller than L.total walks the slots with a stride of
 // gridDim.x.
-template <class I>
+template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) mag_batch_kernel(const StageArgs* __restrict__ items, BatchLaunch L, int stage) {
     for (uint32_t b = blockIdx.x; b < L.total; b += gridDim.x) {
         const uint32_t inst = L.item[b];
@@ -320,7 +323,7 @@ __global__ void __launch_bounds__(256) mag_batch_kernel(const StageArgs* __restr
         const I first = static_cast<I>(b - L.block0[inst]) * chunk + static_cast<I>(threadIdx.x);
         for (int j = 0; j < L.cpt; j++) {
             const I id = first + static_cast<I>(j) * static_cast<I>(blockDim.x);
-            if (id < n) fm_point<I, true>(a, id);
+            if (id < n) fm_point<I, true, kMixed>(a, id);
         }
     }
 }
@@ -329,7 +332,7 @@ __global__ void __launch_bounds__(256) mag_batch_kernel(const StageArgs* __restr
 // sublattice (w / 8) % 2, so that the two sublattices of a slot run on one
 // XCD one dispatch round apart (see afm_stage_kernel).
 // kOne: one work item per workgroup and one cell per thread (no loops).
-template <class I, bool kOne>
+template <class I, bool kOne, bool kMixed>
 __global__ void __launch_bounds__(256) afm_batch_kernel(const AfmStageArgs* __restrict__ items, BatchLaunch L,
                                                          int stage) {
     const uint32_t work = 2u * ((L.total + 7u) / 8u * 8u);
@@ -341,7 +344,7 @@ __global__ void __launch_bounds__(256) afm_batch_kernel(const AfmStageArgs* __re
         const AfmStageArgs& a = items[4 * inst + stage - 1];
         const I n = static_cast<I>(a.nx * a.ny * a.nz);
         const I id = static_cast<I>(b - L.block0[inst]) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
-        if (id < n) afm_point<I, true>(a, id, static_cast<int>((w >> 3) & 1u));
+        if (id < n) afm_point<I, true, kMixed>(a, id, static_cast<int>((w >> 3) & 1u));
         return;
     }
     for (uint32_t w = blockIdx.x; w < work; w += gridDim.x) {
@@ -355,7 +358,8 @@ __global__ void __launch_bounds__(256) afm_batch_kernel(const AfmStageArgs* __re
         const I first = static_cast<I>(b - L.block0[inst]) * chunk + static_cast<I>(threadIdx.x);
         for (int j = 0; j < L.cpt; j++) {
             const I id = first + static_cast<I>(j) * static_cast<I>(blockDim.x);
-            if (id < n) afm_point<I>(a, id, sub);   // lane gathers cost this loop a wave of occupancy
+            // lane gathers cost this loop a wave of occupancy
+            if (id < n) afm_point<I, false, kMixed>(a, id, sub);
         }
     }
 }
@@ -429,15 +433,18 @@ bool narrow(int64_t n) { return n < (int64_t{1} << 28); }
 hipError_t launch_mag_stage(const StageArgs& a, int64_t n, hipStream_t s, const uint32_t* ids, int64_t count) {
     if (ids) {
         const dim3 grid(static_cast<unsigned>((count + 255) / 256));
+        const auto list = a.mixed ? mag_stage_list_kernel<uint32_t, true> : mag_stage_list_kernel<uint32_t, false>;
         if (count > 0 && narrow(n))
-            hipLaunchKernelGGL(mag_stage_list_kernel<uint32_t>, grid, dim3(256), 0, s, a, ids, static_cast<uint32_t>(count));
+            hipLaunchKernelGGL(list, grid, dim3(256), 0, s, a, ids, static_cast<uint32_t>(count));
         else if (count > 0)
-            hipLaunchKernelGGL(mag_stage_list_kernel<int64_t>, grid, dim3(256), 0, s, a, ids, count);
+            hipLaunchKernelGGL((mag_stage_list_kernel<int64_t, true>), grid, dim3(256), 0, s, a, ids, count);
         return hipGetLastError();
     }
     const int64_t blocks = (n + 255) / 256;
-    if (narrow(n)) hipLaunchKernelGGL(mag_stage_kernel<uint32_t>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(mag_stage_kernel<int64_t>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a);
+    const auto stage = !narrow(n)  ? mag_stage_kernel<int64_t, true>
+                       : a.mixed ? mag_stage_kernel<uint32_t, true>
+                                 : mag_stage_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(stage, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
@@ -451,26 +458,36 @@ hipError_t launch_mag_stage_fused(const StageArgs& a, const FusedZArgs& f, bool 
     const unsigned groups = static_cast<unsigned>(a.nx * a.ny / f.P);
     const bool n32 = narrow(a.nx * a.ny * a.nz);
     const dim3 g(groups), t(256);
-    if (hspec && lean && n32) hipLaunchKernelGGL((mag_stage_fused_kernel<true, true, uint32_t>), g, t, lds, s, a, f);
-    else if (hspec && lean) hipLaunchKernelGGL((mag_stage_fused_kernel<true, true, int64_t>), g, t, lds, s, a, f);
-    else if (hspec && n32) hipLaunchKernelGGL((mag_stage_fused_kernel<true, false, uint32_t>), g, t, lds, s, a, f);
-    else if (hspec) hipLaunchKernelGGL((mag_stage_fused_kernel<true, false, int64_t>), g, t, lds, s, a, f);
-    else if (n32) hipLaunchKernelGGL((mag_stage_fused_kernel<false, false, uint32_t>), g, t, lds, s, a, f);
-    else hipLaunchKernelGGL((mag_stage_fused_kernel<false, false, int64_t>), g, t, lds, s, a, f);
+    auto stage = mag_stage_fused_kernel<false, false, true, int64_t>;
+    if (n32 && a.mixed)
+        stage = !hspec ? mag_stage_fused_kernel<false, false, true, uint32_t>
+                : lean ? mag_stage_fused_kernel<true, true, true, uint32_t>
+                       : mag_stage_fused_kernel<true, false, true, uint32_t>;
+    else if (n32)
+        stage = !hspec ? mag_stage_fused_kernel<false, false, false, uint32_t>
+                : lean ? mag_stage_fused_kernel<true, true, false, uint32_t>
+                       : mag_stage_fused_kernel<true, false, false, uint32_t>;
+    else if (hspec)
+        stage = lean ? mag_stage_fused_kernel<true, true, true, int64_t> : mag_stage_fused_kernel<true, false, true, int64_t>;
+    hipLaunchKernelGGL(stage, g, t, lds, s, a, f);
     return hipGetLastError();
 }
 
 hipError_t launch_afm_stage(const AfmStageArgs& a, int64_t n, hipStream_t s) {
     const int64_t blocks = (n + 255) / 256;
     const dim3 grid(static_cast<unsigned>((blocks + 7) / 8 * 16));
-    if (narrow(n)) hipLaunchKernelGGL(afm_stage_kernel<uint32_t>, grid, dim3(256), 0, s, a);
-    else hipLaunchKernelGGL(afm_stage_kernel<int64_t>, grid, dim3(256), 0, s, a);
+    const auto stage = !narrow(n)  ? afm_stage_kernel<int64_t, true>
+                       : a.mixed ? afm_stage_kernel<uint32_t, true>
+                                 : afm_stage_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(stage, grid, dim3(256), 0, s, a);
     return hipGetLastError();
 }
 
 hipError_t launch_mag_batch(const StageArgs* items, const BatchLaunch& L, int stage, hipStream_t s) {
-    if (L.narrow) hipLaunchKernelGGL(mag_batch_kernel<uint32_t>, dim3(L.grid), dim3(L.threads), 0, s, items, L, stage);
-    else hipLaunchKernelGGL(mag_batch_kernel<int64_t>, dim3(L.grid), dim3(L.threads), 0, s, items, L, stage);
+    const auto batch = !L.narrow ? mag_batch_kernel<int64_t, true>
+                       : L.mixed ? mag_batch_kernel<uint32_t, true>
+                                 : mag_batch_kernel<uint32_t, false>;
+    hipLaunchKernelGGL(batch, dim3(L.grid), dim3(L.threads), 0, s, items, L, stage);
     return hipGetLastError();
 }
 
@@ -478,14 +495,12 @@ hipError_t launch_afm_batch(const AfmStageArgs* items, const BatchLaunch& L, int
     // L.grid counts slots; the grid covers both sublattices of each
     const unsigned grid = 2u * ((L.grid + 7u) / 8u * 8u);
     const bool one = L.cpt == 1 && L.grid == L.total;
-    if (L.narrow && one)
-        hipLaunchKernelGGL((afm_batch_kernel<uint32_t, true>), dim3(grid), dim3(L.threads), 0, s, items, L, stage);
+    auto batch = one ? afm_batch_kernel<int64_t, true, true> : afm_batch_kernel<int64_t, false, true>;
+    if (L.narrow && L.mixed)
+        batch = one ? afm_batch_kernel<uint32_t, true, true> : afm_batch_kernel<uint32_t, false, true>;
     else if (L.narrow)
-        hipLaunchKernelGGL((afm_batch_kernel<uint32_t, false>), dim3(grid), dim3(L.threads), 0, s, items, L, stage);
-    else if (one)
-        hipLaunchKernelGGL((afm_batch_kernel<int64_t, true>), dim3(grid), dim3(L.threads), 0, s, items, L, stage);
-    else
-        hipLaunchKernelGGL((afm_batch_kernel<int64_t, false>), dim3(grid), dim3(L.threads), 0, s, items, L, stage);
+        batch = one ? afm_batch_kernel<uint32_t, true, false> : afm_batch_kernel<uint32_t, false, false>;
+    hipLaunchKernelGGL(batch, dim3(grid), dim3(L.threads), 0, s, items, L, stage);
     return hipGetLastError();
 }
 

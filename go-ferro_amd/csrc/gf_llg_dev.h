@@ -64,6 +64,17 @@ __device__ __forceinline__ uint32_t ldu(const uint32_t* p, uint32_t i) {
     return *(GConstU*)((GConstC*)p + (i << 2));
 }
 
+// A kernel's first argument where the launch put it.  Its fields then are
+// scalar loads where they are used; a by-value struct of the size of a stage's is
+// loaded at entry and its fields are kept in lanes of vector registers (28 to 84
+// scalar registers spilled in the magnet stages, each read back by a
+// v_readlane): ferromagnet 30x40x50 without magnetostatics 22.3 -> 20.6 us a step,
+// two stacked antiferromagnets of 128x128x32 cells 287 -> 275.
+template <class T>
+__device__ __forceinline__ const T& first_arg() {
+    return *(const T*)(const __attribute__((address_space(4))) T*)__builtin_amdgcn_kernarg_segment_ptr();
+}
+
 // Exchange-weighted neighbour differences of one store for one cell
 // (get_m_spatial_derivative_local, magnetic_solver.cpp:1639-1831).
 // Returns hx[3] = sum_faces Aij * d2m (before the 2/mu0/Ms factor) and the
@@ -91,27 +102,29 @@ __device__ __forceinline__ I face_nb(int f, I i, I j, I k, I nx, I ny, I nz) {
     }
 }
 
-// The store at the six face neighbours.  Loaded whether or not a face is a
-// surface, so that the loads do not wait for the cell's own code.
-template <class I>
-__device__ __forceinline__ void gather6(const P3 s3, I i, I j, I k, I nx, I ny, I nz, double (&v)[6][3]) {
+// The store at the six face neighbours, and for launches over several materials
+// of the magnet's kind (kMixed) their codes; the others need no code: four loads
+// and two lane shifts less a cell (64x64x32 antiferromagnet, 100 steps 4.11 ->
+// 4.04 ms; the fused stage of 256x256x128 338 -> 333 us).  Loaded whether or not a
+// face is a surface, so that the loads do not wait for the cell's own code: a
+// code read only where the neighbour is of another material waits for it in
+// every wave that holds such a cell (two stacked antiferromagnets of 96x80x12
+// cells 59.7 -> 64.9 us a step), and a branch around the codes inside one kernel
+// splits the group of loads they belong to (antiferromagnet 30x40x50 25 -> 27.5 us).
+template <bool kMixed, class I>
+__device__ __forceinline__ void gather6(const P3 s3, const uint32_t* code, I i, I j, I k, I nx, I ny, I nz,
+                                        double (&v)[6][3], uint32_t (&cd)[6]) {
 #pragma unroll
     for (int f = 0; f < 6; f++) {
         const I nb = face_nb<I>(f, i, j, k, nx, ny, nz);
         for (int q = 0; q < 3; q++) v[f][q] = ldd(s3.p[q], nb);
+        if (kMixed) cd[f] = ldu(code, nb);
     }
 }
 
-// Face coefficient between a cell of material `mat` (constant A, self mean
-// A_self) and a neighbour of code nc: the harmonic mean 2 A1 A2 / (A1 + A2)
-// of magnetic_initialize.cpp:381-524, A_self for the same material.
-template <class MP>
-__device__ __forceinline__ double face_coef(MP mats, uint32_t mat, uint32_t nc, int sub, double A, double A_self) {
-    const uint32_t nm = nc & kMatMask;
-    if (nm == mat) return A_self;
-    const double a2 = sub < 0 ? mats[nm - 1].Aex : mats[nm - 1].aAex[sub];
-    return 2. * A * a2 / (A + a2);
-}
+// Face coefficient between cells of two materials of constants a1 and a2:
+// their harmonic mean (magnetic_initialize.cpp:381-524).
+__device__ __forceinline__ double face_coef(double a1, double a2) { return 2. * a1 * a2 / (a1 + a2); }
 
 // The stencil of get_m_spatial_derivative_local from the cell's store
 // (c0, c1, c2) and its gathered neighbours; see gather6.  ix, iy and iz are
@@ -183,16 +196,27 @@ __device__ __forceinline__ Stencil stencil_core(double c0, double c1, double c2,
     return r;
 }
 
-// stencil_core with the coefficients of a cell at (x, y, z): the material's
-// own (A_self), and only where kMixed says so those of the neighbours' codes.
-template <bool kDmi, class I, class MP>
-__device__ __forceinline__ Stencil magnet_stencil(const double (&c)[3], const double (&v)[6][3], const uint32_t* code,
-                                                  MP mats, uint32_t own, int surf_shift, int sub, I x, I y, I z, I nx,
-                                                  I ny, I nz, double ix, double iy, double iz, double A, double A_self,
+// stencil_core with the material's own coefficient (A_self), or where several
+// materials of the magnet's kind are present (kMixed) those of the neighbours'
+// codes cd, which are read only then.
+template <bool kDmi, bool kMixed, class MP>
+__device__ __forceinline__ Stencil magnet_stencil(const double (&c)[3], const double (&v)[6][3],
+                                                  const uint32_t (&cd)[6], MP mats, uint32_t own, int surf_shift,
+                                                  int sub, double ix, double iy, double iz, double A, double A_self,
                                                   double slope) {
+    // the neighbours' constants together, not face by face (64x64x32 cells of two
+    // antiferromagnets at random 42.8 -> 41.9 us a step, 128x128x64 309 -> 291)
+    double a2[6];
+    const uint32_t mat = own & kMatMask;
+    if (kMixed) {
+#pragma unroll
+        for (int f = 0; f < 6; f++) {
+            const uint32_t m2 = ((own >> (surf_shift + f)) & 1u) ? mat : cd[f] & kMatMask;
+            a2[f] = sub < 0 ? mats[m2 - 1].Aex : mats[m2 - 1].aAex[sub];
+        }
+    }
     return stencil_core<kDmi>(c[0], c[1], c[2], v, own, surf_shift, ix, iy, iz, A, slope, [&](int f) {
-        if (!(own & kMixed)) return A_self;
-        return face_coef(mats, own & kMatMask, ldu(code, face_nb<I>(f, x, y, z, nx, ny, nz)), sub, A, A_self);
+        return !kMixed || (cd[f] & kMatMask) == mat ? A_self : face_coef(A, a2[f]);
     });
 }
 

@@ -46,12 +46,13 @@ int elastic_force() {
 }
 
 // The kernel a list of FM cells runs on a grid of n cells.
-const void* list_kernel(int64_t n, int64_t count) {
+const void* list_kernel(int64_t n, int64_t count, bool mixed = false) {
     static const uint32_t ids = 0;
     g_kernel = nullptr;
     gf::StageArgs a{};
     a.nx = a.ny = 1;
     a.nz = n;
+    a.mixed = mixed;
     return gf::launch_mag_stage(a, n, nullptr, &ids, count) == hipSuccess ? g_kernel : nullptr;
 }
 
@@ -65,6 +66,8 @@ int magnet_list() {
         return 1;
     }
     if (wide != list_kernel(2 * narrow, 2 * narrow - 1) || wide != list_kernel(16 * narrow - 1, 1)) return 1;
+    const void* two = list_kernel(narrow - 1, 1, true);   // several materials: the neighbours' codes are read
+    if (!two || two == small || two == wide || wide != list_kernel(narrow, 1, true)) return 1;
     return list_kernel(100, 0) || list_kernel(narrow, 0);   // no FM cell: no launch
 }
 

@@ -51,16 +51,13 @@ def create(cell, k):
 one = np.ones(shape, np.uint32)
 two = one.copy()
 two[20:] = 2
-counts = []
 for cell in (one, two):
     whole, seen = create(cell, -1)
     assert "failed (-4)" not in whole and seen >= 1, (whole, seen)
     for k in range(seen):
         text, _ = create(cell, k)
         assert "failed (-4)" in text and "allocation" in text, (k, text)
-    counts.append(seen)
-assert counts[1] == counts[0] + 1, counts   # two magnetic materials: the device's codes are a copy
-print("refused", counts)
+print("refused")
 """
 
 

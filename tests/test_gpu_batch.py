@@ -273,3 +273,23 @@ def test_batch_rejects_unbatchable_and_mid_step():
     batch.sync()
     with pytest.raises(GoFerroError, match="twice"):
         Batch([A[0], A[0]])
+
+
+@pytest.mark.parametrize("threads,cpt,cap", [(256, 1, 0), (64, 2, 5)])
+def test_batch_with_an_instance_of_two_antiferromagnets(threads, cpt, cap):
+    """One instance of several materials among instances of one: the launch
+    that serves them all, against the contexts' own steps."""
+    say("case batch, one instance of two AFM materials", threads, cpt, cap)
+    inst = [afm_instance((5, 6, 9), 41), afm_instance((4, 7, 66), 42), afm_instance((8, 8, 4), 43)]
+    prob, fields = inst[1]
+    prob.materials = [prob.materials[0], workloads.afm_block((8, 8, 4), alpha=3e-3, Aex=4e-12)[0].materials[0]]
+    prob.material_cell = np.random.default_rng(44).choice(np.array([1, 2], np.uint32), size=(4, 7, 66))
+    A, B = make(inst), make(inst)
+    batch = Batch(A)
+    batch.set_config(threads, cpt, cap)
+    batch.step(5)
+    batch.sync()
+    for c in B:
+        c.step(5)
+    compare(A, B, inst, "two materials")
+    batch.close()

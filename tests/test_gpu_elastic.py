@@ -212,6 +212,35 @@ def test_magnetoelastic_1000_steps():
     assert rel(g.download(FIELD_V), o.get(FIELD_V)) <= 1e-9
 
 
+@pytest.mark.parametrize("shape,layers", [((4, 5, 33), 7), ((3, 3, 65), 65)])
+def test_magnetoelastic_steps_of_two_magnets(shape, layers):
+    """gf_step with two magnet materials at random in the launch that also runs
+    the elastic force, over the list of magnet cells and over every cell."""
+    from oracle.oracle import Oracle
+    prob, m = magnetoelastic(shape=shape, layers=layers)
+    hard = Material.make()
+    for name, _ in Material._fields_:
+        setattr(hard, name, getattr(prob.materials[0], name))
+    hard.Aex, hard.Ms = 2 * hard.Aex, 1.5 * hard.Ms
+    prob.materials = list(prob.materials) + [hard]
+    cell = prob.material_cell
+    pick = np.random.default_rng(5).random(shape) < 0.5
+    cell[(cell == 1) & pick] = len(prob.materials)
+    u, v = random_uv(shape, 9)
+    say("case magnetoelastic, two magnets", shape, layers)
+    g, o = Context(prob), Oracle(prob)
+    for fid, val in ((FIELD_M, m), (FIELD_U, u), (FIELD_V, v)):
+        g.upload(fid, val)
+        o.set(fid, val)
+    g.step(3)
+    o.step(3)
+    assert np.abs(g.download(FIELD_M) - o.get(FIELD_M)).max() <= 1e-12
+    for fid in (FIELD_U, FIELD_V):
+        assert rel(g.download(fid), o.get(fid)) <= 1e-12, fid
+    g.close()
+    o.close()
+
+
 def fe_elastic(shape=(8, 8, 16), rotate=False):
     from goferro.workloads import pto_material
     T = rot() if rotate else None

@@ -144,9 +144,9 @@ def test_afm_stages_with_demag():
 @pytest.mark.parametrize("shape,periodic", [((6, 7, 5), (True, False, True)), ((3, 4, 70), (False, True, False)),
                                             ((1, 1, 9), (True, True, True))])
 def test_interfaces_of_magnets_of_both_kinds(shape, periodic):
-    """Two ferromagnets and two antiferromagnets side by side, with vacuum: only
-    cells at an interface read their neighbours' codes (harmonic-mean faces),
-    at walls, across periodic wraps and past a wave's length."""
+    """Two ferromagnets and two antiferromagnets side by side, with vacuum:
+    harmonic-mean faces by the neighbours' codes, at walls, across periodic
+    wraps and past a wave's length."""
     prob, m1, m2 = workloads.afm_block(shape)
     other = workloads.afm_block(shape, Aex=3e-12)[0].materials[0]
     fm, m = mixed_fm_problem(shape=shape, flags=0, rotate=False)
@@ -392,3 +392,30 @@ def test_set_material_matches_fresh_context():
     bad = Material.make(if_AFM=1)
     with pytest.raises(Exception, match="kind flags"):
         a.set_material(1, bad)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 65), (3, 5, 64), (2, 7, 9), (4, 4, 130)])
+@pytest.mark.parametrize("kind", ["afm", "afm_vacuum", "fm", "fm_list", "fm_fused"])
+def test_several_materials_of_a_kind(kind, shape):
+    """Two materials of a magnet's kind at random, so that every face takes the
+    mean of two constants or a cell's own: columns shorter than, of and longer
+    than a wave, over all cells, over the list of the magnet's cells and in the
+    stage fused with the z transforms."""
+    if kind == "fm_fused":
+        shape = shape[:2] + ({65: 64, 9: 8, 130: 128}.get(shape[2], shape[2]),)
+    rng = np.random.default_rng(shape[2])
+    cell = rng.choice(np.array([1, 2], np.uint32), size=shape)
+    if kind in ("afm_vacuum", "fm_list"):
+        cell[rng.random(shape) < 0.2] = 0
+    if kind.startswith("afm"):
+        prob, m1, m2 = workloads.afm_block(shape)
+        prob.materials = [prob.materials[0], workloads.afm_block(shape, alpha=3e-3, Aex=4e-12)[0].materials[0]]
+        prob.material_cell = cell
+        for m in (m1, m2):
+            m[:, cell == 0] = 0.0
+        compare_stages(prob, {FIELD_M_AFM1: m1, FIELD_M_AFM2: m2}, fm=False, afm=True)
+        return
+    prob, m = mixed_fm_problem(shape, flags=FLAG_MAGNETOSTATICS if kind == "fm_fused" else 0, rotate=False)
+    prob.material_cell = cell
+    m[:, cell == 0] = 0.0
+    compare_stages(prob, {FIELD_M: m})
