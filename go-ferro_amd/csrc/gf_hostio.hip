@@ -7,23 +7,27 @@
 // of 1 MiB, and from 8 MiB on several threads move them on, each with two
 // slots of its own, so that the faults run in parallel and a slot's copy
 // overlaps the move of the other: 40 steps of that film with the read-back
-// 121 -> 108 ms.  A field of up to one slot takes one wait and one move where
-// the direct copies wait for each component: 16x16x8, one step with its average
-// (whose partial sums go to pinned memory) and read-back 148 -> 107 us; 30x20x30
-// antiferromagnet, 10 steps 344 -> 335 us (369 with an event per component).
+// 121 -> 108 ms.  A small field takes one wait and one move where the direct
+// copies wait for each part: three parts of 8 KB 46 -> 20 us, nine of 8 KB 139 -> 44
+// (16x16x8, one step with its average, whose sums go to pinned memory, and
+// read-back 148 -> 107).  Three parts of 64 KiB to 2 MiB together are copied
+// directly: 34 us for 192 KB and 88 for 1.5 MB, 36 and 86 through the slots, and
+// 154 and 122 for 3 MB.
 //
 // The slots are shared by the process's contexts: at most kSlots of them,
 // allocated when they pay and given back with the last context.  A slot takes
-// about 0.1 ms to allocate and free again, and saves 26 us of a field of up to
-// 48 KB, about 20 us of a MB of a larger one: a program that reads one field
+// about 0.1 ms to allocate and free again, and saves 26 us of a small field,
+// about 20 us of a MB of a large one: a program that reads one field
 // and ends is slower for it (12.6 MB: first read-back 0.79 -> 1.54 ms, end of
-// the context 4.4 -> 5.3 ms).  So slots come with the fourth read-back of up to a
-// slot, or once the larger ones have moved kPays bytes for each slot they
-// need; what came before copied directly.  One
-// call holds them at a time; a call that finds them held (another thread's)
-// copies directly, as does one into memory the runtime knows (which the caller
-// pinned: 201 MB in 3.6 ms, 6.6 through the slots; 1.4 MB 53 and 82 us) and one that cannot allocate a slot or an event.  What
-// a copy, or the work queued before it, fails with is the call's error.
+// the context 4.4 -> 5.3 ms).  So slots come with the fourth small read-back, or
+// once the larger ones have moved kPays bytes for each slot they need; what came
+// before copied directly.
+//
+// One call holds the slots at a time.  A call that finds them held (another
+// thread's) copies directly, as does one that cannot allocate one, and one into
+// memory the runtime knows, which the caller pinned (201 MB in 3.6 ms, 6.6
+// through the slots; 1.4 MB 53 us and 82).  What a copy, or the work queued
+// before it, fails with is the call's error.
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -41,6 +45,7 @@ constexpr int kThreads = 8;
 constexpr int kSlots = 2 * kThreads;
 constexpr size_t kThreadsFrom = size_t{8} << 20;
 constexpr int kParts = 9;         // most arrays of a field
+constexpr size_t kSmall = size_t{64} << 10, kLarge = size_t{2} << 20;
 constexpr int kPaysCalls = 4;
 constexpr size_t kPays = size_t{4} << 20;
 
@@ -91,16 +96,20 @@ struct OnDevice {
     }
 };
 
-struct Events {
-    hipEvent_t e[kSlots] = {};
-    bool make(int n) {
-        for (int i = 0; i < n; i++)
-            if (hipEventCreateWithFlags(&e[i], hipEventDisableTiming) != hipSuccess) return false;
-        return true;
+// A point of the stream to wait for: an event, or where none can be had the
+// stream's end.
+struct Mark {
+    hipEvent_t e = nullptr;
+    hipError_t set(hipStream_t s) {
+        if (!e && hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess) {
+            e = nullptr;
+            (void)hipGetLastError();   // not the next launch's error
+        }
+        return e ? hipEventRecord(e, s) : hipSuccess;
     }
-    ~Events() {
-        for (hipEvent_t v : e)
-            if (v) (void)hipEventDestroy(v);
+    hipError_t wait(hipStream_t s) const { return e ? hipEventSynchronize(e) : hipStreamSynchronize(s); }
+    ~Mark() {
+        if (e) (void)hipEventDestroy(e);
     }
 };
 
@@ -123,20 +132,21 @@ bool have_slots(int n, size_t total) {
 }
 
 // Chunks w, w + workers, ... through the slots w and w + workers.
-hipError_t move_chunks(const Chunks& chunks, const Events& ev, int w, int workers, hipStream_t s) {
+hipError_t move_chunks(const Chunks& chunks, int w, int workers, hipStream_t s) {
+    Mark done[2];
     hipError_t e = hipSuccess;
     auto send = [&](int i, int b) {
         const Chunk k = chunks[i];
-        e = hipMemcpyAsync(g_slot[b], k.src, k.bytes, hipMemcpyDeviceToHost, s);
-        if (e == hipSuccess) e = hipEventRecord(ev.e[b], s);
+        e = hipMemcpyAsync(g_slot[w + b * workers], k.src, k.bytes, hipMemcpyDeviceToHost, s);
+        if (e == hipSuccess) e = done[b].set(s);
     };
     const int n = chunks.size();
-    for (int i = w; i < n && i < 2 * workers && e == hipSuccess; i += workers) send(i, i);
-    int b = w;
-    for (int i = w; i < n && e == hipSuccess; i += workers, b = b == w ? w + workers : w) {
-        if ((e = hipEventSynchronize(ev.e[b])) != hipSuccess) break;
+    for (int b = 0; b < 2 && w + b * workers < n && e == hipSuccess; b++) send(w + b * workers, b);
+    int b = 0;
+    for (int i = w; i < n && e == hipSuccess; i += workers, b ^= 1) {
+        if ((e = done[b].wait(s)) != hipSuccess) break;
         const Chunk k = chunks[i];
-        std::memcpy(k.dst, g_slot[b], k.bytes);
+        std::memcpy(k.dst, g_slot[w + b * workers], k.bytes);
         if (i + 2 * workers < n) send(i + 2 * workers, b);
     }
     // no copy into a slot is left behind when a call fails
@@ -144,14 +154,14 @@ hipError_t move_chunks(const Chunks& chunks, const Events& ev, int w, int worker
     return e;
 }
 
-hipError_t move_large(const Chunks& chunks, const Events& ev, int workers, int device, hipStream_t s) {
+hipError_t move_large(const Chunks& chunks, int workers, int device, hipStream_t s) {
     // the work queued before is waited for once, not by every thread
     hipError_t e = workers > 1 ? hipStreamSynchronize(s) : hipSuccess;
     if (e != hipSuccess) return e;
     std::atomic<int> failed{hipSuccess};
     auto work = [&](int w) {
         hipError_t r = w ? hipSetDevice(device) : hipSuccess;
-        if (r == hipSuccess) r = move_chunks(chunks, ev, w, workers, s);
+        if (r == hipSuccess) r = move_chunks(chunks, w, workers, s);
         int none = hipSuccess;
         if (r != hipSuccess) failed.compare_exchange_strong(none, static_cast<int>(r));
     };
@@ -186,8 +196,9 @@ hipError_t move_small(const Chunks& chunks, hipStream_t s) {
 }
 
 // Through the slots, with the result in *e; false, with nothing copied, when
-// they do not pay yet or a slot or an event cannot be had.
+// a direct copy is no slower, they do not pay yet or a slot cannot be had.
 bool through_slots(gf_ctx* c, const Chunks& chunks, size_t total, hipError_t* e) {
+    if (chunks.parts <= 3 && total > kSmall && total < kLarge) return false;
     if (total <= kSlotBytes) {
         if (!have_slots(1, total)) return false;
         *e = move_small(chunks, c->stream);
@@ -195,9 +206,8 @@ bool through_slots(gf_ctx* c, const Chunks& chunks, size_t total, hipError_t* e)
     }
     const int workers = total < kThreadsFrom ? 1 : kThreads, slots = std::min(2 * workers, chunks.size());
     const OnDevice here(c->device);
-    Events ev;
-    if (!have_slots(slots, total) || !ev.make(slots)) return false;
-    *e = move_large(chunks, ev, workers, c->device, c->stream);
+    if (!have_slots(slots, total)) return false;
+    *e = move_large(chunks, workers, c->device, c->stream);
     return true;
 }
 
@@ -259,9 +269,9 @@ gf_status download_parts(gf_ctx* c, const double* const* src, const int64_t* cou
         e = hipMemcpyAsync(dst, src[p], chunks.bytes(p), hipMemcpyDeviceToHost, c->stream);
         dst += count[p];
     }
+    const hipError_t w = hipStreamSynchronize(c->stream);   // also after a failure: no copy into the caller's is left behind
     const gf_status st = hip_check(c, e, "download");
-    if (st) return st;
-    return hip_check(c, hipStreamSynchronize(c->stream), "download sync");
+    return st ? st : hip_check(c, w, "download sync");
 }
 
 }  // namespace gf

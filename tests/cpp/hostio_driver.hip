@@ -176,11 +176,23 @@ struct Field {
     bool whole() const { return host == want; }
 };
 
-// one slot less, all and more; parts that end in a chunk of one double; the
-// threads' threshold; staggered parts; nine parts
+// one double; the limits of a small field and of a large one; parts of a slot,
+// of one double less and more; the threads' threshold; staggered parts; nine
 const std::vector<std::vector<int64_t>> kFields = {
-    {1, 1, 1}, {43690, 43690, 43690}, {43690, 43691, 43691}, {131072, 131073, 131071}, {349525, 349525, 349525},
-    {349526, 349525, 349526}, {1400011, 1400009, 1400010}, {7, 140000, 900001}, {131072, 1, 131072, 1, 1, 1, 1, 1, 200000}};
+    {1, 1, 1}, {2730, 2731, 2730}, {2731, 2731, 2731}, {43690, 43690, 43690}, {87381, 87381, 87381},
+    {87381, 87381, 87382}, {131072, 131073, 131071}, {349525, 349525, 349525}, {349526, 349525, 349526},
+    {1400011, 1400009, 1400010}, {7, 140000, 900001}, {131072, 1, 131072, 1, 1, 1, 1, 1, 200000},
+    {5000, 5000, 5000, 5000, 5000, 5000, 5000, 5000, 5000}};
+
+size_t bytes_of(const std::vector<int64_t>& n) {
+    size_t b = 0;
+    for (int64_t k : n) b += sizeof(double) * static_cast<size_t>(k);
+    return b;
+}
+// Three parts of 64 KiB to 2 MiB together are copied directly.
+bool direct(const std::vector<int64_t>& n) {
+    return n.size() <= 3 && bytes_of(n) > 65536 && bytes_of(n) < 2097152;
+}
 
 void clear() {
     g_fail = Fail{};
@@ -216,14 +228,14 @@ int whole() {
         for (int device : {0, 1}) {   // the caller's current device, the context's or not
             gf_ctx c;
             c.device = t_device = 1;
-            if (warm(f, c) < 0) return bad("no slot used", f, device);
+            if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, device);
             for (int r = 0; r < 3; r++) {
                 clear();
                 t_device = device;
                 g_known = r != 1;
                 if (f.read(c) || !f.whole() || g_last || g_done != g_queue.size()) return bad("whole", f, r);
                 if (t_device != device || g_events) return bad("left behind", f, r);
-                if (g_to_slots == 0) return bad("no slot used", f, device);
+                if ((g_to_slots == 0) != direct(n)) return bad("slots used", f, device);
             }
         }
         if (g_mallocs != g_frees) return bad("slots not given back", f, g_mallocs - g_frees);
@@ -235,8 +247,9 @@ int whole() {
 // the rule says so, serve other contexts and go with the last one.
 int pays() {
     for (const auto& n : kFields) {
+        if (direct(n)) continue;
         Field f(n);
-        const size_t bytes = sizeof(double) * f.want.size();
+        const size_t bytes = bytes_of(n);
         const int before = g_mallocs;
         {
             gf_ctx a, b;
@@ -270,7 +283,8 @@ int known() {
     return 0;
 }
 
-// A slot or an event that cannot be had: a direct copy, and no error left.
+// A slot that cannot be had: a direct copy; an event: a wait for the stream; and
+// no error left.
 int unavailable() {
     for (const char* what : {"hipHostMalloc", "hipEventCreateWithFlags"})
         for (const auto& n : kFields)
@@ -296,7 +310,7 @@ int errors() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                if (warm(f, c) < 0) return bad("no slot used", f, at);
+                if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, at);
                 clear();
                 g_fail = {what, at, false, hipErrorLaunchFailure};
                 const gf_status st = f.read(c);
@@ -316,7 +330,7 @@ int host_limits() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                if (warm(f, c) < 0) return bad("no slot used", f, at);
+                if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, at);
                 clear();
                 *limit = at;
                 const gf_status st = f.read(c);
@@ -332,7 +346,7 @@ int contended() {
         Field f(n);
         gf_ctx c;
         c.device = t_device = 1;
-        if (warm(f, c) < 0) return bad("no slot used", f, 0);
+        if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, 0);
         clear();
         std::atomic<int> step{0};
         std::thread other([&] {

@@ -23,7 +23,8 @@ def test_read_back(driver, case):
     the caller's current device and of another; the slots given back with the
     last context.  pays: no slot is allocated before it saves what it costs.
     sums: the same of an average's pinned sums.  known: memory the caller pinned is copied to directly.
-    unavailable: no slot or event to be had is a direct copy.
+    unavailable: no slot to be had is a direct copy, no event a wait for the
+    stream.
     errors: a copy, record or wait that fails is the call's error.  host_limits:
     allocations or threads that fail are no exception.  contended: another
     thread's slots are not waited for."""
