@@ -60,7 +60,7 @@ __global__ void __launch_bounds__(256) em_jp_kernel(EmJpArgs a) {
             }
             // the store is updated in place: only this thread reads it now
             const int v = 3 * p + c;
-            em_dev::rk_state(a.stage, id, k_, a.jp[v][id], a.stage > 1 ? a.jacc[v][id] : 0., a.jp[v], a.jacc[v],
+            em_dev::rk_state(a.stage, id, k_, a.stage < 4 ? a.jp[v][id] : 0., a.stage > 1 ? a.jacc[v][id] : 0., a.jp[v], a.jacc[v],
                              a.jps[v]);
             if (a.stage == 4) a.jps[3 * p + c][id] = a.jp[3 * p + c][id];
         }
@@ -90,8 +90,9 @@ __global__ void __launch_bounds__(256) em_cells_kernel(EmCellArgs a) {
         const double* ez = a.es[2];
         const I x00 = (i * (ny + 1) + j) * (nz + 1) + k, x10 = (i * (ny + 1) + j + 1) * (nz + 1) + k;
         const I y00 = (i * ny + j) * (nz + 1) + k, y10 = ((i + 1) * ny + j) * (nz + 1) + k;
-        double vx[4] = {ldd(ex, x00), ldd(ex, x10), ldd(ex, x00 + 1), ldd(ex, x10 + 1)};
-        double vy[4] = {ldd(ey, y00), ldd(ey, y10), ldd(ey, y00 + 1), ldd(ey, y10 + 1)};
+        // (a constant beside the 32-bit offset: the two k of an edge line are one load)
+        double vx[4] = {ldd(ex, x00), ldd(ex, x10), ldd(ex + 1, x00), ldd(ex + 1, x10)};
+        double vy[4] = {ldd(ey, y00), ldd(ey, y10), ldd(ey + 1, y00), ldd(ey + 1, y10)};
         if (a.zwall && (k == 0 || k == nz - 1)) {
             // the wall edges this cell reads, from the wall condition; the
             // cell of a line's own (i, j) writes it (and the last cell the
@@ -133,7 +134,7 @@ __global__ void __launch_bounds__(256) em_cells_kernel(EmCellArgs a) {
             }
             std_(a.hcell[2], id, h);
         } else {
-            std_(a.hcell[2], id, (ldd(a.hs[2], (i * ny + j) * (nz + 1) + k) + ldd(a.hs[2], (i * ny + j) * (nz + 1) + k + 1)) / 2.);
+            std_(a.hcell[2], id, (ldd(a.hs[2], (i * ny + j) * (nz + 1) + k) + ldd(a.hs[2] + 1, (i * ny + j) * (nz + 1) + k)) / 2.);
         }
     }
 }

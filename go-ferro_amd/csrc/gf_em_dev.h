@@ -33,8 +33,8 @@ __host__ __device__ __forceinline__ unsigned em_groups(int64_t n) {
     return static_cast<unsigned>((n + kEmGroup - 1) / kEmGroup);
 }
 
-// RK update of element i from its preloaded base and (at stages 2-4)
-// accumulator.
+// RK update of element i from its preloaded base (at stages 1-3) and (at
+// stages 2-4) accumulator.
 template <class I>
 __device__ __forceinline__ void rk_state(int stage, I i, double k, double y, double ac, double* base, double* acc,
                                          double* out) {
@@ -144,13 +144,35 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
     auto HY = [&](I i, I j, I k) { return (i * (ny + 1) + j) * nz + k; };
     auto HZ = [&](I i, I j, I k) { return (i * ny + j) * (nz + 1) + k; };
     auto near = [](I v, I n) { return v <= 1 || v >= n - 1; };
+    const bool last = a.stage == 4;
     int comp, wall = 0;   // -1, 1: an edge of the bottom, top z wall whose thread takes the one next to it first
     bool hist, dead;      // on a plane a Mur wall reads (two next to each non-periodic wall); a wall edge
+    I in;                 // the edge whose increment this thread evaluates
     I cell[4], ci[4], cj[4], ck[4], hp[4];
-    int hf[2];            // curl = (H_hf0[hp0] - H_hf0[hp1]) rh0 - (H_hf1[hp2] - H_hf1[hp3]) rh1
-    double rh[2];
+    uint32_t tq[4];
+    double y, yw, ac, es, rh[2], hv[4], qv[4] = {0., 0., 0., 0.};
+    // The reads of an edge of component c, whose curl is (H_h0[hp0] - H_h0[hp1])
+    // rh0 - (H_h1[hp2] - H_h1[hp3]) rh1; c, h0 and h1 are constants of each
+    // call, so that the arrays' bases stay in scalar registers.
+    auto read = [&](int c, int h0, int h1) __attribute__((always_inline)) {
+        comp = c;
+        // A wall's thread reads what its neighbour's own thread may write in
+        // this launch only at the stages where it does not (the base before
+        // stage 4, the accumulator at stage 4).
+        in = wall == 0 ? e : (wall < 0 ? e + 1 : e - 1);
+        // at stage 4 the base is read only to keep it (a whole array less to read)
+        y = !last || (a.keep && hist && !wall) ? ldd(a.eb[c], in) : 0.;
+        yw = wall && !last ? ldd(a.eb[c], e) : 0.;
+        ac = (wall ? last : a.stage > 1) ? ldd(a.eacc[c], in) : 0.;
+        es = ldd(a.es[c], in);
+        for (int q = 0; q < 4; q++) {
+            cell[q] = C(ci[q], cj[q], ck[q]);
+            tq[q] = ldu(a.code, cell[q]);
+            hv[q] = ldd(a.hs[q < 2 ? h0 : h1], hp[q]);
+            if (kQ && a.q[0]) qv[q] = ldd(a.q[c], cell[q]);
+        }
+    };
     if (e < nEx) {
-        comp = 0;
         const I l = e / (nz + 1), i = l / (ny + 1), j = l - i * (ny + 1);
         I k = e - l * (nz + 1);
         hist = (!a.per[1] && near(j, ny)) || (!a.per[2] && near(k, nz));
@@ -159,10 +181,10 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         dead = (wj && !a.per[1]) || (wk && !a.per[2]);
         const I y1 = wj ? ny - 1 : j - 1, y3 = wj ? 0 : j, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
         for (int q = 0; q < 4; q++) { ci[q] = i; cj[q] = q < 2 ? y1 : y3; ck[q] = q & 1 ? z2 : z1; }
-        hf[0] = 2; hf[1] = 1; rh[0] = a.rdy; rh[1] = a.rdz;
+        rh[0] = a.rdy; rh[1] = a.rdz;
         hp[0] = HZ(i, y3, z2); hp[1] = HZ(i, y1, z2); hp[2] = HY(i, y3, z2); hp[3] = HY(i, y3, z1);
+        read(0, 2, 1);
     } else if (e < nEx + nEy) {
-        comp = 1;
         e -= nEx;
         const I l = e / (nz + 1), i = l / ny, j = l - i * ny;
         I k = e - l * (nz + 1);
@@ -172,10 +194,10 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         dead = (wi && !a.per[0]) || (wk && !a.per[2]);
         const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, z1 = wk ? nz - 1 : k - 1, z2 = wk ? 0 : k;
         for (int q = 0; q < 4; q++) { ci[q] = q < 2 ? x1 : x3; cj[q] = j; ck[q] = q & 1 ? z2 : z1; }
-        hf[0] = 0; hf[1] = 2; rh[0] = a.rdz; rh[1] = a.rdx;
+        rh[0] = a.rdz; rh[1] = a.rdx;
         hp[0] = C(x3, j, z2); hp[1] = C(x3, j, z1); hp[2] = HZ(x3, j, z2); hp[3] = HZ(x1, j, z2);
+        read(1, 0, 2);
     } else {
-        comp = 2;
         e -= nEx + nEy;
         const I l = e / nz, k = e - l * nz, i = l / (ny + 1), j = l - i * (ny + 1);
         hist = (!a.per[0] && near(i, nx)) || (!a.per[1] && near(j, ny));
@@ -183,25 +205,9 @@ __device__ __forceinline__ void em_edge(const EmArgs& a, double* tab, I e) {
         dead = (wi && !a.per[0]) || (wj && !a.per[1]);
         const I x1 = wi ? nx - 1 : i - 1, x3 = wi ? 0 : i, y1 = wj ? ny - 1 : j - 1, y2 = wj ? 0 : j;
         for (int q = 0; q < 4; q++) { ci[q] = q < 2 ? x1 : x3; cj[q] = q & 1 ? y2 : y1; ck[q] = k; }
-        hf[0] = 1; hf[1] = 0; rh[0] = a.rdx; rh[1] = a.rdy;
+        rh[0] = a.rdx; rh[1] = a.rdy;
         hp[0] = HY(x3, y2, k); hp[1] = HY(x1, y2, k); hp[2] = C(x3, y2, k); hp[3] = C(x3, y1, k);
-    }
-    // in: the edge whose increment this thread evaluates.  A wall's thread
-    // reads what its neighbour's own thread may write in this launch only at
-    // the stages where it does not (the base before stage 4, the accumulator
-    // at stage 4).
-    const I in = wall == 0 ? e : (wall < 0 ? e + 1 : e - 1);
-    const bool last = a.stage == 4;
-    const double y = wall && last ? 0. : ldd(a.eb[comp], in), es = ldd(a.es[comp], in);
-    const double yw = wall && !last ? ldd(a.eb[comp], e) : 0.;
-    const double ac = (wall ? last : a.stage > 1) ? ldd(a.eacc[comp], in) : 0.;
-    uint32_t tq[4];
-    double qv[4] = {0., 0., 0., 0.}, hv[4];
-    for (int q = 0; q < 4; q++) {
-        cell[q] = C(ci[q], cj[q], ck[q]);
-        tq[q] = ldu(a.code, cell[q]);
-        hv[q] = ldd(a.hs[hf[q >> 1]], hp[q]);
-        if (kQ && a.q[0]) qv[q] = ldd(a.q[comp], cell[q]);
+        read(2, 1, 0);
     }
     load_emtab(tab, a.mats, a.nmat);
     if (!live) return;
@@ -252,40 +258,42 @@ __device__ __forceinline__ void em_face(const EmArgs& a, I f) {
     auto EX = [&](I i, I j, I k) { return (i * (ny + 1) + j) * (nz + 1) + k; };
     auto EY = [&](I i, I j, I k) { return (i * ny + j) * (nz + 1) + k; };
     auto EZ = [&](I i, I j, I k) { return (i * (ny + 1) + j) * nz + k; };
-    int comp, ef[2];      // curl = (E_ef0[ep0] - E_ef0[ep1]) re0 - (E_ef1[ep2] - E_ef1[ep3]) re1
-    I c1, c2, ep[4];      // the two cells beside the face
-    double re[2];
+    const bool mag = a.dm[0] || a.dma1[0];
+    int comp;
+    CellDm m1{}, m2{};    // of the two cells beside the face
+    double y, ac, re[2], ev[4];   // curl = (ev0 - ev1) re0 - (ev2 - ev3) re1
+    // the cells first (their materials' records are a second trip to memory),
+    // with a constant component in each call
+    auto read = [&](int c, I c1, I c2) __attribute__((always_inline)) {
+        comp = c;
+        if (mag) { m1 = load_dm<I>(a, c, c1); m2 = load_dm<I>(a, c, c2); }
+        y = a.stage < 4 ? ldd(a.hb[c], f) : 0.;
+        ac = a.stage > 1 ? ldd(a.hacc[c], f) : 0.;
+    };
     if (f < nHx) {
-        comp = 0;
         const I l = f / nz, k = f - l * nz, i = l / ny, j = l - i * ny;
         const I x1 = i == 0 ? (a.per[0] ? nx - 1 : 0) : i - 1, x2 = i == nx ? (a.per[0] ? 0 : nx - 1) : i;
-        ef[0] = 2; ef[1] = 1; re[0] = a.rdy; re[1] = a.rdz;
-        ep[0] = EZ(i, j + 1, k); ep[1] = EZ(i, j, k); ep[2] = EY(i, j, k + 1); ep[3] = EY(i, j, k);
-        c1 = C(x1, j, k); c2 = C(x2, j, k);
+        read(0, C(x1, j, k), C(x2, j, k));
+        re[0] = a.rdy; re[1] = a.rdz;
+        ev[0] = ldd(a.es[2], EZ(i, j + 1, k)); ev[1] = ldd(a.es[2], EZ(i, j, k));
+        ev[2] = ldd(a.es[1] + 1, EY(i, j, k)); ev[3] = ldd(a.es[1], EY(i, j, k));
     } else if (f < nHx + nHy) {
-        comp = 1;
         f -= nHx;
         const I l = f / nz, k = f - l * nz, i = l / (ny + 1), j = l - i * (ny + 1);
         const I y1 = j == 0 ? (a.per[1] ? ny - 1 : 0) : j - 1, y2 = j == ny ? (a.per[1] ? 0 : ny - 1) : j;
-        ef[0] = 0; ef[1] = 2; re[0] = a.rdz; re[1] = a.rdx;
-        ep[0] = EX(i, j, k + 1); ep[1] = EX(i, j, k); ep[2] = EZ(i + 1, j, k); ep[3] = EZ(i, j, k);
-        c1 = C(i, y1, k); c2 = C(i, y2, k);
+        read(1, C(i, y1, k), C(i, y2, k));
+        re[0] = a.rdz; re[1] = a.rdx;
+        ev[0] = ldd(a.es[0] + 1, EX(i, j, k)); ev[1] = ldd(a.es[0], EX(i, j, k));
+        ev[2] = ldd(a.es[2], EZ(i + 1, j, k)); ev[3] = ldd(a.es[2], EZ(i, j, k));
     } else {
-        comp = 2;
         f -= nHx + nHy;
         const I l = f / (nz + 1), k = f - l * (nz + 1), i = l / ny, j = l - i * ny;
         const I z1 = k == 0 ? (a.per[2] ? nz - 1 : 0) : k - 1, z2 = k == nz ? (a.per[2] ? 0 : nz - 1) : k;
-        ef[0] = 1; ef[1] = 0; re[0] = a.rdx; re[1] = a.rdy;
-        ep[0] = EY(i + 1, j, k); ep[1] = EY(i, j, k); ep[2] = EX(i, j + 1, k); ep[3] = EX(i, j, k);
-        c1 = C(i, j, z1); c2 = C(i, j, z2);
+        read(2, C(i, j, z1), C(i, j, z2));
+        re[0] = a.rdx; re[1] = a.rdy;
+        ev[0] = ldd(a.es[1], EY(i + 1, j, k)); ev[1] = ldd(a.es[1], EY(i, j, k));
+        ev[2] = ldd(a.es[0], EX(i, j + 1, k)); ev[3] = ldd(a.es[0], EX(i, j, k));
     }
-    // the cells first: their materials' records are a second trip to memory
-    const bool mag = a.dm[0] || a.dma1[0];
-    CellDm m1{}, m2{};
-    if (mag) { m1 = load_dm<I>(a, comp, c1); m2 = load_dm<I>(a, comp, c2); }
-    const double y = ldd(a.hb[comp], f), ac = a.stage > 1 ? ldd(a.hacc[comp], f) : 0.;
-    double ev[4];
-    for (int q = 0; q < 4; q++) ev[q] = ldd(a.es[ef[q >> 1]], ep[q]);
     double k_ = -a.dt / kMu0 * ((ev[0] - ev[1]) * re[0] - (ev[2] - ev[3]) * re[1]);
     if (mag) {
         double cnt = 0.;

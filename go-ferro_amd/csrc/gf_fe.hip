@@ -31,7 +31,7 @@ __device__ __forceinline__ double landau(const DevMaterial& M, double pa, double
            2. * M.a1123 * pa * b2 * c2 * (2. * a2 + b2 + c2);
 }
 
-// RK update of one component from its base y and (at stages 2-4)
+// RK update of one component from its base y (at stages 1-3) and (at stages 2-4)
 // accumulator ac.
 template <class I>
 __device__ __forceinline__ void rk(int stage, I id, double k, double y, double ac, double* acc, double* out) {
@@ -82,8 +82,8 @@ __device__ __forceinline__ void fe_cell(const FeStageArgs& a, I id) {
             const I x0 = (i * (ny + 1) + j) * (nz + 1) + k, x1 = x0 + nz + 1;
             const I y0 = (i * ny + j) * (nz + 1) + k, y1 = y0 + ny * (nz + 1);
             const I z0 = (i * (ny + 1) + j) * nz + k, z1 = z0 + (ny + 1) * nz;
-            e0 = (ldd(a.es[0], x0) + ldd(a.es[0], x1) + ldd(a.es[0], x0 + 1) + ldd(a.es[0], x1 + 1)) / 4.;
-            e1 = (ldd(a.es[1], y0) + ldd(a.es[1], y1) + ldd(a.es[1], y0 + 1) + ldd(a.es[1], y1 + 1)) / 4.;
+            e0 = (ldd(a.es[0], x0) + ldd(a.es[0], x1) + ldd(a.es[0] + 1, x0) + ldd(a.es[0] + 1, x1)) / 4.;
+            e1 = (ldd(a.es[1], y0) + ldd(a.es[1], y1) + ldd(a.es[1] + 1, y0) + ldd(a.es[1] + 1, y1)) / 4.;
             e2 = (ldd(a.es[2], z0) + ldd(a.es[2], z1) + ldd(a.es[2], z0 + nz) + ldd(a.es[2], z1 + nz)) / 4.;
         } else if (a.ecell[0]) {
             e0 = ldd(a.ecell[0], id); e1 = ldd(a.ecell[1], id); e2 = ldd(a.ecell[2], id);
@@ -147,8 +147,9 @@ __device__ __forceinline__ void fe_cell(const FeStageArgs& a, I id) {
     }
     // the update's reads go out together, before its first write: a read
     // after a write waits for both
-    double yp[3], yq[3], ap[3] = {0., 0., 0.}, aq[3] = {0., 0., 0.};
-    for (int c = 0; c < 3; c++) { yp[c] = ldd(a.pbase[c], id); yq[c] = ldd(a.qbase[c], id); }
+    double yp[3] = {0., 0., 0.}, yq[3] = {0., 0., 0.}, ap[3] = {0., 0., 0.}, aq[3] = {0., 0., 0.};
+    if (a.stage < 4)
+        for (int c = 0; c < 3; c++) { yp[c] = ldd(a.pbase[c], id); yq[c] = ldd(a.qbase[c], id); }
     if (a.stage > 1)
         for (int c = 0; c < 3; c++) { ap[c] = ldd(a.pacc[c], id); aq[c] = ldd(a.qacc[c], id); }
     const double qs[3] = {q0, q1, q2};
