@@ -7,21 +7,22 @@
 // of 1 MiB, and from 8 MiB on several threads move them on, each with two
 // slots of its own, so that the faults run in parallel and a slot's copy
 // overlaps the move of the other: 40 steps of that film with the read-back
-// 121 -> 108 ms.  A small field takes one wait and one move where the direct
-// copies wait for each part: three parts of 8 KB 46 -> 20 us, nine of 8 KB 139 -> 44
-// (16x16x8, one step with its average, whose sums go to pinned memory, and
-// read-back 148 -> 107).  Three parts of 64 KiB to 2 MiB together are copied
-// directly: 34 us for 192 KB and 88 for 1.5 MB, 36 and 86 through the slots, and
-// 154 and 122 for 3 MB.
+// 121 -> 108 ms.  A field of up to one slot takes one wait and one move where the
+// direct copies wait for each part: three parts of 8 KB 46 -> 20 us, nine of 8 KB
+// 139 -> 44 (16x16x8, one step with its average, whose sums go to pinned memory,
+// and read-back 148 -> 107).  From 64 KiB to 2 MiB both take the same time into
+// memory in use (34 and 36 us for 192 KB, 88 and 86 for 1.5 MB), but not into new
+// memory: the first read-back of 96 antiferromagnets, 192 fields of 1.3 MB on
+// average, makes their 100 steps 182 ms directly and 155 through the slots.
 //
 // The slots are shared by the process's contexts: at most kSlots of them,
 // allocated when they pay and given back with the last context.  A slot takes
-// about 0.1 ms to allocate and free again, and saves 26 us of a small field,
-// about 20 us of a MB of a large one: a program that reads one field
-// and ends is slower for it (12.6 MB: first read-back 0.79 -> 1.54 ms, end of
-// the context 4.4 -> 5.3 ms).  So slots come with the fourth small read-back, or
-// once the larger ones have moved kPays bytes for each slot they need; what came
-// before copied directly.
+// about 0.1 ms to allocate and free again, and saves 26 us of a small field, 20 to
+// 120 us of a MB of a larger one: a program that reads one field and ends is
+// slower for it (12.6 MB: first read-back 0.79 -> 1.54 ms, end of the context 4.4
+// -> 5.3 ms).  So slots come with the fourth read-back of up to a slot, or once
+// kPays bytes have been read for each slot needed; what came before copied
+// directly.
 //
 // One call holds the slots at a time.  A call that finds them held (another
 // thread's) copies directly, as does one that cannot allocate one, and one into
@@ -45,16 +46,15 @@ constexpr int kThreads = 8;
 constexpr int kSlots = 2 * kThreads;
 constexpr size_t kThreadsFrom = size_t{8} << 20;
 constexpr int kParts = 9;         // most arrays of a field
-constexpr size_t kSmall = size_t{64} << 10, kLarge = size_t{2} << 20;
 constexpr int kPaysCalls = 4;
-constexpr size_t kPays = size_t{4} << 20;
+constexpr size_t kPays = size_t{2} << 20;
 
 std::mutex g_slots_lock;          // held while the slots are used or freed
 std::mutex g_users_lock;
 int64_t g_users = 0;              // contexts alive
 char* g_slot[kSlots] = {};
-int g_small_reads = 0;            // read-backs since the slots were last given back
-size_t g_large_bytes = 0;
+int g_reads = 0;                  // read-backs that found no slot since they were last given back
+size_t g_bytes = 0;
 
 // The parts of a field one after another in host memory, as chunks of at most
 // a slot.
@@ -117,12 +117,9 @@ struct Mark {
 // yet; false when they do not pay yet or cannot be had.
 bool have_slots(int n, size_t total) {
     if (g_slot[n - 1]) return true;
-    if (total <= kSlotBytes) {
-        if (++g_small_reads < kPaysCalls) return false;
-    } else {
-        g_large_bytes += total;
-        if (g_large_bytes / static_cast<size_t>(n) < kPays) return false;
-    }
+    g_reads++;
+    g_bytes += total;
+    if (!(n == 1 && g_reads >= kPaysCalls) && g_bytes / static_cast<size_t>(n) < kPays) return false;
     for (int i = 0; i < n; i++)
         if (!g_slot[i] && hipHostMalloc(reinterpret_cast<void**>(&g_slot[i]), kSlotBytes, hipHostMallocPortable) != hipSuccess) {
             g_slot[i] = nullptr;
@@ -196,9 +193,8 @@ hipError_t move_small(const Chunks& chunks, hipStream_t s) {
 }
 
 // Through the slots, with the result in *e; false, with nothing copied, when
-// a direct copy is no slower, they do not pay yet or a slot cannot be had.
+// they do not pay yet or a slot cannot be had.
 bool through_slots(gf_ctx* c, const Chunks& chunks, size_t total, hipError_t* e) {
-    if (chunks.parts <= 3 && total > kSmall && total < kLarge) return false;
     if (total <= kSlotBytes) {
         if (!have_slots(1, total)) return false;
         *e = move_small(chunks, c->stream);
@@ -234,8 +230,8 @@ void host_slots_release() {
         if (p) (void)hipHostFree(p);
         p = nullptr;
     }
-    g_small_reads = 0;
-    g_large_bytes = 0;
+    g_reads = 0;
+    g_bytes = 0;
 }
 
 // A kernel's partial sums straight in pinned memory save the copy after it, 11

@@ -176,7 +176,7 @@ struct Field {
     bool whole() const { return host == want; }
 };
 
-// one double; the limits of a small field and of a large one; parts of a slot,
+// one double; fields below and above a slot; parts of a slot,
 // of one double less and more; the threads' threshold; staggered parts; nine
 const std::vector<std::vector<int64_t>> kFields = {
     {1, 1, 1}, {2730, 2731, 2730}, {2731, 2731, 2731}, {43690, 43690, 43690}, {87381, 87381, 87381},
@@ -189,11 +189,6 @@ size_t bytes_of(const std::vector<int64_t>& n) {
     for (int64_t k : n) b += sizeof(double) * static_cast<size_t>(k);
     return b;
 }
-// Three parts of 64 KiB to 2 MiB together are copied directly.
-bool direct(const std::vector<int64_t>& n) {
-    return n.size() <= 3 && bytes_of(n) > 65536 && bytes_of(n) < 2097152;
-}
-
 void clear() {
     g_fail = Fail{};
     g_queue.clear();
@@ -228,14 +223,14 @@ int whole() {
         for (int device : {0, 1}) {   // the caller's current device, the context's or not
             gf_ctx c;
             c.device = t_device = 1;
-            if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, device);
+            if (warm(f, c) < 0) return bad("no slot used", f, device);
             for (int r = 0; r < 3; r++) {
                 clear();
                 t_device = device;
                 g_known = r != 1;
                 if (f.read(c) || !f.whole() || g_last || g_done != g_queue.size()) return bad("whole", f, r);
                 if (t_device != device || g_events) return bad("left behind", f, r);
-                if ((g_to_slots == 0) != direct(n)) return bad("slots used", f, device);
+                if (g_to_slots == 0) return bad("no slot used", f, device);
             }
         }
         if (g_mallocs != g_frees) return bad("slots not given back", f, g_mallocs - g_frees);
@@ -247,7 +242,6 @@ int whole() {
 // the rule says so, serve other contexts and go with the last one.
 int pays() {
     for (const auto& n : kFields) {
-        if (direct(n)) continue;
         Field f(n);
         const size_t bytes = bytes_of(n);
         const int before = g_mallocs;
@@ -258,7 +252,8 @@ int pays() {
             int chunks = 0;
             for (int64_t k : n) chunks += static_cast<int>((sizeof(double) * k + gf::kSlotBytes - 1) / gf::kSlotBytes);
             const size_t slots = bytes <= gf::kSlotBytes ? 1 : std::min(bytes < gf::kThreadsFrom ? 2 : gf::kSlots, chunks);
-            const int want = bytes <= gf::kSlotBytes ? 3 : static_cast<int>((slots * gf::kPays + bytes - 1) / bytes) - 1;
+            const int paid = static_cast<int>((slots * gf::kPays + bytes - 1) / bytes) - 1;
+            const int want = slots == 1 ? std::min(paid, gf::kPaysCalls - 1) : paid;
             if (reads != want || g_mallocs - before != static_cast<int>(slots)) return bad("pays", f, reads);
             if (warm(f, b) != 0) return bad("another context", f, 0);
         }
@@ -310,7 +305,7 @@ int errors() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, at);
+                if (warm(f, c) < 0) return bad("no slot used", f, at);
                 clear();
                 g_fail = {what, at, false, hipErrorLaunchFailure};
                 const gf_status st = f.read(c);
@@ -330,7 +325,7 @@ int host_limits() {
                 Field f(n);
                 gf_ctx c;
                 c.device = t_device = 1;
-                if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, at);
+                if (warm(f, c) < 0) return bad("no slot used", f, at);
                 clear();
                 *limit = at;
                 const gf_status st = f.read(c);
@@ -346,7 +341,7 @@ int contended() {
         Field f(n);
         gf_ctx c;
         c.device = t_device = 1;
-        if ((warm(f, c) < 0) != direct(n)) return bad("slots used", f, 0);
+        if (warm(f, c) < 0) return bad("no slot used", f, 0);
         clear();
         std::atomic<int> step{0};
         std::thread other([&] {
