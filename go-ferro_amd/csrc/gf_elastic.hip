@@ -384,7 +384,7 @@ __global__ void __launch_bounds__(256) el_prep_kernel(ElStageArgs a) {
 // that says whether it is free.  Here the store, codes and the P's of the y
 // and z faces are loaded before any code is known and the z neighbours come
 // from the adjacent lanes; the x faces' P's (9 values) are loaded after the
-// other axes are done, so that the kernel stays at 124 VGPRs and 4 waves per
+// other axes are done, so that the kernel stays at 126 VGPRs and 4 waves per
 // SIMD (with them first: 141 and 3 waves).  1M cells (128x128x64): 95.4 ->
 // 86.5 us; 70k cells (45x38x41): 13.9 -> 12.2 us.
 // group: the workgroup's index among those of the force.
@@ -572,7 +572,7 @@ __global__ void __launch_bounds__(kGroup) el_force_kernel(ElStageArgs a) {
 // (45x38x41) each launch is mostly latency, and the magnet's 7.8 us hide in
 // the force's: 60 steps 7.66 -> 6.34 ms; 128x128x64: 45.5 -> 43.7 ms.
 template <bool kMixed>
-__global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, StageArgs m, const uint32_t* ids,
+__global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, StageArgs, const uint32_t* ids,
                                                               uint32_t count, unsigned mag_groups) {
     extern __shared__ double ctab[];   // the materials' constants (load_ctab)
     if (blockIdx.x >= mag_groups) {
@@ -581,6 +581,10 @@ __global__ void __launch_bounds__(kGroup) el_force_mag_kernel(ElStageArgs a, Sta
     }
     const uint32_t t = blockIdx.x * kGroup + threadIdx.x;
     if (t >= count) return;
+    // by value beside the force's, 96 scalar registers spill (128x128x64 with 4
+    // layers of magnet 588 us a step, 586 so; 48x48x48 101.9 and 100.3); the force's
+    // read like this is slower on small grids (12x10x16: 63 us, 67)
+    const StageArgs& m = launch_arg<StageArgs, sizeof(ElStageArgs)>();
     if (ids) fm_point<uint32_t, false, kMixed>(m, ldu(ids, t));
     else fm_point<uint32_t, true, kMixed>(m, t);
 }

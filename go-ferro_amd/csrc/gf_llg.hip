@@ -32,7 +32,7 @@ static_assert(kLeanMats * sizeof(DevMaterial) / sizeof(double) <= kMatWordsPerTh
 
 template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) mag_stage_kernel(StageArgs) {
-    const StageArgs& a = first_arg<StageArgs>();
+    const StageArgs& a = launch_arg<StageArgs>();
     const I n = static_cast<I>(a.nx * a.ny * a.nz);
     const I id = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (id >= n) return;
@@ -44,7 +44,7 @@ __global__ void __launch_bounds__(256) mag_stage_kernel(StageArgs) {
 // list is of 32-bit indices on every grid that has one (up to 2^32 cells).
 template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) mag_stage_list_kernel(StageArgs, const uint32_t* ids, I count) {
-    const StageArgs& a = first_arg<StageArgs>();
+    const StageArgs& a = launch_arg<StageArgs>();
     const I t = static_cast<I>(blockIdx.x) * static_cast<I>(blockDim.x) + static_cast<I>(threadIdx.x);
     if (t >= count) return;
     fm_point<I, false, kMixed>(a, static_cast<I>(ldu(ids, t)));
@@ -293,10 +293,10 @@ __device__ __forceinline__ void afm_point(const AfmStageArgs& a, I id, int sub) 
 // (workgroups are dealt to the 8 XCDs round-robin) one dispatch round
 // apart, so the second finds the shared reads (code, Hstat, the other
 // sublattice's store) in that XCD's L2.  Over one material the by-value argument
-// is the faster one (64x64x32: 36.3 us a step, 37.9 through first_arg).
+// is the faster one (64x64x32: 36.3 us a step, 37.9 through launch_arg).
 template <class I, bool kMixed>
 __global__ void __launch_bounds__(256) afm_stage_kernel(AfmStageArgs byval) {
-    const AfmStageArgs& a = kMixed ? first_arg<AfmStageArgs>() : byval;
+    const AfmStageArgs& a = kMixed ? launch_arg<AfmStageArgs>() : byval;
     const unsigned b = blockIdx.x;
     const unsigned blk = (b >> 4) * 8u + (b & 7u);
     const int sub = static_cast<int>((b >> 3) & 1u);

@@ -64,15 +64,17 @@ __device__ __forceinline__ uint32_t ldu(const uint32_t* p, uint32_t i) {
     return *(GConstU*)((GConstC*)p + (i << 2));
 }
 
-// A kernel's first argument where the launch put it.  Its fields then are
-// scalar loads where they are used; a by-value struct of the size of a stage's is
+// A kernel's argument where the launch put it, kOffset bytes into its
+// arguments.  Its fields then are scalar loads where they are used; a by-value struct of the size of a stage's is
 // loaded at entry and its fields are kept in lanes of vector registers (28 to 84
 // scalar registers spilled in the magnet stages, each read back by a
 // v_readlane): ferromagnet 30x40x50 without magnetostatics 22.3 -> 20.6 us a step,
 // two stacked antiferromagnets of 128x128x32 cells 287 -> 275.
-template <class T>
-__device__ __forceinline__ const T& first_arg() {
-    return *(const T*)(const __attribute__((address_space(4))) T*)__builtin_amdgcn_kernarg_segment_ptr();
+template <class T, size_t kOffset = 0>
+__device__ __forceinline__ const T& launch_arg() {
+    static_assert(kOffset % alignof(T) == 0, "arguments follow each other at their alignment");
+    typedef const __attribute__((address_space(4))) char Byte;
+    return *(const T*)(const __attribute__((address_space(4))) T*)((Byte*)__builtin_amdgcn_kernarg_segment_ptr() + kOffset);
 }
 
 // Exchange-weighted neighbour differences of one store for one cell
