@@ -59,9 +59,11 @@ def test_threads_read_their_own_contexts():
         c.upload(FIELD_M, m)
         ctxs.append((c, m))
     bad = []
+    together = threading.Barrier(len(ctxs))
 
     def read(c, m):
-        for _ in range(5):
+        for _ in range(12):
+            together.wait(timeout=60)
             if not np.array_equal(c.download(FIELD_M), m):
                 bad.append(m.shape)
 
