@@ -52,7 +52,7 @@ __device__ __forceinline__ void rk(int stage, I id, double k, double y, double a
 // The stage of cell id.  Bound by the latency of its loads: the neighbours'
 // reads used to wait for one another face by face, and each of the update's
 // for the write before it.  96x128x32 film, half of it ferroelectric: 26.3 ->
-// 17.8 us with each group read together and 32-bit offsets (from 24.1 us with
+// 16.7 us with each group read together and 32-bit offsets (from 24.1 us with
 // the offsets alone).
 template <class I>
 __device__ __forceinline__ void fe_cell(const FeStageArgs& a, I id) {
@@ -172,7 +172,7 @@ __global__ void __launch_bounds__(256) fe_stage_kernel(FeStageArgs a) {
 // q_s dt) and neither reads what the other writes; the FE stage reads the
 // E store of the stage, directly or as the cell arrays made from it.  With
 // the z walls and the cells' E in it a stage of the 8x8x1024 column is this
-// launch alone: 300 steps 21.3 -> 14.2 ms (the cells launch was 4.9 us of 17.7).
+// launch alone: 300 steps 21.3 -> 12.6 ms (the cells launch was 4.9 us of 17.7).
 template <class I>
 __global__ void __launch_bounds__(em_dev::kEmGroup) fe_em_kernel(FeStageArgs f, EmArgs e) {
     extern __shared__ double emtab[];
